@@ -202,11 +202,12 @@ __global__ __launch_bounds__(BLK) void k_norm(long v5, const TT<P> *x, double *p
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// epilogues for operators that cannot fuse them (Wilson kernel)
+// epilogues for operators that cannot fuse them (Wilson kernel); the sums
+// take nb entries, so block 0 zero-fills those past this grid
 __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o, const double2 *w,
                                              double2 *r, double2 *x, const double2 *p,
                                              const double *a, const double *b, const int *stop,
-                                             double *partial) {
+                                             double *partial, int nb) {
   if (stop && *stop) return;
   const long i = (long)blockIdx.x * BLK + threadIdx.x;
   double red = 0.0;
@@ -229,6 +230,8 @@ __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o
   }
   const double t = block_sum(red);
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
+  if (blockIdx.x == 0)
+    for (int k = (int)(gridDim.x + threadIdx.x); k < nb; k += BLK) partial[k] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -527,7 +530,7 @@ static int apply_op_epi(const OpDesc &op, int dagger, const double2 *in, double2
     if (rc) return rc;
     if (mode != EPI_STORE) {
       hipLaunchKernelGGL(k_epi, dim3(nblk(op.d.v5())), dim3(BLK), 0, s, op.d.v5(), mode, o, w, r,
-                         x, p, a, b, stop, partial);
+                         x, p, a, b, stop, partial, (int)dslash_blocks(op.d));
       THR_HIP(hipGetLastError());
     }
     return THR_OK;
