@@ -30,6 +30,43 @@ def smooth(dims, seed):
     return rng, O.coef(th, dims)
 
 
+# iterations around the 32-iteration blocks of the shift updates: a cap inside
+# the first block, at its end, one past it, and in the third block
+@pytest.mark.parametrize("kernel", ["shamir", "wilson"])
+@pytest.mark.parametrize("maxcg", [0, 1, 31, 32, 33, 65])
+def test_multishift_blocks_at_the_cap(G, maxcg, kernel):
+    dims = (3, 5, 4, 12)
+    rng, u = smooth(dims, 31)
+    inp = D.rand_spinor(dims, rng)
+    sig = np.array([1e-4, 0.05, 0.7, 9.0])
+    print("case: multishift cap", maxcg, kernel, flush=True)
+    # the heavier shifts converge inside a block and leave the window
+    og, cg, cgs = G.multishift(u, dims, 0.05, 3, sig, np.ones(4), inp, res=1e-5, maxcg=maxcg,
+                               kernel=kernel)
+    oo, co, cos = O.multishift(u, dims, 0.05, 3, sig, np.ones(4), inp, res=1e-5, maxcg=maxcg,
+                               kernel=kernel)
+    assert cg == co and np.array_equal(cgs, cos)
+    if maxcg == 0:
+        assert not og.any()
+    else:
+        assert rel(og, oo) <= 1e-11
+
+
+@pytest.mark.parametrize("n", [1, 25, 32])
+def test_multishift_shift_counts(G, n):
+    """One shift, the 25 of the rational approximation, the most allowed."""
+    dims = (4, 4, 6, 8)
+    rng, u = smooth(dims, 32)
+    inp = D.rand_spinor(dims, rng)
+    sig = np.geomspace(1e-3, 60.0, n)
+    num = np.geomspace(0.01, 3.0, n)
+    print("case: multishift shifts", n, flush=True)
+    og, cg, cgs = G.multishift(u, dims, 0.1, 3, sig, num, inp, res=1e-6, maxcg=500)
+    oo, co, cos = O.multishift(u, dims, 0.1, 3, sig, num, inp, res=1e-6, maxcg=500)
+    assert cg == co and np.array_equal(cgs, cos)
+    assert rel(og, oo) <= 1e-11
+
+
 def test_wilson_congrad_after_a_larger_shamir_solve(G):
     """The Wilson kernel's epilogue fills fewer partial sums than the next sum
     takes: what a Shamir solve on another lattice left there must not count."""

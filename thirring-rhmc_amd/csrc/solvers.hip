@@ -10,6 +10,7 @@
 // exactly those of the reference's loop structure.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <map>
@@ -205,9 +206,9 @@ __global__ __launch_bounds__(BLK) void k_norm(long v5, const TT<P> *x, double *p
 // epilogues for operators that cannot fuse them (Wilson kernel); the sums
 // take nb entries, so block 0 zero-fills those past this grid
 __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o, const double2 *w,
-                                             double2 *r, double2 *x, const double2 *p,
-                                             const double *a, const double *b, const int *stop,
-                                             double *partial, int nb) {
+                                             const double2 *r, double2 *ro, double2 *x,
+                                             const double2 *p, const double *a, const double *b,
+                                             const int *stop, double *partial, int nb) {
   if (stop && *stop) return;
   const long i = (long)blockIdx.x * BLK + threadIdx.x;
   double red = 0.0;
@@ -220,9 +221,13 @@ __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o
       } else if (mode == EPI_DOTW) {
         const cx<double> wv = ldc(w, e);
         red += wv.r * ov.r + wv.i * ov.i;
+      } else if (mode == EPI_HREC) {
+        const cx<double> hv = ov + (*b) * ldc(x, e);
+        st(x, e, hv);
+        red += norm2(hv);
       } else if (mode == EPI_CG) {
         const cx<double> rv = ldc(r, e) - (*a) * ov;
-        st(r, e, rv);
+        st(ro, e, rv);
         red += norm2(rv);
         if (b) st(x, e, ldc(x, e) + (*b) * ldc(p, e));
       }
@@ -315,6 +320,9 @@ __global__ __launch_bounds__(BLK) void k_cg_p(long n, const double2 *r, double2 
 // ---------------------------------------------------------------------------
 // multishift state (multishift_module.F90:71-282)
 // ---------------------------------------------------------------------------
+// iterations per block of the blocked shift updates (k_ms_flush)
+constexpr int MSR = 32;
+
 struct MsState {
   double delta, alpha, lambda, omega, omega_save, gammag;
   double zeta_i[MAXSHIFT], zeta_ii[MAXSHIFT], zeta_iii[MAXSHIFT], omegas[MAXSHIFT],
@@ -324,6 +332,16 @@ struct MsState {
   int nonfinite;  // a dot product came out NaN/Inf: the solve stopped there
   float res;
   double resd;  // threshold used by the convergence test
+  // blocked shift updates: the scalars of iteration j of the block for every
+  // shift updated in it, how many iterations of the block updated shift i,
+  // and the block's iterations so far
+  double rec_om[MSR][MAXSHIFT], rec_ga[MSR][MAXSHIFT], rec_ze[MSR][MAXSHIFT];
+  int cnt[MAXSHIFT], jcount;
+  double minus_omega;
+  // the block's coefficients for its flush: p_i = ca P_i + sum cb R,
+  // x_i = X_i + cc P_i + sum cd R
+  double ca[MAXSHIFT], cc[MAXSHIFT], cb[MAXSHIFT][MSR], cd[MAXSHIFT][MSR];
+  int fcnt[MAXSHIFT], fact[MAXSHIFT], fjc;
 };
 
 __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *partial, int nb) {
@@ -345,6 +363,8 @@ __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *part
     st->mini = 1;
     st->umin = 1;
     st->umax = 0;
+    for (int i = 0; i < MAXSHIFT; i++) st->cnt[i] = 0;
+    st->jcount = 0;
     st->nonfinite = isfinite(d) ? 0 : 1;
     st->stop = (st->maxcg <= 0 || st->n <= 0 || st->nonfinite) ? 1 : 0;
     st->done = st->stop;
@@ -354,72 +374,204 @@ __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *part
   }
 }
 
-__global__ void k_ms_alpha(MsState *st, const double *partial, int nb) {
+// The shift recurrences take one thread per shift (MAXSHIFT <= 64: all in
+// wave 0); each shift's arithmetic is the serial loop's.  One thread walking
+// 25 shifts took 5.9 (alpha) and 11.7 us (lambda) per launch at 16^3 x 48,
+// most of it the memory latency of one shift after another.
+__global__ __launch_bounds__(BLK) void k_ms_alpha(MsState *st, const double *partial, int nb) {
   if (st->stop) {
     if (threadIdx.x == 0) st->done = 1;
     return;
   }
-  const double al = fin_sum(partial, nb);
+  __shared__ double s_al;
+  const double sum = fin_sum(partial, nb);
+  if (threadIdx.x == 0) s_al = sum;
+  __syncthreads();
+  const double al = s_al, os = st->omega, gg = st->gammag, om = -st->delta / al;
+  const bool ok = isfinite(om);
+  const int i = threadIdx.x;
+  if (ok && i >= st->mini - 1 && i < st->maxi) {
+    const double z1 = st->zeta_i[i], z2 = st->zeta_ii[i];
+    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - st->aden[i] * om));
+    st->zeta_iii[i] = z3;
+    st->omegas[i] = om * z3 / z2;
+  }
+  __syncthreads();  // every thread has read the scalars before thread 0 writes them
   if (threadIdx.x == 0) {
     st->cg_return += 1;
     st->alpha = al;
-    st->omega_save = st->omega;
-    st->omega = -st->delta / al;
-    if (!isfinite(st->omega)) {
+    st->omega_save = os;
+    st->omega = om;
+    st->minus_omega = -om;
+    if (!ok) {
       // nothing downstream of a non-finite omega is meaningful: stop before
       // any vector of this iteration is updated
       st->nonfinite = 1;
       st->stop = 1;
       st->done = 1;
-      return;
-    }
-    const double om = st->omega, os = st->omega_save, gg = st->gammag;
-    for (int i = st->mini - 1; i < st->maxi; i++) {
-      st->zeta_iii[i] = (st->zeta_i[i] * st->zeta_ii[i] * os) /
-                        (om * gg * (st->zeta_i[i] - st->zeta_ii[i]) +
-                         st->zeta_i[i] * os * (1.0 - st->aden[i] * om));
-      st->omegas[i] = om * st->zeta_iii[i] / st->zeta_ii[i];
     }
   }
 }
 
-__global__ void k_ms_lambda(MsState *st, const double *partial, int nb) {
+// REC: record the iteration's shift scalars for the block's flush
+template <bool REC>
+__global__ __launch_bounds__(BLK) void k_ms_lambda(MsState *st, const double *partial, int nb) {
   if (st->stop) return;
-  const double lam = fin_sum(partial, nb);
-  if (threadIdx.x == 0) {
-    if (!isfinite(lam)) {
+  __shared__ double s_lam;
+  __shared__ int s_nmin, s_nmax;
+  const double sum = fin_sum(partial, nb);
+  if (threadIdx.x == 0) s_lam = sum;
+  __syncthreads();
+  const double lam = s_lam;
+  if (!isfinite(lam)) {
+    if (threadIdx.x == 0) {
       st->nonfinite = 1;
       st->stop = 1;
       st->done = 1;
-      return;
     }
-    st->lambda = lam;
-    st->gammag = lam / st->delta;
-    for (int i = st->mini - 1; i < st->maxi; i++) {
-      st->gammas[i] = st->gammag * st->zeta_iii[i] * st->omegas[i] / (st->zeta_ii[i] * st->omega);
-      st->cg_returns[i] = st->cg_return;
-    }
-    st->umin = st->mini;
-    st->umax = st->maxi;
-    int nmax = 0, nmin = st->n + 1;
-    for (int i = 0; i < st->n; i++) {
-      if (st->flags[i]) {
-        if (sqrt(st->delta * st->zeta_ii[i] * st->zeta_ii[i]) * st->corr[i] < st->resd) {
-          st->flags[i] = 0;
-        } else {
-          nmax = max(nmax, i + 1);
-          nmin = min(nmin, i + 1);
+    return;
+  }
+  const int i = threadIdx.x, mini = st->mini, maxi = st->maxi, n = st->n, j = st->jcount;
+  const double delta = st->delta, gg = lam / delta, om = st->omega, resd = st->resd;
+  const int cg = st->cg_return, maxcg = st->maxcg;
+  if (i < 64) {  // wave 0: the ballot spans every shift
+    const bool mine = i >= mini - 1 && i < maxi;
+    double z2 = 0.0, z3 = 0.0;
+    bool on = false;
+    if (i < n) {
+      z2 = st->zeta_ii[i];
+      if (mine) {
+        z3 = st->zeta_iii[i];
+        const double omi = st->omegas[i], ga = gg * z3 * omi / (z2 * om);
+        st->gammas[i] = ga;
+        st->cg_returns[i] = cg;
+        if constexpr (REC) {
+          st->rec_om[j][i] = omi;
+          st->rec_ga[j][i] = ga;
+          st->rec_ze[j][i] = z3;
+          st->cnt[i] = j + 1;
         }
       }
+      on = st->flags[i] && !(sqrt(delta * z2 * z2) * st->corr[i] < resd);
+      if (!on) st->flags[i] = 0;
     }
-    st->maxi = nmax;
-    st->mini = nmin;
-    for (int i = nmin - 1; i < nmax; i++) {
-      st->zeta_i[i] = st->zeta_ii[i];
-      st->zeta_ii[i] = st->zeta_iii[i];
+    const unsigned long long live = __ballot(on);
+    const int nmax = live ? 64 - __clzll(live) : 0, nmin = live ? __ffsll((long long)live) : n + 1;
+    // the window only shrinks, so its shifts have their zeta in registers
+    if (i >= nmin - 1 && i < nmax) {
+      st->zeta_i[i] = z2;
+      st->zeta_ii[i] = z3;
     }
+    if (i == 0) {
+      s_nmin = nmin;
+      s_nmax = nmax;
+    }
+  }
+  __syncthreads();  // also: every thread has read the scalars
+  if (threadIdx.x == 0) {
+    st->lambda = lam;
+    st->gammag = gg;
+    st->umin = mini;
+    st->umax = maxi;
+    st->mini = s_nmin;
+    st->maxi = s_nmax;
     st->delta = lam;
-    if (!(st->maxi > st->mini - 1 && st->cg_return < st->maxcg)) st->stop = 1;
+    if (REC) st->jcount = j + 1;
+    if (!(s_nmax > s_nmin - 1 && cg < maxcg)) st->stop = 1;
+  }
+}
+
+// The block's coefficients from its recorded scalars, one thread per shift.
+// With p_{j+1} = g_j p_j + z_j R_j and x_{j+1} = x_j - o_j p_j (shift i, j =
+// 0 .. c-1), backwards over j: the weight of R_j in the last p is z_j times
+// the product of the later g, and in x it is -z_j G_j with
+// G_{j-1} = o_j + g_j G_j.  O(c) per shift and block, instead of updating c
+// coefficients in every iteration.
+__global__ __launch_bounds__(64) void k_ms_coef(MsState *st) {
+  const int i = threadIdx.x, n = st->n;
+  if (i < n) {
+    const int c = st->cnt[i];
+    double g = 0.0, prod = 1.0;
+    for (int q = MSR - 1; q >= 0; q--) {
+      double b = 0.0, d = 0.0;
+      if (q < c) {
+        const double ze = st->rec_ze[q][i], ga = st->rec_ga[q][i];
+        b = ze * prod;
+        d = -(ze * g);
+        prod *= ga;
+        g = st->rec_om[q][i] + ga * g;
+      }
+      st->cb[i][q] = b;
+      st->cd[i][q] = d;
+    }
+    st->ca[i] = prod;
+    st->cc[i] = -g;
+    st->fcnt[i] = c;
+    st->fact[i] = !st->stop && i >= st->mini - 1 && i < st->maxi;
+    st->cnt[i] = 0;
+  }
+  if (i == 0) {
+    st->fjc = st->jcount;
+    st->jcount = 0;
+  }
+}
+
+// x_i, p_i of every shift that the block updated, from its residuals R_0 ..
+// R_{c-1}: ring slot q of residual j = t0 + q.  Bound by memory: one read of
+// each residual and, per shift, p and x read and written (c + 4 k field
+// streams per block of c iterations, against 4 k + 3 per iteration when every
+// iteration updates its shifts).  The residuals of an element stay in
+// registers for all shifts.  The first block starts from p_i = b, x_i = 0 and
+// writes every shift (x_i = 0 where nothing was updated).
+__global__ __launch_bounds__(BLK) void k_ms_flush(long ns, const MsState *S, const double2 *b,
+                                                  const double2 *ring, double2 *X, double2 *P,
+                                                  int first) {
+  const int jc = S->fjc, n = S->n;
+  if (jc == 0 && !first) return;
+  __shared__ double sa[MAXSHIFT], sc[MAXSHIFT], sb[MAXSHIFT][MSR], sd[MAXSHIFT][MSR];
+  __shared__ int scnt[MAXSHIFT], sact[MAXSHIFT];
+  for (int k = threadIdx.x; k < n * MSR; k += BLK) {
+    (&sb[0][0])[k] = (&S->cb[0][0])[k];
+    (&sd[0][0])[k] = (&S->cd[0][0])[k];
+  }
+  for (int k = threadIdx.x; k < n; k += BLK) {
+    sa[k] = S->ca[k];
+    sc[k] = S->cc[k];
+    scnt[k] = S->fcnt[k];
+    sact[k] = S->fact[k];
+  }
+  __syncthreads();
+  const long e = (long)blockIdx.x * BLK + threadIdx.x;
+  if (e >= ns) return;
+  cx<double> R[MSR];
+#pragma unroll
+  for (int q = 0; q < MSR; q++) R[q] = q < jc ? ldc(ring, q * ns + e) : cx<double>{0.0, 0.0};
+  const cx<double> bv = first ? ldc(b, e) : cx<double>{0.0, 0.0};
+  for (int i = 0; i < n; i++) {
+    if (!scnt[i]) {
+      if (first) st(X, i * ns + e, cx<double>{0.0, 0.0});
+      if (first && sact[i]) st(P, i * ns + e, bv);
+      continue;
+    }
+    const cx<double> base = first ? bv : ldc(P, i * ns + e);
+    cx<double> x = first ? cx<double>{0.0, 0.0} : ldc(X, i * ns + e);
+    x = x + sc[i] * base;
+    if (sact[i]) {
+      cx<double> p = sa[i] * base;
+#pragma unroll
+      for (int q = 0; q < MSR; q++) {
+        if (q < jc) {
+          x = x + sd[i][q] * R[q];
+          p = p + sb[i][q] * R[q];
+        }
+      }
+      st(P, i * ns + e, p);
+    } else {
+#pragma unroll
+      for (int q = 0; q < MSR; q++)
+        if (q < jc) x = x + sd[i][q] * R[q];
+    }
+    st(X, i * ns + e, x);
   }
 }
 
@@ -516,48 +668,38 @@ int apply_op(const OpDesc &op, int dagger, const double2 *in, double2 *out, hipS
   return launch_dslash(L, s);
 }
 
-// M or M^+ with a fused (Shamir) or separate (Wilson) epilogue, FP64
-static int apply_op_epi(const OpDesc &op, int dagger, const double2 *in, double2 *out, int mode,
-                        const double2 *w, double2 *r, double2 *x, const double2 *p,
-                        const double *a, const double *b, double *partial, const int *stop,
-                        hipStream_t s) {
+// M or M^+ with a fused (Shamir) or separate (Wilson) epilogue, FP64.  L
+// holds the epilogue's fields (mode, in, out, w, r, r_out, x, p, a_ptr,
+// b_ptr, partial, done) and dagger; cfg is the solve's launch shape
+static int apply_op_epi(const OpDesc &op, DslashLaunch L, const DslashConfig &cfg, hipStream_t s) {
   if (op.kernel == 1) {
-    // skip when stopped: the Wilson path is unfused, so gate the whole sequence
-    double2 *o = out ? out : (double2 *)workspace(2, sizeof(double2) * op.d.nspinor());
+    // the operator's passes are not gated by the stop flag, the epilogue is
+    const bool direct = L.out && L.mode != EPI_HREC;  // HREC reads the old out
+    double2 *o = direct ? (double2 *)L.out : (double2 *)workspace(2, sizeof(double2) * op.d.nspinor());
     double2 *tmp = (double2 *)workspace(1, sizeof(double2) * op.d.nspinor());
     THR_CHECK(o && tmp, THR_ERR_HIP, "workspace allocation failed");
-    int rc = launch_dslash_wilson(op.d, 1, dagger, op.imass, op.am, op.am3, in, o, op.u64, tmp, s);
-    if (rc) return rc;
-    if (mode != EPI_STORE) {
-      hipLaunchKernelGGL(k_epi, dim3(nblk(op.d.v5())), dim3(BLK), 0, s, op.d.v5(), mode, o, w, r,
-                         x, p, a, b, stop, partial, (int)dslash_blocks(op.d));
+    TRY_RC(launch_dslash_wilson(op.d, 1, L.dagger, op.imass, op.am, op.am3, (const double2 *)L.in, o,
+                                op.u64, tmp, s));
+    if (L.mode != EPI_STORE) {
+      hipLaunchKernelGGL(k_epi, dim3(nblk(op.d.v5())), dim3(BLK), 0, s, op.d.v5(), L.mode, o,
+                         (const double2 *)L.w, (const double2 *)L.r,
+                         (double2 *)(L.r_out ? L.r_out : L.r),
+                         (double2 *)(L.mode == EPI_HREC ? L.out : L.x), (const double2 *)L.p,
+                         L.a_ptr, L.b_ptr, L.done, L.partial, (int)dslash_blocks(op.d));
       THR_HIP(hipGetLastError());
     }
     return THR_OK;
   }
-  DslashLaunch L{};
   L.d = op.d;
   L.nrhs = 1;
   L.prec = P64;
-  L.dagger = dagger;
   L.imass = op.imass;
   L.am3 = op.am3;
   L.am[0] = op.am;
-  L.in = in;
-  L.out = out;
   L.links = op.u64;
-  L.mode = mode;
-  L.w = w;
-  L.r = r;
-  L.x = x;
-  L.p = p;
-  L.a_ptr = a;
-  L.b_ptr = b;
   L.sc_stride = 1;
-  L.partial = partial;
-  L.done = stop;
   L.done_stride = 1;
-  return launch_dslash(L, s);
+  return launch_dslash_cfg(L, cfg, s);
 }
 
 // poll a device int every `batch` iterations; batches grow to bound host syncs.
@@ -632,14 +774,28 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
   THR_HIP(hipMemcpyAsync(r, phi, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
   hipLaunchKernelGGL(k_cg_init, dim3(1), dim3(1), 0, s, st, resid, niterc);
   const int *stop = &st->stop;
+  const DslashConfig cfg = dslash_config(d, P64);
   auto iter = [&]() -> int {
-    int rc = apply_op_epi(op, 0, p, x1, EPI_NORM, nullptr, nullptr, nullptr, nullptr, nullptr,
-                          nullptr, partial, stop, s);
-    if (rc) return rc;
+    DslashLaunch a{};
+    a.in = p;
+    a.out = x1;
+    a.mode = EPI_NORM;
+    a.partial = partial;
+    a.done = stop;
+    TRY_RC(apply_op_epi(op, a, cfg, s));
     hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
-    rc = apply_op_epi(op, 1, x1, nullptr, EPI_CG, nullptr, r, x, p, &st->alpha, &st->alpha_x,
-                      partial, stop, s);
-    if (rc) return rc;
+    DslashLaunch c{};
+    c.dagger = 1;
+    c.in = x1;
+    c.mode = EPI_CG;
+    c.r = r;
+    c.x = x;
+    c.p = p;
+    c.a_ptr = &st->alpha;
+    c.b_ptr = &st->alpha_x;
+    c.partial = partial;
+    c.done = stop;
+    TRY_RC(apply_op_epi(op, c, cfg, s));
     hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_cg_p, dim3(nblk(n)), dim3(BLK), 0, s, n, r, p, st);
     THR_HIP(hipGetLastError());
@@ -660,8 +816,11 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
 static int ms_setup(MsState *st, int n, const double *aden, const double *anum, float res,
                     int maxcg, hipStream_t s, int plain = 0) {
   THR_CHECK(n >= 1 && n <= MAXSHIFT, THR_ERR_ARG, "number of shifts out of range");
-  MsState h;
-  std::memset(&h, 0, sizeof(h));
+  MsState *hp = (MsState *)host_workspace(20, sizeof(MsState));
+  THR_CHECK(hp, THR_ERR_HIP, "host workspace allocation failed");
+  MsState &h = *hp;
+  const size_t head = offsetof(MsState, rec_om);  // the rest is written before it is read
+  std::memset(&h, 0, head);
   h.n = n;
   h.res = res;
   h.maxcg = maxcg;
@@ -677,9 +836,75 @@ static int ms_setup(MsState *st, int n, const double *aden, const double *anum, 
     h.aden[i] = aden[i];
   }
   h.plain = plain;
-  THR_HIP(hipMemcpyAsync(st, &h, sizeof(h), hipMemcpyHostToDevice, s));
-  THR_HIP(hipStreamSynchronize(s));  // h is a stack object
+  THR_HIP(hipMemcpyAsync(st, &h, head, hipMemcpyHostToDevice, s));
+  THR_HIP(hipStreamSynchronize(s));  // the pinned copy is written again by the read-back
   return THR_OK;
+}
+
+// the solve's counts and its error, read back from the device state
+static int ms_result(const MsState *st, int n, int *cg_return, int *cg_returns, hipStream_t s) {
+  MsState *h = (MsState *)host_workspace(20, sizeof(MsState));
+  THR_CHECK(h, THR_ERR_HIP, "host workspace allocation failed");
+  const size_t head = offsetof(MsState, rec_om);  // the counts and flags lie before the records
+  THR_HIP(hipMemcpyAsync(h, st, head, hipMemcpyDeviceToHost, s));
+  THR_HIP(hipStreamSynchronize(s));
+  *cg_return = h->cg_return;
+  if (cg_returns)
+    for (int i = 0; i < n; i++) cg_returns[i] = h->cg_returns[i];
+  THR_CHECK(!h->nonfinite, THR_ERR_NONFINITE,
+            "multishift: non-finite dot product (NaN or Inf in the source or links)");
+  return THR_OK;
+}
+
+// The same solve with the shift vectors updated once per block of MSR
+// iterations (k_ms_coef, k_ms_flush) and neither p nor M^+M p stored: alpha =
+// |M p|^2 comes from the M pass, h = M p obeys h_new = M r_new + gamma h (M is
+// linear), and the M^+ pass updates r in its epilogue, into the next slot of
+// the residual ring.  16^3 x 48, 25 poles: 195 us per iteration with the shift
+// updates in every iteration (four streams per active shift: 120 us), of which
+// this leaves the two operator passes and (MSR + 4 k) / MSR streams.
+static int multishift_blocked(const OpDesc &op, int n, const double2 *input, double2 *out,
+                              MsState *st, double2 *h, double2 *ring, double2 *P, double *partial,
+                              int maxcg, const DslashConfig &cfg, hipStream_t s) {
+  const Dims &d = op.d;
+  const long ns = d.nspinor();
+  // the entries that the operator's epilogue fills
+  const int nbl = op.kernel == 0 ? (int)dslash_grid_blocks(d, cfg) : (int)nblk(d.v5());
+  int *stop = (int *)host_workspace(21, sizeof(int));
+  THR_CHECK(stop, THR_ERR_HIP, "host workspace allocation failed");
+  for (long t0 = 0;; t0 += MSR) {
+    for (long t = t0; t < t0 + MSR; t++) {
+      const double2 *rin = t == 0 ? input : ring + ((t - 1) % MSR) * ns;
+      DslashLaunch a{};
+      a.in = rin;
+      a.out = h;
+      a.mode = t == 0 ? EPI_NORM : EPI_HREC;
+      a.b_ptr = t == 0 ? nullptr : &st->gammag;
+      a.partial = partial;
+      a.done = &st->stop;
+      TRY_RC(apply_op_epi(op, a, cfg, s));
+      hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
+      DslashLaunch b{};
+      b.dagger = 1;
+      b.in = h;
+      b.mode = EPI_CG;
+      b.r = const_cast<double2 *>(rin);
+      b.r_out = ring + (t % MSR) * ns;
+      b.a_ptr = &st->minus_omega;
+      b.partial = partial;
+      b.done = &st->stop;
+      TRY_RC(apply_op_epi(op, b, cfg, s));
+      hipLaunchKernelGGL(k_ms_lambda<true>, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
+    }
+    hipLaunchKernelGGL(k_ms_coef, dim3(1), dim3(64), 0, s, st);
+    hipLaunchKernelGGL(k_ms_flush, dim3(nblk(ns)), dim3(BLK), 0, s, ns, st, input, ring, out, P,
+                       t0 == 0 ? 1 : 0);
+    THR_HIP(hipGetLastError());
+    THR_HIP(hipMemcpyAsync(stop, &st->stop, sizeof(int), hipMemcpyDeviceToHost, s));
+    THR_HIP(hipStreamSynchronize(s));
+    if (*stop) return THR_OK;
+    THR_CHECK(t0 <= (long)maxcg + 2 * MSR, THR_ERR_STATE, "solver did not raise its stop flag");
+  }
 }
 
 int multishift_reference(const OpDesc &op, int n, const double *aden, const double *anum,
@@ -688,50 +913,67 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   const Dims &d = op.d;
   const long ns = d.nspinor();
   const int nb = (int)dslash_blocks(d);
-  double2 *r = (double2 *)workspace(20, sizeof(double2) * ns);
   double2 *h = (double2 *)workspace(21, sizeof(double2) * ns);
-  double2 *sv = (double2 *)workspace(22, sizeof(double2) * ns);
-  double2 *p = (double2 *)workspace(23, sizeof(double2) * ns);
   double2 *ps = (double2 *)workspace(24, sizeof(double2) * ns * n);
   MsState *st = (MsState *)workspace(25, sizeof(MsState));
   double *partial = partial_buffer(nb);
-  THR_CHECK(r && h && sv && p && ps && st && partial, THR_ERR_HIP, "workspace allocation failed");
+  THR_CHECK(h && ps && st && partial, THR_ERR_HIP, "workspace allocation failed");
+  // Blocked updates keep MSR residuals (16 GiB at most here: 512 MiB fields;
+  // 32^3 x 64 takes 4.3); larger fields, and contexts where the ring does not
+  // fit beside the caller's memory, update every shift in every iteration.
+  const size_t ring_bytes = sizeof(double2) * ns * MSR;
+  double2 *ring = nullptr;
+  if (ring_bytes <= (size_t(16) << 30)) {
+    ring = (double2 *)workspace(26, ring_bytes);
+    if (!ring) (void)hipGetLastError();
+  }
   int rc = ms_setup(st, n, aden, anum, res, maxcg, s, plain);
   if (rc) return rc;
+  const DslashConfig cfg = dslash_config(d, P64);
+  hipLaunchKernelGGL(k_norm<P64>, dim3(nb), dim3(BLK), 0, s, d.v5(), input, partial);
+  hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+  THR_HIP(hipGetLastError());
+  if (ring) {
+    TRY_RC(multishift_blocked(op, n, input, out, st, h, ring, ps, partial, maxcg, cfg, s));
+    return ms_result(st, n, cg_return, cg_returns, s);
+  }
+  double2 *r = (double2 *)workspace(20, sizeof(double2) * ns);
+  double2 *sv = (double2 *)workspace(22, sizeof(double2) * ns);
+  double2 *p = (double2 *)workspace(23, sizeof(double2) * ns);
+  THR_CHECK(r && sv && p, THR_ERR_HIP, "workspace allocation failed");
   THR_HIP(hipMemcpyAsync(r, input, sizeof(double2) * ns, hipMemcpyDeviceToDevice, s));
   THR_HIP(hipMemcpyAsync(p, input, sizeof(double2) * ns, hipMemcpyDeviceToDevice, s));
   THR_HIP(hipMemsetAsync(out, 0, sizeof(double2) * ns * n, s));
   hipLaunchKernelGGL(k_bcast_copy<P64>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, n, input, ps);
-  hipLaunchKernelGGL(k_norm<P64>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, partial);
-  hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(BLK), 0, s, st, partial, nb);
   THR_HIP(hipGetLastError());
   const int *stop = &st->stop;
   auto iter = [&]() -> int {
-    int rc2 = apply_op_epi(op, 0, p, h, EPI_STORE, nullptr, nullptr, nullptr, nullptr, nullptr,
-                           nullptr, nullptr, stop, s);
-    if (rc2) return rc2;
-    rc2 = apply_op_epi(op, 1, h, sv, EPI_DOTW, p, nullptr, nullptr, nullptr, nullptr, nullptr,
-                       partial, stop, s);
-    if (rc2) return rc2;
+    DslashLaunch a{};
+    a.in = p;
+    a.out = h;
+    a.mode = EPI_STORE;
+    a.done = stop;
+    TRY_RC(apply_op_epi(op, a, cfg, s));
+    DslashLaunch b{};
+    b.dagger = 1;
+    b.in = h;
+    b.out = sv;
+    b.mode = EPI_DOTW;
+    b.w = p;
+    b.partial = partial;
+    b.done = stop;
+    TRY_RC(apply_op_epi(op, b, cfg, s));
     hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_axpy_norm<P64>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, sv, &st->omega,
                        stop, partial);
-    hipLaunchKernelGGL(k_ms_lambda, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+    hipLaunchKernelGGL(k_ms_lambda<false>, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_ms_update<P64>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, r, p, out, ps, st);
     THR_HIP(hipGetLastError());
     return THR_OK;
   };
   rc = run_batched(iter, stop, s, maxcg);
   if (rc) return rc;
-  MsState hs;
-  THR_HIP(hipMemcpyAsync(&hs, st, sizeof(MsState), hipMemcpyDeviceToHost, s));
-  THR_HIP(hipStreamSynchronize(s));
-  *cg_return = hs.cg_return;
-  if (cg_returns)
-    for (int i = 0; i < n; i++) cg_returns[i] = hs.cg_returns[i];
-  THR_CHECK(!hs.nonfinite, THR_ERR_NONFINITE,
-            "multishift: non-finite dot product (NaN or Inf in the source or links)");
-  return THR_OK;
+  return ms_result(st, n, cg_return, cg_returns, s);
 }
 
 int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const double *anum,
@@ -796,7 +1038,7 @@ int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const d
     hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_axpy_norm<P32>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, sv, &st->omega,
                        stop, partial);
-    hipLaunchKernelGGL(k_ms_lambda, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+    hipLaunchKernelGGL(k_ms_lambda<false>, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_ms_update<P32>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, r, p, xs, ps, st);
     THR_HIP(hipGetLastError());
     return THR_OK;
@@ -804,15 +1046,7 @@ int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const d
   rc = run_batched(iter, stop, s, maxcg);
   if (rc) return rc;
   TRY_RC(convert_spinors(d, n, xs, nullptr, P32, out, nullptr, P64, s));
-  MsState hs;
-  THR_HIP(hipMemcpyAsync(&hs, st, sizeof(MsState), hipMemcpyDeviceToHost, s));
-  THR_HIP(hipStreamSynchronize(s));
-  *cg_return = hs.cg_return;
-  if (cg_returns)
-    for (int i = 0; i < n; i++) cg_returns[i] = hs.cg_returns[i];
-  THR_CHECK(!hs.nonfinite, THR_ERR_NONFINITE,
-            "multishift: non-finite dot product (NaN or Inf in the source or links)");
-  return THR_OK;
+  return ms_result(st, n, cg_return, cg_returns, s);
 }
 
 }  // namespace thr
