@@ -81,3 +81,49 @@ def test_wilson_congrad_after_a_larger_shamir_solve(G):
     o = O.congrad(phi, xo, u, dims, res=1e-3, am=0.1, imass=3, kernel="wilson")
     assert g == o
     assert rel(O.interior(xg), O.interior(xo)) <= 1e-10
+
+
+# s-lines in segments of 1, 4, 16, 32 and 64 lanes, filled and part filled;
+# Ls = 80 takes the kernel that walks the slice pairs
+@pytest.mark.parametrize("dims", [(4, 3, 2, 1), (3, 5, 4, 4), (5, 3, 4, 12), (3, 3, 5, 20),
+                                  (4, 5, 3, 48), (2, 3, 3, 64), (3, 2, 3, 80)])
+@pytest.mark.parametrize("iflag", [0, 1])
+@pytest.mark.parametrize("imass", [1, 3])
+def test_derivs_wilson_lines(G, imass, iflag, dims):
+    """The sums have 8 Ls terms of equal size: 1e-12 as for the Shamir force."""
+    rng = np.random.default_rng(35)
+    R, X2 = D.rand_spinor(dims, rng), D.rand_spinor(dims, rng)
+    base = np.asfortranarray(rng.standard_normal(dims[:3] + (3,)))
+    print("case: derivs wilson", dims, imass, iflag, flush=True)
+    a = dict(kernel="wilson", am=0.3, imass=imass)
+    dg = G.derivs(R, X2, 0.37, iflag, dims, base.copy(order="F"), **a)
+    do = O.derivs(R, X2, 0.37, iflag, dims, base.copy(order="F"), **a)
+    assert rel(dg - base, do - base) <= 1e-12
+
+
+@pytest.mark.parametrize("dims", [(4, 3, 2, 1), (3, 5, 4, 4), (5, 3, 4, 12), (3, 3, 5, 20),
+                                  (4, 5, 3, 48), (2, 3, 3, 64), (3, 2, 3, 80)])
+@pytest.mark.parametrize("imass", [1, 3])
+def test_dslash_wilson_lines(G, imass, dims):
+    """The Wilson-kernel operator on the same line lengths, to the Dslash tolerance 1e-13."""
+    rng, u = smooth(dims, 36)
+    r = D.rand_spinor(dims, rng)
+    print("case: dslash wilson", dims, imass, flush=True)
+    for g, o in ((G.dslash, O.dslash), (G.dslashd, O.dslashd)):
+        a = g(r, u, dims, 0.3, imass, kernel="wilson")
+        b = o(r, u, dims, 0.3, imass, kernel="wilson")
+        assert rel(O.interior(a), O.interior(b)) <= 1e-13
+
+
+@pytest.mark.parametrize("dims", [(14, 14, 3, 20), (3, 5, 4, 4), (3, 2, 3, 80)])
+def test_congrad_wilson_lines(G, dims):
+    """The fused epilogues of the Wilson kernel (more blocks than the Shamir
+    grid at 14 x 14 x 20) and, above Ls = 64, the separate ones."""
+    rng, u = smooth(dims, 37)
+    phi = D.rand_spinor(dims, rng)
+    xg, xo = np.zeros_like(phi), np.zeros_like(phi)
+    print("case: congrad wilson", dims, flush=True)
+    g = G.congrad(phi, xg, u, dims, res=1e-2, am=0.2, imass=3, kernel="wilson")
+    o = O.congrad(phi, xo, u, dims, res=1e-2, am=0.2, imass=3, kernel="wilson")
+    assert g == o
+    assert rel(O.interior(xg), O.interior(xo)) <= 1e-11

@@ -107,10 +107,14 @@ void dslash_set_config(const Dims &d, int prec, DslashConfig c, int which = -1);
 int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *best,
                     hipStream_t s, int nrhs = 1);
 
-// Wilson-kernel operator on device (FP64): slice-composed, imass 1 or 3
+// Wilson-kernel operator on device (FP64), imass 1 or 3; tmp: a scratch spinor,
+// used for Ls > 64 only
 int launch_dslash_wilson(const Dims &d, int nrhs, int dagger, int imass, float am, float am3,
                          const double2 *in, double2 *out, const double2 *links, double2 *tmp,
                          hipStream_t s);
+// the same with L's epilogue (fields as for launch_dslash), Ls <= 64; partial sums: wilson_blocks(d) per right-hand side
+int launch_wilson_epi(DslashLaunch L, hipStream_t s);
+long wilson_blocks(const Dims &d);
 
 // layout conversion between the reference's haloed complex128 arrays and the
 // device layout; prec selects the device storage

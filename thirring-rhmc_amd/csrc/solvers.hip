@@ -203,12 +203,11 @@ __global__ __launch_bounds__(BLK) void k_norm(long v5, const TT<P> *x, double *p
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// epilogues for operators that cannot fuse them (Wilson kernel); the sums
-// take nb entries, so block 0 zero-fills those past this grid
+// epilogues for operators that cannot fuse them (Wilson kernel, Ls > 64)
 __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o, const double2 *w,
                                              const double2 *r, double2 *ro, double2 *x,
                                              const double2 *p, const double *a, const double *b,
-                                             const int *stop, double *partial, int nb) {
+                                             const int *stop, double *partial) {
   if (stop && *stop) return;
   const long i = (long)blockIdx.x * BLK + threadIdx.x;
   double red = 0.0;
@@ -235,8 +234,6 @@ __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o
   }
   const double t = block_sum(red);
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
-  if (blockIdx.x == 0)
-    for (int k = (int)(gridDim.x + threadIdx.x); k < nb; k += BLK) partial[k] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -647,8 +644,11 @@ int convert_d2f(long n, const double2 *a, float2 *b, hipStream_t s) {
 
 int apply_op(const OpDesc &op, int dagger, const double2 *in, double2 *out, hipStream_t s) {
   if (op.kernel == 1) {
-    double2 *tmp = (double2 *)workspace(1, sizeof(double2) * op.d.nspinor());
-    THR_CHECK(tmp, THR_ERR_HIP, "workspace allocation failed");
+    double2 *tmp = nullptr;
+    if (op.d.ls > 64) {
+      tmp = (double2 *)workspace(1, sizeof(double2) * op.d.nspinor());
+      THR_CHECK(tmp, THR_ERR_HIP, "workspace allocation failed");
+    }
     return launch_dslash_wilson(op.d, 1, dagger, op.imass, op.am, op.am3, in, out, op.u64, tmp, s);
   }
   DslashLaunch L{};
@@ -668,10 +668,20 @@ int apply_op(const OpDesc &op, int dagger, const double2 *in, double2 *out, hipS
   return launch_dslash(L, s);
 }
 
-// M or M^+ with a fused (Shamir) or separate (Wilson) epilogue, FP64.  L
+// M or M^+ with a fused or (Wilson kernel, Ls > 64) separate epilogue, FP64.  L
 // holds the epilogue's fields (mode, in, out, w, r, r_out, x, p, a_ptr,
 // b_ptr, partial, done) and dagger; cfg is the solve's launch shape
 static int apply_op_epi(const OpDesc &op, DslashLaunch L, const DslashConfig &cfg, hipStream_t s) {
+  L.d = op.d;
+  L.nrhs = 1;
+  L.prec = P64;
+  L.imass = op.imass;
+  L.am3 = op.am3;
+  L.am[0] = op.am;
+  L.links = op.u64;
+  L.sc_stride = 1;
+  L.done_stride = 1;
+  if (op.kernel == 1 && op.d.ls <= 64) return launch_wilson_epi(L, s);
   if (op.kernel == 1) {
     // the operator's passes are not gated by the stop flag, the epilogue is
     const bool direct = L.out && L.mode != EPI_HREC;  // HREC reads the old out
@@ -685,21 +695,17 @@ static int apply_op_epi(const OpDesc &op, DslashLaunch L, const DslashConfig &cf
                          (const double2 *)L.w, (const double2 *)L.r,
                          (double2 *)(L.r_out ? L.r_out : L.r),
                          (double2 *)(L.mode == EPI_HREC ? L.out : L.x), (const double2 *)L.p,
-                         L.a_ptr, L.b_ptr, L.done, L.partial, (int)dslash_blocks(op.d));
+                         L.a_ptr, L.b_ptr, L.done, L.partial);
       THR_HIP(hipGetLastError());
     }
     return THR_OK;
   }
-  L.d = op.d;
-  L.nrhs = 1;
-  L.prec = P64;
-  L.imass = op.imass;
-  L.am3 = op.am3;
-  L.am[0] = op.am;
-  L.links = op.u64;
-  L.sc_stride = 1;
-  L.done_stride = 1;
   return launch_dslash_cfg(L, cfg, s);
+}
+
+// the partial sums that an operator's epilogue writes, all of them
+static int op_partials(const OpDesc &op, const DslashConfig &cfg) {
+  return (int)(op.kernel == 1 ? wilson_blocks(op.d) : dslash_grid_blocks(op.d, cfg));
 }
 
 // poll a device int every `batch` iterations; batches grow to bound host syncs.
@@ -749,7 +755,7 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
   B.r = (double2 *)workspace(11, sizeof(double2) * n);
   B.p = (double2 *)workspace(12, sizeof(double2) * n);
   B.state = workspace(13, sizeof(CgState));
-  B.partial = partial_buffer((int)dslash_blocks(d));
+  B.partial = partial_buffer((int)std::max(dslash_blocks(d), wilson_blocks(d)));
   THR_CHECK(B.x1 && B.r && B.p && B.state && B.partial, THR_ERR_HIP,
             "workspace allocation failed");
   return cg_reference_bufs(op, phi, x, res, niterc, itercg, iterations, s, B, nullptr);
@@ -760,7 +766,8 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
                       int *host_flag) {
   const Dims &d = op.d;
   const long n = d.nspinor();
-  const int nb = (int)dslash_blocks(d);
+  const DslashConfig cfg = dslash_config(d, P64);
+  const int nb = op_partials(op, cfg);
   double2 *x1 = B.x1, *r = B.r, *p = B.p;
   CgState *st = (CgState *)B.state;
   double *partial = B.partial;
@@ -774,7 +781,6 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
   THR_HIP(hipMemcpyAsync(r, phi, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
   hipLaunchKernelGGL(k_cg_init, dim3(1), dim3(1), 0, s, st, resid, niterc);
   const int *stop = &st->stop;
-  const DslashConfig cfg = dslash_config(d, P64);
   auto iter = [&]() -> int {
     DslashLaunch a{};
     a.in = p;
@@ -868,8 +874,7 @@ static int multishift_blocked(const OpDesc &op, int n, const double2 *input, dou
                               int maxcg, const DslashConfig &cfg, hipStream_t s) {
   const Dims &d = op.d;
   const long ns = d.nspinor();
-  // the entries that the operator's epilogue fills
-  const int nbl = op.kernel == 0 ? (int)dslash_grid_blocks(d, cfg) : (int)nblk(d.v5());
+  const int nbl = op_partials(op, cfg);
   int *stop = (int *)host_workspace(21, sizeof(int));
   THR_CHECK(stop, THR_ERR_HIP, "host workspace allocation failed");
   for (long t0 = 0;; t0 += MSR) {
@@ -916,7 +921,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   double2 *h = (double2 *)workspace(21, sizeof(double2) * ns);
   double2 *ps = (double2 *)workspace(24, sizeof(double2) * ns * n);
   MsState *st = (MsState *)workspace(25, sizeof(MsState));
-  double *partial = partial_buffer(nb);
+  double *partial = partial_buffer((int)std::max<long>(nb, wilson_blocks(d)));
   THR_CHECK(h && ps && st && partial, THR_ERR_HIP, "workspace allocation failed");
   // Blocked updates keep MSR residuals (16 GiB at most here: 512 MiB fields;
   // 32^3 x 64 takes 4.3); larger fields, and contexts where the ring does not
@@ -947,6 +952,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   hipLaunchKernelGGL(k_bcast_copy<P64>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, n, input, ps);
   THR_HIP(hipGetLastError());
   const int *stop = &st->stop;
+  const int nbl = op_partials(op, cfg);
   auto iter = [&]() -> int {
     DslashLaunch a{};
     a.in = p;
@@ -963,7 +969,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
     b.partial = partial;
     b.done = stop;
     TRY_RC(apply_op_epi(op, b, cfg, s));
-    hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+    hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
     hipLaunchKernelGGL(k_axpy_norm<P64>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, sv, &st->omega,
                        stop, partial);
     hipLaunchKernelGGL(k_ms_lambda<false>, dim3(1), dim3(BLK), 0, s, st, partial, nb);

@@ -8,7 +8,9 @@
 //        Q(s) = P+ R(s-1) + P- R(s+1)       (interior s)
 //             + c1 P+ R(Ls) at s=1, c2 P- R(1) at s=Ls
 //   M^+R = T + R + P- cA (T - R)(s_A) + P+ cB (T - R)(s_B),  T = D_W^+ R
-// so each application is one 4-D stencil pass plus two local passes.
+// so each application is one 4-D stencil pass: the s-couplings come by wave
+// shuffles where an s-line fits one wave (Ls <= 64, k_wilson), and as two local
+// passes around the Dslash kernel's 4-D form above that.
 //
 // Force, derivs_module.F90:99-196: for every link (x, mu) the sum over s and
 // spin of the Wilson and Dirac parts of d/dtheta Re<R, M^(+) X2>, with the
@@ -17,11 +19,204 @@
 #include <cstdlib>
 #include <vector>
 
-#include "kernels.h"
+#include "dslash_site.h"
 
 namespace thr {
 
 namespace {
+
+__device__ inline void ld_spinor(const double2 *__restrict__ p, unsigned v5, unsigned site,
+                                 cx<double> v[4]) {
+#pragma unroll
+  for (int a = 0; a < 4; a++) v[a] = ldc(p, (long)a * v5 + site);
+}
+
+// The Wilson kernel's s-couplings of a spinor held one site per lane, an
+// s-line per segment of lanes: q = Q v with
+//   (Q v)(s) = P+ v(s-1) + P- v(s+1),  P+ the spins 1, 2 and P- the spins 3, 4,
+// and the wall terms c1 P+ v(Ls) at s = 1, c2 P- v(1) at s = Ls.  DAG: P+ and P-
+// trade places (c1 goes with s - 1 and c2 with s + 1 as before).  lane0: the
+// segment's first lane.  Every lane of the wave takes part.
+struct WallCoef {
+  double c1r, c1i, c2r, c2i;
+};
+template <bool DAG>
+__device__ inline void couplings(const cx<double> v[4], cx<double> q[4], unsigned s, unsigned ls,
+                                 unsigned lane0, const WallCoef &w) {
+  const int dn = (int)(lane0 + (s == 0 ? ls - 1 : s - 1)), up = (int)(lane0 + (s + 1 < ls ? s + 1 : 0));
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    const bool below = (a < 2) != DAG;
+    const int src = below ? dn : up;
+    const cx<double> n{__shfl(v[a].r, src, 64), __shfl(v[a].i, src, 64)};
+    const bool wall = below ? s == 0 : s + 1 == ls;
+    const cx<double> c = below ? cx<double>{w.c1r, w.c1i} : cx<double>{w.c2r, w.c2i};
+    q[a] = wall ? cmul(c, n) : n;
+  }
+}
+__device__ inline void add_couplings(cx<double> v[4], unsigned s, unsigned ls, unsigned lane0,
+                                     const WallCoef &w) {
+  cx<double> q[4];
+  couplings<false>(v, q, s, ls, lane0, w);
+#pragma unroll
+  for (int a = 0; a < 4; a++) v[a] = v[a] + q[a];
+}
+
+// One side of a 4-D hop of M (half_hop) on the P+ part of v (spins 1, 2) and
+// on its P- part (spins 3, 4) apart: A -= 1/2 (1 + SIG gamma_mu) U P+ v, B the
+// same of P- v.
+template <int MU, int SIG>
+__device__ inline void half_hop_split(cx<double> A[4], cx<double> B[4], cx<double> u,
+                                      const Site<P64> &S) {
+  constexpr int p0 = kGamP[MU][0], p1 = kGamP[MU][1];
+  constexpr double h = 0.5, hs = SIG > 0 ? 0.5 : -0.5;
+  const cx<double> w0 = cmul(u, S.v[0]), w1 = cmul(u, S.v[1]);
+  A[0] = A[0] - h * w0;
+  A[1] = A[1] - h * w1;
+  A[p0] = A[p0] - hs * phase<kGamE[MU][p0]>(w0);
+  A[p1] = A[p1] - hs * phase<kGamE[MU][p1]>(w1);
+  const cx<double> z0 = cmul(u, phase<kGamE[MU][0]>(S.v[p0])), z1 = cmul(u, phase<kGamE[MU][1]>(S.v[p1]));
+  B[0] = B[0] - hs * z0;
+  B[1] = B[1] - hs * z1;
+  B[p0] = B[p0] - h * phase<kGamE[MU][p0]>(z0);
+  B[p1] = B[p1] - h * phase<kGamE[MU][p1]>(z1);
+}
+
+// value of v at the segment's lane `src`, times c where it crossed the wall
+__device__ inline cx<double> from_line(cx<double> v, int src, bool wall, cx<double> c) {
+  const cx<double> n{__shfl(v.r, src, 64), __shfl(v.i, src, 64)};
+  return wall ? cmul(c, n) : n;
+}
+
+// smallest power of two >= ls (ls <= 64): lanes per s-line
+inline unsigned segment(int ls) {
+  unsigned w = 1;
+  while (w < (unsigned)ls) w <<= 1;
+  return w;
+}
+
+// Wilson-kernel M or M^+ with the epilogues of the Dslash kernel, FP64, Ls <=
+// 64: an s-line per lane segment, one site per lane, one t step per thread.
+//   M:   out = A + B + R + (A - P+ R)(s-1) + (B - P- R)(s+1) with A = D_W P+ R
+//        and B = D_W P- R (D_W is diagonal in s, so the shift along s may
+//        follow it: 8 shuffled numbers per site instead of 28 when Y = R + Q R
+//        is formed on each of the 7 loaded sites, and 11.3 us)
+//   M^+: out = T + R + Q^+ (T - R),  T = D_W^+ R
+// Bound by latency on the lattices this kernel is generated on (14^2 x 18 x
+// 20: 4.5 MB fields), so everything is one pass with all loads issued
+// together.  The passes it replaces took 16.5 us for M (couplings, stencil,
+// combination) and 18.4 for M^+ (stencil, couplings, epilogue) there; this one
+// takes 9.9 with its epilogue, and 7.8.
+template <bool DAG, int MODE>
+__global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigned wseg,
+                                                   const WallCoef wall) {
+  const int rhs = blockIdx.y;
+  if (L.done && L.done[(long)rhs * L.done_stride]) return;
+  const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
+  const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
+  const unsigned nl = BLK / wseg, nb2 = (v2 + nl - 1) / nl;  // lines per block, blocks per t
+  const unsigned t = blockIdx.x / nb2, lb = blockIdx.x - t * nb2;
+  const unsigned line = threadIdx.x / wseg, s = threadIdx.x - line * wseg;
+  const unsigned col = lb * nl + line;  // 2-D site x + lx y
+  const bool valid = s < ls && col < v2;
+  const unsigned lane0 = (threadIdx.x & 63) - s;
+  const long off = (long)rhs * 4 * v5;
+  const unsigned i = s + ls * col + v3 * t;
+  Site<P64> c{}, f[3]{}, b[3]{}, old{};  // old: the epilogue's h or r
+  cx<double> uf[3]{}, ub[3]{};
+  const double ea = MODE == EPI_CG ? L.a_ptr[(long)rhs * L.sc_stride] : 0.0;
+  const double eb = (MODE == EPI_HREC || (MODE == EPI_CG && L.b_ptr))
+                        ? L.b_ptr[(long)rhs * L.sc_stride] : 0.0;
+  if (valid) {
+    const double2 *in = (const double2 *)L.in + off, *u = (const double2 *)L.links;
+    const unsigned x = col % lx, y = col / lx;
+    const unsigned xf = x + 1 == lx ? 0 : x + 1, xb = x == 0 ? lx - 1 : x - 1;
+    const unsigned yf = y + 1 == ly ? 0 : y + 1, yb = y == 0 ? ly - 1 : y - 1;
+    const unsigned tf = t + 1 == lt ? 0 : t + 1, tb = t == 0 ? lt - 1 : t - 1;
+    ld_spinor(in, v5, i, c.v);
+    ld_spinor(in, v5, s + ls * (xf + lx * y) + v3 * t, f[0].v);
+    ld_spinor(in, v5, s + ls * (xb + lx * y) + v3 * t, b[0].v);
+    ld_spinor(in, v5, s + ls * (x + lx * yf) + v3 * t, f[1].v);
+    ld_spinor(in, v5, s + ls * (x + lx * yb) + v3 * t, b[1].v);
+    ld_spinor(in, v5, s + ls * col + v3 * tf, f[2].v);
+    ld_spinor(in, v5, s + ls * col + v3 * tb, b[2].v);
+    uf[0] = ldc(u, col + v2 * t);
+    ub[0] = conj(ldc(u, xb + lx * y + v2 * t));
+    uf[1] = ldc(u, v4 + col + v2 * t);
+    ub[1] = conj(ldc(u, v4 + x + lx * yb + v2 * t));
+    uf[2] = ldc(u, 2 * v4 + col + v2 * t);
+    ub[2] = conj(ldc(u, 2 * v4 + col + v2 * tb));
+    if constexpr (MODE == EPI_HREC) ld_spinor((const double2 *)L.out + off, v5, i, old.v);
+    if constexpr (MODE == EPI_CG) ld_spinor((const double2 *)L.r + off, v5, i, old.v);
+  }
+  const double diag = (double)(3.0f + (-L.am3));
+  cx<double> o[4];
+  if constexpr (!DAG) {
+    cx<double> A[4]{}, B[4]{};
+    A[0] = diag * c.v[0];
+    A[1] = diag * c.v[1];
+    B[2] = diag * c.v[2];
+    B[3] = diag * c.v[3];
+    half_hop_split<0, -1>(A, B, uf[0], f[0]);
+    half_hop_split<0, 1>(A, B, ub[0], b[0]);
+    half_hop_split<1, -1>(A, B, uf[1], f[1]);
+    half_hop_split<1, 1>(A, B, ub[1], b[1]);
+    half_hop_split<2, -1>(A, B, uf[2], f[2]);
+    half_hop_split<2, 1>(A, B, ub[2], b[2]);
+    const int dn = (int)(lane0 + (s == 0 ? ls - 1 : s - 1));
+    const int up = (int)(lane0 + (s + 1 < ls ? s + 1 : 0));
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      o[a] = A[a] + B[a] + c.v[a];
+      if (a < 2)
+        A[a] = A[a] - c.v[a];
+      else
+        B[a] = B[a] - c.v[a];
+      o[a] = o[a] + from_line(A[a], dn, s == 0, {wall.c1r, wall.c1i});
+      o[a] = o[a] + from_line(B[a], up, s + 1 == ls, {wall.c2r, wall.c2i});
+    }
+  } else {
+    centre(o, diag, c);
+    hop<0, DAG>(o, uf[0], f[0], ub[0], b[0]);
+    hop<1, DAG>(o, uf[1], f[1], ub[1], b[1]);
+    hop<2, DAG>(o, uf[2], f[2], ub[2], b[2]);
+    cx<double> w[4], q[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++) w[a] = o[a] - c.v[a];
+    couplings<true>(w, q, s, ls, lane0, wall);
+#pragma unroll
+    for (int a = 0; a < 4; a++) o[a] = o[a] + c.v[a] + q[a];
+  }
+  double red = 0.0;
+  if (valid) {
+    double2 *out = (double2 *)L.out + off;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      const long e = (long)a * v5 + i;
+      if constexpr (MODE == EPI_CG) {
+        const cx<double> rv = old.v[a] - ea * o[a];
+        st((double2 *)(L.r_out ? L.r_out : L.r) + off, e, rv);
+        red += norm2(rv);
+        if (L.b_ptr) {
+          double2 *xo = (double2 *)L.x + off;
+          st(xo, e, ldc(xo, e) + eb * ldc((const double2 *)L.p + off, e));
+        }
+      } else {
+        if constexpr (MODE == EPI_HREC) o[a] = o[a] + eb * old.v[a];
+        st(out, e, o[a]);
+        if constexpr (MODE == EPI_NORM || MODE == EPI_HREC) red += norm2(o[a]);
+        if constexpr (MODE == EPI_DOTW) {
+          const cx<double> wv = ldc((const double2 *)L.w + off, e);
+          red += wv.r * o[a].r + wv.i * o[a].i;
+        }
+      }
+    }
+  }
+  if constexpr (MODE != EPI_STORE) {
+    const double tot = block_sum(red);
+    if (threadIdx.x == 0) L.partial[(long)rhs * gridDim.x + blockIdx.x] = tot;
+  }
+}
 
 // Y = R + Q  (M) ; coefficients c1, c2 multiply the wall terms
 __global__ __launch_bounds__(BLK) void k_wk_pre(const Dims d, int nrhs, const double2 *R,
@@ -124,12 +319,6 @@ __device__ inline double derivs_term(const cx<double> R0[4], const cx<double> X0
   return w1 * sw + w2 * sd;
 }
 
-__device__ inline void ld_spinor(const double2 *__restrict__ p, unsigned v5, unsigned site,
-                                 cx<double> v[4]) {
-#pragma unroll
-  for (int a = 0; a < 4; a++) v[a] = ldc(p, (long)a * v5 + site);
-}
-
 // LDS x exchange of the batched derivs: with 64-lane segments (32 < Ls <=
 // 64) and Lx % 4 == 0 a block's 4 waves are 4 consecutive x of one (y, t),
 // so the x+1 neighbour of waves 0-2 is the centre of the next wave: each wave
@@ -163,10 +352,20 @@ struct DXBuf {
 // butterfly of wave shuffles inside the segment (a fixed order, no LDS and no
 // block barrier); segment lane 0 adds the three link terms into dSdpi.  The
 // t march and loads are those of k_derivs_march below.
+//
+// WK 1, 2: the Wilson kernel's force.  Its extra terms (derivs_module.F90:
+// 41-97, 198-410) are the same bilinear form between slices of R and of X2,
+// masked to two spins, with the s-couplings' factors; summed over s they are
+// the form of (R + Q R, X2) for iflag 0 (WK 1) and of (R, X2 + Q X2) for
+// iflag 1 (WK 2).  The couplings come by wave shuffles from the loaded
+// lines, so the whole force is this one pass: 15^2 x 21 x 20 takes 11 us
+// (the s-sum without them 9.6) against 155 with a second kernel that walked
+// the 2 Ls slice pairs of each link one after another.
+template <int WK>
 __global__ __launch_bounds__(BLK, 3) void k_derivs_seg(const Dims d, const double2 *__restrict__ R,
                                                     const double2 *__restrict__ X2, float tzi,
                                                     int iflag, unsigned wseg, unsigned tchunk,
-                                                    double *ds) {
+                                                    double *ds, const WallCoef wall) {
   const unsigned lx = d.lx, ly = d.ly, lt = d.lt, ls = d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   const unsigned nl = BLK / wseg;           // lines per block
@@ -185,23 +384,38 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg(const Dims d, const doubl
   }
   const unsigned xf = (x + 1 == lx) ? 0 : x + 1, yf = (y + 1 == ly) ? 0 : y + 1;
   const unsigned j = s + ls * col, jx = s + ls * (xf + lx * y), jy = s + ls * (x + lx * yf);
+  const unsigned lane0 = (threadIdx.x & 63) - s;
   cx<double> R0[4], X0[4];
   if (valid) {
     ld_spinor(R, v5, j + v3 * t0, R0);
     ld_spinor(X2, v5, j + v3 * t0, X0);
   }
+  if constexpr (WK == 1) add_couplings(R0, s, ls, lane0, wall);
+  if constexpr (WK == 2) add_couplings(X0, s, ls, lane0, wall);
   for (unsigned t = t0; t < t1; t++) {
     double v[3] = {0.0, 0.0, 0.0};
+    cx<double> Rx[4], Xx[4], Ry[4], Xy[4], Rt[4], Xt[4];
     if (valid) {
       // all six neighbour spinors of the step in flight together
       const unsigned tf = (t + 1 == lt) ? 0 : t + 1;
-      cx<double> Rx[4], Xx[4], Ry[4], Xy[4], Rt[4], Xt[4];
       ld_spinor(R, v5, jx + v3 * t, Rx);
       ld_spinor(X2, v5, jx + v3 * t, Xx);
       ld_spinor(R, v5, jy + v3 * t, Ry);
       ld_spinor(X2, v5, jy + v3 * t, Xy);
       ld_spinor(R, v5, j + v3 * tf, Rt);
       ld_spinor(X2, v5, j + v3 * tf, Xt);
+    }
+    if constexpr (WK == 1) {
+      add_couplings(Rx, s, ls, lane0, wall);
+      add_couplings(Ry, s, ls, lane0, wall);
+      add_couplings(Rt, s, ls, lane0, wall);
+    }
+    if constexpr (WK == 2) {
+      add_couplings(Xx, s, ls, lane0, wall);
+      add_couplings(Xy, s, ls, lane0, wall);
+      add_couplings(Xt, s, ls, lane0, wall);
+    }
+    if (valid) {
       v[0] = derivs_term<0>(R0, X0, Rx, Xx, w1, w2);
       v[1] = derivs_term<1>(R0, X0, Ry, Xy, w1, w2);
       v[2] = derivs_term<2>(R0, X0, Rt, Xt, w1, w2);
@@ -405,9 +619,10 @@ __global__ __launch_bounds__(BLK) void k_derivs(const Dims d, const double2 *__r
   ds[i] += acc;
 }
 
-// Wilson-kernel extra force terms (derivs_module.F90:41-97, 198-410): the
-// s-couplings of the Wilson-kernel operator, each a derivSlice() between a
-// slice of R and a slice of X2 with spin masks and a complex multiplier.
+// Wilson-kernel extra force terms (derivs_module.F90:41-97, 198-410) where an
+// s-line does not fit one wave (Ls > 64): the s-couplings of the
+// Wilson-kernel operator, each a derivSlice() between a slice of R and a slice
+// of X2 with spin masks and a complex multiplier.
 struct SlicePair {
   int sl, sr;       // 0-based s of the R slice and the X2 slice
   int l0, l1;       // R spins kept [l0, l1)
@@ -459,19 +674,28 @@ __global__ __launch_bounds__(BLK) void k_derivs_wilson_extra(const Dims d, const
 
 }  // namespace
 
+static int launch_derivs_wk(const Dims &d, const double2 *R, const double2 *X2, double anum,
+                            int iflag, int wk, const WallCoef &wall, double *dsdpi, hipStream_t s);
+
 int launch_derivs_wilson(const Dims &d, const double2 *R, const double2 *X2, double anum,
                          int iflag, float am, int imass, double *dsdpi, void *pair_buf,
                          hipStream_t s) {
   THR_CHECK(imass == 1 || imass == 3, THR_ERR_ARG, "Wilson kernel supports imass 1 and 3");
-  int rc = launch_derivs(d, R, X2, anum, iflag, dsdpi, s);
-  if (rc) return rc;
   const int L = d.ls;
-  std::vector<SlicePair> pr;
   const double m = (double)am;
   // derivsWilsonMass (derivs_module.F90:198-249): cmplx(-am,0) | cmplx(0,-am), then
   // cmplx(-am,0) | cmplx(0,am)
   const double c1r = imass == 1 ? -m : 0.0, c1i = imass == 1 ? 0.0 : -m;
   const double c2r = imass == 1 ? -m : 0.0, c2i = imass == 1 ? 0.0 : m;
+  if (L <= 64) {
+    // an s-line fits one wave: the extra terms join the s-sum.  On R (iflag 0)
+    // the walls' factors are conj(c2), conj(c1), which are c1, c2
+    const WallCoef w{c1r, c1i, c2r, c2i};
+    return launch_derivs_wk(d, R, X2, anum, iflag, iflag == 0 ? 1 : iflag == 1 ? 2 : 0, w, dsdpi, s);
+  }
+  int rc = launch_derivs(d, R, X2, anum, iflag, dsdpi, s);
+  if (rc) return rc;
+  std::vector<SlicePair> pr;
   if (iflag == 1) {
     pr.push_back({0, L - 1, 0, 4, 0, 2, c1r, c1i});   // DP: L all, R spins 1:2
     pr.push_back({L - 1, 0, 0, 4, 2, 4, c2r, c2i});   // DM: L all, R spins 3:4
@@ -501,10 +725,63 @@ int launch_derivs_wilson(const Dims &d, const double2 *R, const double2 *X2, dou
   return THR_OK;
 }
 
+long wilson_blocks(const Dims &d) {
+  if (d.ls > 64) return (d.v5() + BLK - 1) / BLK;
+  const long nl = BLK / segment(d.ls);
+  return ((long)d.lx * d.ly + nl - 1) / nl * d.lt;
+}
+
+int launch_wilson_epi(DslashLaunch L, hipStream_t s) {
+  THR_CHECK(L.imass == 1 || L.imass == 3, THR_ERR_ARG, "Wilson kernel supports imass 1 and 3");
+  THR_CHECK(L.d.ls <= 64, THR_ERR_ARG, "fused Wilson kernel: Ls above 64");
+  THR_CHECK(4 * L.d.v5() * (long)sizeof(double2) < (1L << 32), THR_ERR_SIZE,
+            "spinor too large for the Wilson kernel");
+  const double m = (double)L.am[0];
+  // -am | -i am at s = 1 (dirac.F90:274-278, 602-606), -am | +i am at s = Ls
+  // (287-291, 615-619)
+  const WallCoef w = L.imass == 1 ? WallCoef{-m, 0.0, -m, 0.0} : WallCoef{0.0, -m, 0.0, m};
+  const dim3 grid((unsigned)wilson_blocks(L.d), (unsigned)L.nrhs);
+  const unsigned seg = segment(L.d.ls);
+#define THR_GO(D, M) hipLaunchKernelGGL((k_wilson<D, M>), grid, dim3(BLK), 0, s, L, seg, w)
+#define THR_DAG(M)         \
+  do {                     \
+    if (L.dagger)          \
+      THR_GO(true, M);     \
+    else                   \
+      THR_GO(false, M);    \
+  } while (0)
+  switch (L.mode) {
+    case EPI_STORE: THR_DAG(EPI_STORE); break;
+    case EPI_NORM: THR_DAG(EPI_NORM); break;
+    case EPI_DOTW: THR_DAG(EPI_DOTW); break;
+    case EPI_HREC: THR_DAG(EPI_HREC); break;
+    default: THR_DAG(EPI_CG); break;
+  }
+#undef THR_DAG
+#undef THR_GO
+  THR_HIP(hipGetLastError());
+  return THR_OK;
+}
+
 int launch_dslash_wilson(const Dims &d, int nrhs, int dagger, int imass, float am, float am3,
                          const double2 *in, double2 *out, const double2 *links, double2 *tmp,
                          hipStream_t s) {
   THR_CHECK(imass == 1 || imass == 3, THR_ERR_ARG, "Wilson kernel supports imass 1 and 3");
+  if (d.ls <= 64) {
+    DslashLaunch F{};
+    F.d = d;
+    F.nrhs = nrhs;
+    F.dagger = dagger;
+    F.imass = imass;
+    F.am3 = am3;
+    F.am[0] = am;
+    F.in = in;
+    F.out = out;
+    F.links = links;
+    F.mode = EPI_STORE;
+    return launch_wilson_epi(F, s);
+  }
+  THR_CHECK(tmp, THR_ERR_ARG, "Wilson kernel: scratch spinor required");
   const long n = d.v5() * nrhs;
   const unsigned nb = (unsigned)((n + BLK - 1) / BLK);
   DslashLaunch L{};
@@ -567,8 +844,7 @@ int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs_host,
   const long n = 3 * d.v4();
   THR_HIP(hipMemcpyAsync(pairs_dev, pairs_host, sizeof(DerivPair) * npair, hipMemcpyHostToDevice,
                          s));
-  unsigned w = 1;
-  while (w < (unsigned)d.ls) w <<= 1;
+  const unsigned w = segment(d.ls);
   const unsigned nl = BLK / w;
   const unsigned v2 = (unsigned)(d.lx * d.ly);
   const unsigned nb = ((v2 + nl - 1) / nl) * (unsigned)d.lt;
@@ -588,6 +864,13 @@ int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs_host,
 
 int launch_derivs(const Dims &d, const double2 *R, const double2 *X2, double anum, int iflag,
                   double *dsdpi, hipStream_t s) {
+  return launch_derivs_wk(d, R, X2, anum, iflag, 0, WallCoef{}, dsdpi, s);
+}
+
+// wk: the Wilson kernel's couplings on R (1) or X2 (2), Ls <= 64 only
+static int launch_derivs_wk(const Dims &d, const double2 *R, const double2 *X2, double anum,
+                            int iflag, int wk, const WallCoef &wall, double *dsdpi,
+                            hipStream_t s) {
   const float tzi = 2.0f * (float)anum;  // real :: tzi_real = 2*real(anum)
   THR_CHECK(d.v5() * 4 < (1L << 31), THR_ERR_SIZE, "derivs: 4*V5 must be below 2^31");
   // one t step per thread: marching longer t-chunks reuses the t neighbour
@@ -608,12 +891,18 @@ int launch_derivs(const Dims &d, const double2 *R, const double2 *X2, double anu
   const unsigned nchunk = (d.lt + tchunk - 1) / tchunk;
   const unsigned v2 = (unsigned)d.lx * d.ly;
   if (d.ls <= 64) {
-    unsigned w = 1;
-    while (w < (unsigned)d.ls) w <<= 1;
+    const unsigned w = segment(d.ls);
     const unsigned nl = BLK / w;
     const unsigned nb = ((v2 + nl - 1) / nl) * nchunk;
-    hipLaunchKernelGGL(k_derivs_seg, dim3(nb), dim3(BLK), pad, s, d, R, X2, tzi, iflag, w, tchunk,
-                       dsdpi);
+#define THR_SEG(K) \
+  hipLaunchKernelGGL(K, dim3(nb), dim3(BLK), pad, s, d, R, X2, tzi, iflag, w, tchunk, dsdpi, wall)
+    if (wk == 1)
+      THR_SEG(k_derivs_seg<1>);
+    else if (wk == 2)
+      THR_SEG(k_derivs_seg<2>);
+    else
+      THR_SEG(k_derivs_seg<0>);
+#undef THR_SEG
     THR_HIP(hipGetLastError());
     return THR_OK;
   }
