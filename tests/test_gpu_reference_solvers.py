@@ -127,3 +127,47 @@ def test_congrad_wilson_lines(G, dims):
     o = O.congrad(phi, xo, u, dims, res=1e-2, am=0.2, imass=3, kernel="wilson")
     assert g == o
     assert rel(O.interior(xg), O.interior(xo)) <= 1e-11
+
+
+# one site per thread (the default of small launches): lines of every
+# remainder, blocks that end inside a slab, lattices the XCD boxes do and do
+# not divide
+@pytest.mark.parametrize("dims", [(1, 1, 1, 1), (3, 5, 2, 1), (2, 2, 2, 2), (5, 3, 7, 12), (4, 4, 4, 48),
+                                  (8, 8, 8, 8), (3, 5, 4, 70), (4, 2, 8, 64)])
+@pytest.mark.parametrize("imass", [1, 3, 5])
+def test_dslash_one_site_per_thread(G, imass, dims):
+    """FP64 to the Dslash tolerance 1e-13; FP32 and FP16 fields against the
+    FP64 result to 2e-6 and 4e-3 (one rounding per stored number, as
+    test_device_precisions), two right-hand sides of different mass."""
+    from hiprt import DeviceArray
+    rng, u = smooth(dims, 38)
+    v5 = int(np.prod(dims))
+    am = np.array([0.05, 0.3], dtype=np.float32)
+    r = [D.rand_spinor(dims, rng) for _ in am]
+    xh = np.stack([D.interior_vec(a) for a in r])  # (2, 4 V5) spin planes
+    lin = u[1:-1, 1:-1, 1:-1, :].reshape(-1, order="F")
+    l64 = DeviceArray.from_host(np.stack([lin.real, lin.imag], axis=-1))
+    l32 = DeviceArray.from_host(np.stack([lin.real, lin.imag], axis=-1).astype(np.float32))
+    ri = np.stack([xh.real, xh.imag], axis=-1)  # (2, 4 V5, 2)
+    sites = ri.reshape(2, 4, v5, 2).transpose(0, 2, 1, 3)
+    scale = np.abs(sites).max(axis=(2, 3)).astype(np.float32)
+    print("case: one site per thread", dims, imass, flush=True)
+    for dagger, of in ((False, O.dslash), (True, O.dslashd)):
+        ref = np.stack([D.interior_vec(of(a, u, dims, float(m), imass)) for a, m in zip(r, am)])
+        out = DeviceArray(ri.shape, np.float64)
+        G.dslash_dev(out, DeviceArray.from_host(ri), l64, dims, am, imass=imass, dagger=dagger,
+                     nrhs=2)
+        got = out.to_host()
+        assert rel(got[..., 0] + 1j * got[..., 1], ref) <= 1e-13
+        refs = np.stack([ref.real, ref.imag], -1).reshape(2, 4, v5, 2).transpose(0, 2, 1, 3)
+        out = DeviceArray(sites.shape, np.float32)
+        G.dslash_dev(out, DeviceArray.from_host(np.ascontiguousarray(sites).astype(np.float32)), l32,
+                     dims, am, imass=imass, dagger=dagger, prec="f32", nrhs=2)
+        assert rel(out.to_host().astype(np.float64), refs) <= 2e-6
+        q = DeviceArray.from_host(np.ascontiguousarray((sites / scale[..., None, None])
+                                                       .astype(np.float16)))
+        out, on = DeviceArray(sites.shape, np.float16), DeviceArray(scale.shape, np.float32)
+        G.dslash_dev(out, q, l32, dims, am, imass=imass, dagger=dagger, prec="f16", nrhs=2,
+                     in_norm=DeviceArray.from_host(scale), out_norm=on)
+        got = out.to_host().astype(np.float64) * on.to_host()[..., None, None]
+        assert rel(got, refs) <= 4e-3

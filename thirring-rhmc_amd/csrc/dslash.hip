@@ -226,6 +226,33 @@ template <int PREC> struct BAcc {
   __device__ inline cx<C> load1(unsigned site, unsigned a) const { return ld(site, a, scale(site)); }
 };
 
+typedef __attribute__((ext_vector_type(2))) unsigned U2v;
+// spins a, a + 1 of a site
+template <int PREC>
+__device__ inline void load_pair(const BAcc<PREC> &in, unsigned site, unsigned a,
+                                  Spin<PREC> out[2]) {
+  if constexpr (PREC == P64) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const double2 v = __builtin_bit_cast(
+          double2, __builtin_amdgcn_raw_buffer_load_b128(in.rs, site * 16u, (a + k) * in.plane, 0));
+      out[k].v = {v.x, v.y};
+    }
+  } else if constexpr (PREC == P32) {
+    const float4 v = __builtin_bit_cast(
+        float4, __builtin_amdgcn_raw_buffer_load_b128(in.rs, site * 32u + a * 8u, 0, 0));
+    out[0].v = {v.x, v.y};
+    out[1].v = {v.z, v.w};
+  } else {
+    const U2v q = __builtin_amdgcn_raw_buffer_load_b64(in.rs, site * 16u + a * 4u, 0, 0);
+    const unsigned e0 = q[0], e1 = q[1];
+    const float sc = __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(in.rn, site * 4u, 0, 0));
+    out[0] = {e0, sc};
+    out[1] = {e1, sc};
+  }
+}
+
 template <int PREC> __device__ inline Site<PREC> load_site(const BAcc<PREC> &in, unsigned site) {
   Site<PREC> S;
   if constexpr (PREC == P16) {  // the site's 4 spins in one 128-bit load
@@ -784,6 +811,224 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
   }
 }
 
+// One site per thread and one t step, for launches too small to hide memory
+// latency by occupancy (DslashConfig::site).  There the time is the chain of
+// dependent waits, so this kernel has one: every load (the site, its 6
+// neighbours, the two half spinors along s, the links, the epilogue's old
+// field, the partial sums of a fused scalar) is issued before the first is
+// waited for.  The neighbours along s wrap around the line, which is where the
+// wall terms read from, so the s hops and the walls need no loads of their own
+// behind branches.
+template <int PREC, bool DAG, int MODE, bool NT>
+__global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, const Tiling TL) {
+  using C = typename Store<PREC>::C;
+  using T = typename Store<PREC>::T;
+  const int rhs = blockIdx.y;
+  const int dn = L.done ? L.done[(long)rhs * L.done_stride] : 0;
+  const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
+  const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
+  constexpr bool SUM = MODE == EPI_CG || MODE == EPI_HREC;
+  // the first 4 * BLK partial sums of the previous pass
+  const bool fsum = SUM && L.fsum;
+  constexpr int NP = 4;
+  double part[NP] = {};
+  // the epilogue's scalars: delta of a fused one, else a (EPI_CG) or b
+  const double *sp = fsum ? L.fdelta : MODE == EPI_CG ? L.a_ptr : L.b_ptr;
+  const double *bp = MODE == EPI_CG && L.b_ptr ? L.b_ptr : sp;
+  double sc = 0.0, sb = 0.0;
+  if constexpr (SUM) {
+    sc = sp[(long)rhs * L.sc_stride];
+    sb = bp[(long)rhs * L.sc_stride];
+  }
+  if constexpr (SUM) {
+    if (fsum) {
+      const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<double *>(L.fsum + (long)rhs * L.fsum_stride), (short)0, L.fsum_n * 8, BUF_DWORD3);
+#pragma unroll
+      for (int k = 0; k < NP; k++)  // out of range: 0
+        part[k] = __builtin_bit_cast(
+            double, __builtin_amdgcn_raw_buffer_load_b64(rp, (threadIdx.x + k * BLK) * 8u, 0, 0));
+    }
+  }
+  unsigned s, x, y, t;
+  bool valid;
+  if (TL.mode == TILE_BOXES) {
+    const unsigned k = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const unsigned rx = k % TL.px, ry = (k / TL.px) % TL.py, rt = k / (TL.px * TL.py);
+    const unsigned chunk = l / TL.nb3, jr = (l - chunk * TL.nb3) * BLK + threadIdx.x;
+    valid = jr < ls * TL.bx * TL.by;
+    const unsigned q = jr / ls;
+    s = jr - q * ls;
+    x = rx * TL.bx + q % TL.bx;
+    y = ry * TL.by + q / TL.bx;
+    t = rt * TL.bt + chunk;
+  } else {
+    unsigned b = blockIdx.x;
+    if (TL.mode == TILE_REMAP) {
+      const unsigned per = gridDim.x >> 3, full = per << 3;
+      if (b < full) b = (b & 7) * per + (b >> 3);
+    }
+    t = b / TL.nb3;
+    const unsigned j = (b - t * TL.nb3) * BLK + threadIdx.x;
+    valid = j < v3;
+    const unsigned xy = j / ls;
+    s = j - xy * ls;
+    y = xy / lx;
+    x = xy - y * lx;
+  }
+  if (!valid) s = x = y = 0;  // loads a site that exists; nothing is stored
+  const unsigned xy = x + lx * y, l4 = v2 * t;
+  const unsigned xf = (x + 1 == lx) ? 0 : x + 1, xb = (x == 0) ? lx - 1 : x - 1;
+  const unsigned yf = (y + 1 == ly) ? 0 : y + 1, yb = (y == 0) ? ly - 1 : y - 1;
+  const unsigned tf = (t + 1 == lt) ? 0 : t + 1, tb = (t == 0) ? lt - 1 : t - 1;
+  const unsigned col = ls * xy + v3 * t, i = s + col;
+  const long roff = (long)rhs * 4 * v5;
+  const BAcc<PREC> in((const T *)L.in + roff, L.in_norm ? L.in_norm + (long)rhs * v5 : nullptr, v5);
+  const BLinks<C> lk(L.links, 3 * v4);
+  constexpr int up0 = DAG ? 0 : 2, dn0 = DAG ? 2 : 0;
+  const Site<PREC> cur = load_site(in, i);
+  const Site<PREC> rxf = load_site(in, s + ls * (xf + lx * y) + v3 * t);
+  const Site<PREC> rxb = load_site(in, s + ls * (xb + lx * y) + v3 * t);
+  const Site<PREC> ryf = load_site(in, s + ls * (x + lx * yf) + v3 * t);
+  const Site<PREC> ryb = load_site(in, s + ls * (x + lx * yb) + v3 * t);
+  const Site<PREC> rtf = load_site(in, s + ls * xy + v3 * tf);
+  const Site<PREC> rtb = load_site(in, s + ls * xy + v3 * tb);
+  Spin<PREC> su[2], sd[2];
+  load_pair(in, s + 1 == ls ? col : i + 1, up0, su);
+  load_pair(in, s == 0 ? col + ls - 1 : i - 1, dn0, sd);
+  const cx<C> uxf = lk(xy + l4), uxb = conj(lk(xb + lx * y + l4));
+  const cx<C> uyf = lk(v4 + xy + l4), uyb = conj(lk(v4 + x + lx * yb + l4));
+  const cx<C> utf = lk(2 * v4 + xy + l4), utb = conj(lk(2 * v4 + xy + v2 * tb));
+  Site<PREC> old{};
+  if constexpr (MODE == EPI_HREC) {
+    const BAcc<PREC> ho((const T *)L.out + roff,
+                        L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
+    old = load_site(ho, i);
+  }
+  if constexpr (MODE == EPI_CG) {
+    const BAcc<PREC> ro((const T *)L.r + roff, L.r_norm ? L.r_norm + (long)rhs * v5 : nullptr, v5);
+    old = load_site(ro, i);
+  }
+  asm volatile("" ::: "memory");  // the loads stay above the branch and the barriers
+  if (dn) return;
+  C ea = C(0), eb = C(0);
+  if constexpr (SUM) {
+    if (fsum) {
+      // the finalize kernels' order of summation (partial_thread, block_sum)
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < NP; k++)
+        if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
+      const double *p = L.fsum + (long)rhs * L.fsum_stride;
+      for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += p[k];
+      __shared__ double s_fs;
+      v = block_sum(v);
+      if (threadIdx.x == 0) {
+        s_fs = v;
+        if (blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
+      }
+      __syncthreads();
+      if constexpr (MODE == EPI_CG) {
+        const double om = -sc / s_fs;  // omega = -delta / alpha
+        sc = -om;
+      } else {
+        sc = s_fs / sc;  // gamma = lambda / delta
+      }
+    }
+    if constexpr (MODE == EPI_CG) {
+      ea = (C)sc;
+      eb = (C)sb;
+    } else {
+      eb = (C)sc;
+    }
+  }
+  const C diag = L.wilson4d ? (C)(3.0f + (-L.am3)) : (C)((3.0f - L.am3) + 1.0f);
+  const int imass = L.wilson4d ? 0 : L.imass;
+  const C m = (C)L.am[rhs];
+  cx<C> o[4];
+  centre(o, diag, cur);
+  hop<0, DAG>(o, uxf, rxf, uxb, rxb);
+  hop<1, DAG>(o, uyf, ryf, uyb, ryb);
+  hop<2, DAG>(o, utf, rtf, utb, rtb);
+  if (!L.wilson4d) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      // s + 1: the hop, or at s = Ls the wall term from s = 1
+      const cx<C> u = spin_value(su[k]), d = spin_value(sd[k]);
+      if (s + 1 < ls)
+        sub_spin(o[up0 + k], su[k]);
+      else if (imass != 5)
+        o[up0 + k] = o[up0 + k] + (imass == 1 ? m * u : m * muli(u));
+      if (s > 0)
+        sub_spin(o[dn0 + k], sd[k]);
+      else if (imass != 5)
+        o[dn0 + k] = o[dn0 + k] + (imass == 1 ? m * d : (-m) * muli(d));
+    }
+    if (imass == 5) {
+      const C sg = DAG ? C(-1) : C(1);
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        if (s + 1 == ls)
+          o[up0 + k] = o[up0 + k] + (sg * m) * muli(spin_value(spin_of(cur, dn0 + k)));
+        if (s == 0)
+          o[dn0 + k] = o[dn0 + k] + (sg * m) * muli(spin_value(spin_of(cur, up0 + k)));
+      }
+    }
+  }
+  // threads past the slab store to the first site past the field, which the
+  // buffer resource drops: a branch around the stores would end in a wait for
+  // every load and store before the sum below
+  const unsigned is = valid ? i : v5;
+  double red = 0.0;
+  if constexpr (MODE == EPI_CG) {
+    cx<C> rv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      rv[k] = spin_value(spin_of(old, k)) - ea * o[k];
+      red += (double)norm2(rv[k]);
+    }
+    T *ro = (T *)(L.r_out ? L.r_out : L.r) + roff;
+    float *rn = L.r_out ? L.r_out_norm : const_cast<float *>(L.r_norm);
+    const BOut<PREC, NT> rout(ro, rn ? rn + (long)rhs * v5 : nullptr, v5);
+    rout.store4(is, rv);
+    if (L.b_ptr && valid) {
+      const Acc<PREC> pp{(const T *)L.p + roff, nullptr, v5}, xx{(const T *)L.x + roff, nullptr, v5};
+      cx<C> pv[4], xv[4];
+      pp.load4(i, pv);
+      xx.load4(i, xv);
+#pragma unroll
+      for (int k = 0; k < 4; k++) xv[k] = xv[k] + eb * pv[k];
+      const Out<PREC> xo{(T *)L.x + roff, nullptr, v5};
+      xo.store4(i, xv);
+    }
+  } else {
+    if constexpr (MODE == EPI_HREC) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) o[k] = o[k] + eb * spin_value(spin_of(old, k));
+    }
+    const BOut<PREC, NT> out((T *)L.out + roff,
+                                L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
+    out.store4(is, o);
+    if constexpr (MODE == EPI_NORM || MODE == EPI_HREC) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) red += (double)norm2(o[k]);
+    } else if constexpr (MODE == EPI_DOTW) {
+      const Acc<PREC> w{(const T *)L.w + roff, nullptr, v5};
+      cx<C> wv[4];
+      w.load4(i, wv);
+#pragma unroll
+      for (int k = 0; k < 4; k++) red += (double)(wv[k].r * o[k].r + wv[k].i * o[k].i);
+    }
+  }
+  if constexpr (MODE != EPI_STORE) {
+    const double tot = block_sum(valid ? red : 0.0);
+    double *P = L.partial + (long)rhs * TL.pstride;
+    if (threadIdx.x == 0) P[blockIdx.x] = tot;
+    if (blockIdx.x == 0)
+      for (unsigned k = gridDim.x + threadIdx.x; k < TL.pstride; k += BLK) P[k] = 0.0;
+  }
+}
+
 }  // namespace
 
 // bound on every Dslash grid: t-chunk 1 with ceil(Lx Ly Ls / BLK) blocks per
@@ -822,7 +1067,8 @@ static bool box_split(const Dims &d, unsigned &px, unsigned &py, unsigned &pt) {
 // XCD boxes, uniform (scalar) links, lane-shift s hops.  The default is fixed (results
 // identical run to run); dslash_autotune times the candidates on scratch
 // fields and pins the fastest for the process.  THR_DSLASH_TCHUNK / _REMAP /
-// _UNIFORM / _LANESHIFT / _BOXES / _LDSX / _NT override the default.
+// _UNIFORM / _LANESHIFT / _BOXES / _LDSX / _LDSY / _NT / _OCC / _SITE override the
+// default.
 // ---------------------------------------------------------------------------
 namespace {
 // shapes are pinned per lattice, precision and batch class (one right-hand
@@ -837,22 +1083,50 @@ struct TuneKey {
 std::mutex g_tune_mu;
 std::map<TuneKey, DslashConfig> g_tuned;
 
-DslashConfig default_config(const Dims &d) {
+// The default shape of a launch, from the times of every shape over 17
+// lattices (8^4 to 32^3 x 64), 1 to 16 right-hand sides and all precisions on
+// fields that rotate beyond the Infinity Cache (us, one right-hand side
+// unless stated):
+//  * Non-temporal output stores: faster everywhere (32^3 x 64 FP64 76 -> 69;
+//    24^3 x 32 FP32 with 16 right-hand sides 118 -> 110).
+//  * One site per thread (k_dslash_site) while a launch has too few waves to
+//    hide latency.  Where the march has scalar links and LDS exchange (Ls =
+//    32, 64) it wins above 2^18 sites in FP64 (16^3 x 64: march 10.7, site
+//    11.0; 16^3 x 32: 8.1 and 7.7) and above 2^19 in FP32 and FP16 (24^3 x 32
+//    FP32: march 11.7, site 9.7; with 8 right-hand sides 60 and 67).  For
+//    other Ls the site kernel wins in FP64 up to 2^20 sites (24^3 x 48: march
+//    30, site 29; 32^3 x 48: 62 and 67) and always in FP32 and FP16 (32^3 x 48:
+//    37 and 34, 33 and 25).
+//  * Marching: one step up to 2^20 sites (24^3 x 32 FP64: t-chunk 1 17.8, 3
+//    18.8); above, Ls = 32 best at 2 on XCD boxes in every precision (within
+//    4% of the best of 45 shapes on 7 batches).  Ls = 64: FP64 8 (batches 4)
+//    on the XCD remap with at most 3 blocks per CU (32^3 x 64: 64.9; without
+//    the cap 70.9), FP32 4 on 4 x 2-line blocks, FP16 2 on the remap.
+DslashConfig default_config(const Dims &d, int prec, int nrhs) {
   DslashConfig c;
-  // t-chunk 8 (the measured best at 32^3 x 64) unless the lattice is too
-  // small for it to give ~512 blocks per right-hand side: a thread's t
-  // steps run one after another, so a small lattice marched in long chunks
-  // is a few blocks waiting on memory latency (8^3 x 8 at chunk 8: 2 blocks)
-  {
-    const long nb3 = ((long)d.lx * d.ly * d.ls + BLK - 1) / BLK;
-    const long chunks = std::max(1L, (512 + nb3 - 1) / nb3);
-    c.tchunk = (int)std::max(1L, std::min<long>(std::min(8, d.lt), d.lt / chunks));
+  const long sites = d.v5() * nrhs;
+  const bool lines = d.ls == 64 || d.ls == 32;  // scalar links, LDS exchange
+  c.nt_stores = 1;
+  c.site = lines ? sites < (prec == P64 ? 1L << 18 : (1L << 19) + 1)
+                 : prec != P64 || sites <= (1L << 20);
+  c.tchunk = sites <= (1L << 20) ? 1 : 2;
+  if (d.ls == 64 && sites > (1L << 20)) {
+    c.box = 0;
+    if (prec == P64) {
+      c.tchunk = nrhs == 1 ? 8 : 4;
+      c.occ_cap = 2;
+    } else if (prec == P32) {
+      c.tchunk = 4;
+      c.lds_y = 1;
+    }
   }
+  c.tchunk = std::min(c.tchunk, d.lt);
   // lane shifts pay when every wave holds whole s-lines; when lines cross
   // waves the edge-lane loads cost as much as they save (measured at Ls = 48)
   c.laneshift = (64 % d.ls) == 0 ? 1 : 0;
-  c.uniform_links = (d.ls == 64 || d.ls == 32) ? 1 : 0;
+  c.uniform_links = lines ? 1 : 0;
   c.lds_x = c.uniform_links;
+  if (const char *e = std::getenv("THR_DSLASH_SITE")) c.site = std::atoi(e) ? 1 : 0;
   if (const char *e = std::getenv("THR_DSLASH_TCHUNK")) c.tchunk = std::max(1, std::atoi(e));
   if (const char *e = std::getenv("THR_DSLASH_REMAP")) c.remap = std::atoi(e) ? 1 : 0;
   if (const char *e = std::getenv("THR_DSLASH_UNIFORM")) c.uniform_links = std::atoi(e) ? 1 : 0;
@@ -873,7 +1147,7 @@ DslashConfig dslash_config(const Dims &d, int prec, int nrhs) {
     auto it = g_tuned.find(TuneKey{d.lx, d.ly, d.lt, d.ls, prec, m});
     if (it != g_tuned.end()) return it->second;
   }
-  return default_config(d);
+  return default_config(d, prec, nrhs);
 }
 
 void dslash_set_config(const Dims &d, int prec, DslashConfig c, int which) {
@@ -889,7 +1163,8 @@ static Tiling make_tiling(const Dims &d, const DslashConfig &c, unsigned *nblock
   TL.pstride = (unsigned)dslash_blocks(d);
   // 4 x 2-line blocks: the Ls = 64 LDS x exchange (scalar links, lane shifts)
   // on a slab or box of whole tiles
-  const bool ylc = c.lds_y && c.lds_x && c.uniform_links && c.laneshift && d.ls == 64;
+  const bool ylc = !c.site && c.lds_y && c.lds_x && c.uniform_links && c.laneshift && d.ls == 64;
+  const int tc = c.site ? 1 : c.tchunk;
   unsigned px = 1, py = 1, pt = 8;
   if (c.box && box_split(d, px, py, pt)) {
     TL.mode = TILE_BOXES;
@@ -898,14 +1173,14 @@ static Tiling make_tiling(const Dims &d, const DslashConfig &c, unsigned *nblock
     TL.bx = d.lx / px;
     TL.by = d.ly / py;
     TL.bt = d.lt / pt;
-    TL.tchunk = (unsigned)std::max(1, std::min<int>(c.tchunk, (int)TL.bt));
+    TL.tchunk = (unsigned)std::max(1, std::min<int>(tc, (int)TL.bt));
     TL.yl = ylc && TL.bx % 4 == 0 && TL.by % 2 == 0;
     TL.ntx = TL.bx / 4;
     TL.nb3 = TL.yl ? TL.ntx * (TL.by / 2) : ((unsigned)d.ls * TL.bx * TL.by + BLK - 1) / BLK;
     *nblocks = 8 * TL.nb3 * ((TL.bt + TL.tchunk - 1) / TL.tchunk);
   } else {
     TL.mode = c.remap ? TILE_REMAP : TILE_LINEAR;
-    TL.tchunk = (unsigned)std::max(1, std::min(c.tchunk, d.lt));
+    TL.tchunk = (unsigned)std::max(1, std::min(tc, d.lt));
     TL.yl = ylc && d.lx % 4 == 0 && d.ly % 2 == 0;
     TL.ntx = d.lx / 4;
     TL.nb3 = TL.yl ? TL.ntx * (d.ly / 2) : ((unsigned)d.lx * d.ly * d.ls + BLK - 1) / BLK;
@@ -991,6 +1266,37 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
   THR_CHECK(!TL.yl || xl, THR_ERR_STATE, "y exchange without the x exchange");
   THR_CHECK(4 * L.d.v5() * Store<P64>::bytes < (1L << 32), THR_ERR_SIZE,
             "spinor too large for 32-bit buffer offsets");
+  if (c.site) {
+#define THR_SITE(P, D, M)                                                            \
+  do {                                                                               \
+    if (nt)                                                                          \
+      hipLaunchKernelGGL((k_dslash_site<P, D, M, true>), grid, block, 0, s, L, TL);  \
+    else                                                                             \
+      hipLaunchKernelGGL((k_dslash_site<P, D, M, false>), grid, block, 0, s, L, TL); \
+  } while (0)
+#define THR_SITE1(P, D)                                      \
+  switch (L.mode) {                                          \
+    case EPI_STORE: THR_SITE(P, D, EPI_STORE); break;        \
+    case EPI_NORM: THR_SITE(P, D, EPI_NORM); break;          \
+    case EPI_DOTW: THR_SITE(P, D, EPI_DOTW); break;          \
+    case EPI_HREC: THR_SITE(P, D, EPI_HREC); break;          \
+    default: THR_SITE(P, D, EPI_CG); break;                  \
+  }
+#define THR_SITE2(P) \
+  if (L.dagger) { THR_SITE1(P, true); } else { THR_SITE1(P, false); }
+    if (L.prec == P64) {
+      THR_SITE2(P64);
+    } else if (L.prec == P32) {
+      THR_SITE2(P32);
+    } else {
+      THR_SITE2(P16);
+    }
+#undef THR_SITE2
+#undef THR_SITE1
+#undef THR_SITE
+    THR_HIP(hipGetLastError());
+    return THR_OK;
+  }
 #define THR_GO(K)                                                                       \
   do {                                                                                  \
     const void *kf = (const void *)(K);                                                 \
@@ -1070,7 +1376,7 @@ int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *be
   std::vector<float *> inn(nbuf, nullptr), outn(nbuf, nullptr);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = THR_OK;
-  DslashConfig pick = default_config(d);
+  DslashConfig pick = default_config(d, prec, nrhs);
   auto cleanup = [&]() {
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
@@ -1167,6 +1473,18 @@ int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *be
       if (!rc) first.push_back({ms, c});
     }
   }
+  // one site per thread, on both tilings (not one of the pinnable flags: a
+  // shape pinned by flags always marches)
+  for (int v = 0; v < 4 && !rc; v++) {
+    DslashConfig c;
+    c.site = 1;
+    c.box = v & 1;
+    c.nt_stores = (v >> 1) & 1;
+    for (int k = 0; k < 2 && !rc; k++) rc = launch(c);  // warm
+    float ms = 0.f;
+    if (!rc) rc = timed(c, 2 * nbuf, &ms);
+    if (!rc) first.push_back({ms, c});
+  }
   // the short first pass ranks the shapes; the best few are timed again in
   // interleaved rounds (clock and neighbour noise then hits them alike)
   if (!rc && !first.empty()) {
@@ -1177,7 +1495,7 @@ int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *be
     // timed in ten interleaved rounds of at least 16 launches each
     std::vector<DslashConfig> fin;
     for (size_t k = 0; k < std::min<size_t>(6, first.size()); k++)
-      for (int cap = 0; cap <= 3; cap++) {
+      for (int cap = 0; cap <= (first[k].c.site ? 0 : 3); cap++) {
         DslashConfig c = first[k].c;
         c.occ_cap = cap;
         fin.push_back(c);

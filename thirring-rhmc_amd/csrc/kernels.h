@@ -60,7 +60,7 @@ struct DslashLaunch {
 
 // launch shape of the Dslash kernel: t-chunk marched by each thread and
 // whether blocks are remapped so each XCD owns a contiguous lattice range
-// (the defaults are the fastest shape measured at 32^3 x 64; options whose
+// (dslash_config gives a launch its defaults by size; options whose
 // preconditions a lattice does not meet fall back by themselves)
 struct DslashConfig {
   int tchunk = 8;
@@ -76,6 +76,7 @@ struct DslashConfig {
   int nt_stores = 0;      // non-temporal output stores
   int occ_cap = 0;        // 0: no cap; k = 1..3: at most k + 1 blocks per CU (k + 1 waves per
                           // SIMD for 4-wave blocks), by padding each block's LDS
+  int site = 0;           // one site per thread, all loads issued at once (small launches)
 };
 
 // block -> lattice mapping of one Dslash launch (see dslash.hip)
