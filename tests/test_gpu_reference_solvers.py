@@ -171,3 +171,22 @@ def test_dslash_one_site_per_thread(G, imass, dims):
                      in_norm=DeviceArray.from_host(scale), out_norm=on)
         got = out.to_host().astype(np.float64) * on.to_host()[..., None, None]
         assert rel(got, refs) <= 4e-3
+
+
+# congrad's batches poll after 4, 12, 28, 60, ... iterations: caps inside a
+# batch, at its end and one past it, with the passes carrying the scalar steps
+# (24: small launch) and as launches of their own (a pinned shape)
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("niterc", [0, 1, 2, 4, 5, 12, 13, 30])
+def test_congrad_batches_at_the_cap(G, niterc, pinned):
+    dims = (4, 4, 6, 24) if not pinned else (4, 6, 4, 24)
+    rng, u = smooth(dims, 39)
+    phi, x0 = D.rand_spinor(dims, rng), D.rand_spinor(dims, rng)
+    if pinned:
+        G.dslash_set_config(dims, "f64", 2, G.SHAPE_XCD_REMAP)
+    xg, xo = x0.copy(order="F"), x0.copy(order="F")
+    print("case: congrad cap", niterc, pinned, flush=True)
+    g = G.congrad(phi, xg, u, dims, res=1e-9, am=0.1, imass=3, niterc=niterc)
+    o = O.congrad(phi, xo, u, dims, res=1e-9, am=0.1, imass=3, niterc=niterc)
+    assert g == o
+    assert rel(O.interior(xg), O.interior(xo)) <= 1e-11

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "dslash_site.h"
+#include "krylov_scalars.h"
 
 namespace thr {
 
@@ -483,7 +484,8 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
   // the previous pass's partial sums of this right-hand side (the finalize
   // kernels' loop and tree, so the value is theirs bit for bit)
   double fs = 0.0;
-  if constexpr (MODE == EPI_CG || MODE == EPI_HREC) {
+  constexpr bool HREC = MODE == EPI_HREC || MODE == EPI_HPREC;
+  if constexpr (MODE == EPI_CG || HREC) {
     if (L.fsum) {
       __shared__ double s_fs;
       // the first BLK threads sum as the finalize kernels do (the other
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
           threadIdx.x < BLK ? partial_thread(L.fsum + (long)rhs * L.fsum_stride, L.fsum_n) : 0.0);
       if (threadIdx.x == 0) {
         s_fs = v;
-        if (blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
+        if (L.frec && blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
       }
       __syncthreads();
       fs = s_fs;
@@ -581,10 +583,10 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
         ea = (C)L.a_ptr[(long)rhs * L.sc_stride];
       }
       if (L.b_ptr) eb = (C)L.b_ptr[(long)rhs * L.sc_stride];
-    } else if constexpr (MODE == EPI_HREC) {
+    } else if constexpr (HREC) {
       if (L.fsum)
         eb = (C)(fs / L.fdelta[(long)rhs * L.sc_stride]);  // gamma = lambda / delta
-      else
+      else if (MODE == EPI_HREC || L.b_ptr)
         eb = (C)L.b_ptr[(long)rhs * L.sc_stride];
     }
 
@@ -772,7 +774,7 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
       } else {
         const BOut<PREC, NT> out((T *)L.out + roff, L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr,
                                  v5);
-        if constexpr (MODE == EPI_HREC) {
+        if constexpr (HREC) {
           // out = M in + b out: this thread reads its own site before writing it
           const C bb = eb;
           Acc<PREC> ho{(const T *)L.out + roff, L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr,
@@ -786,6 +788,17 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
           }
         }
         out.store4(i, o);
+        if constexpr (MODE == EPI_HPREC) {
+          const Acc<PREC> po{(const T *)L.x + roff, nullptr, v5};
+          const Out<PREC> px{(T *)L.x + roff, nullptr, v5};
+          cx<C> pv[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) pv[k] = {C(0), C(0)};
+          if (L.b_ptr) po.load4(i, pv);
+#pragma unroll
+          for (int k = 0; k < 4; k++) pv[k] = spin_value(spin_of(cur, k)) + eb * pv[k];
+          px.store4(i, pv);
+        }
         if constexpr (MODE == EPI_NORM) {
 #pragma unroll
           for (int k = 0; k < 4; k++) red += (double)norm2(o[k]);
@@ -827,7 +840,10 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   const int dn = L.done ? L.done[(long)rhs * L.done_stride] : 0;
   const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
-  constexpr bool SUM = MODE == EPI_CG || MODE == EPI_HREC;
+  constexpr bool HREC = MODE == EPI_HREC || MODE == EPI_HPREC;
+  constexpr bool SUM = MODE == EPI_CG || HREC;
+  // the launch's field blocks; one more carries the scalar step
+  const unsigned nbl = gridDim.x - (SUM && PREC == P64 && L.scal ? 1u : 0u);
   // the first 4 * BLK partial sums of the previous pass
   const bool fsum = SUM && L.fsum;
   constexpr int NP = 4;
@@ -835,10 +851,13 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   // the epilogue's scalars: delta of a fused one, else a (EPI_CG) or b
   const double *sp = fsum ? L.fdelta : MODE == EPI_CG ? L.a_ptr : L.b_ptr;
   const double *bp = MODE == EPI_CG && L.b_ptr ? L.b_ptr : sp;
+  const bool first = MODE == EPI_HPREC && !L.b_ptr;  // b = 0
   double sc = 0.0, sb = 0.0;
   if constexpr (SUM) {
-    sc = sp[(long)rhs * L.sc_stride];
-    sb = bp[(long)rhs * L.sc_stride];
+    if (sp) {
+      sc = sp[(long)rhs * L.sc_stride];
+      sb = bp[(long)rhs * L.sc_stride];
+    }
   }
   if constexpr (SUM) {
     if (fsum) {
@@ -865,7 +884,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   } else {
     unsigned b = blockIdx.x;
     if (TL.mode == TILE_REMAP) {
-      const unsigned per = gridDim.x >> 3, full = per << 3;
+      const unsigned per = nbl >> 3, full = per << 3;
       if (b < full) b = (b & 7) * per + (b >> 3);
     }
     t = b / TL.nb3;
@@ -876,6 +895,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     y = xy / lx;
     x = xy - y * lx;
   }
+  if (t >= lt) t = 0;  // the scalar block: no site of its own
   if (!valid) s = x = y = 0;  // loads a site that exists; nothing is stored
   const unsigned xy = x + lx * y, l4 = v2 * t;
   const unsigned xf = (x + 1 == lx) ? 0 : x + 1, xb = (x == 0) ? lx - 1 : x - 1;
@@ -899,11 +919,15 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   const cx<C> uxf = lk(xy + l4), uxb = conj(lk(xb + lx * y + l4));
   const cx<C> uyf = lk(v4 + xy + l4), uyb = conj(lk(v4 + x + lx * yb + l4));
   const cx<C> utf = lk(2 * v4 + xy + l4), utb = conj(lk(2 * v4 + xy + v2 * tb));
-  Site<PREC> old{};
-  if constexpr (MODE == EPI_HREC) {
+  Site<PREC> old{}, pold{};
+  if constexpr (HREC) {
     const BAcc<PREC> ho((const T *)L.out + roff,
                         L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
     old = load_site(ho, i);
+  }
+  if constexpr (MODE == EPI_HPREC) {
+    const BAcc<PREC> po((const T *)L.x + roff, nullptr, v5);
+    pold = load_site(po, i);
   }
   if constexpr (MODE == EPI_CG) {
     const BAcc<PREC> ro((const T *)L.r + roff, L.r_norm ? L.r_norm + (long)rhs * v5 : nullptr, v5);
@@ -925,9 +949,15 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
       v = block_sum(v);
       if (threadIdx.x == 0) {
         s_fs = v;
-        if (blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
+        if (L.frec && blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
       }
       __syncthreads();
+      if constexpr (PREC == P64) {
+        if (L.scal && blockIdx.x == nbl) {
+          scalar_step(L.scal, L.sst, L.sslot, s_fs);
+          return;
+        }
+      }
       if constexpr (MODE == EPI_CG) {
         const double om = -sc / s_fs;  // omega = -delta / alpha
         sc = -om;
@@ -937,9 +967,9 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     }
     if constexpr (MODE == EPI_CG) {
       ea = (C)sc;
-      eb = (C)sb;
+      eb = fsum ? ea : (C)sb;  // a fused x += b p is the CG's: b = a
     } else {
-      eb = (C)sc;
+      eb = first ? C(0) : (C)sc;
     }
   }
   const C diag = L.wilson4d ? (C)(3.0f + (-L.am3)) : (C)((3.0f - L.am3) + 1.0f);
@@ -1002,14 +1032,24 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
       xo.store4(i, xv);
     }
   } else {
-    if constexpr (MODE == EPI_HREC) {
+    if constexpr (HREC) {
 #pragma unroll
       for (int k = 0; k < 4; k++) o[k] = o[k] + eb * spin_value(spin_of(old, k));
+    }
+    if constexpr (MODE == EPI_HPREC) {
+      cx<C> pv[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const cx<C> in_k = spin_value(spin_of(cur, k));
+        pv[k] = first ? in_k : in_k + eb * spin_value(spin_of(pold, k));
+      }
+      const BOut<PREC, NT> pout((T *)L.x + roff, nullptr, v5);
+      pout.store4(is, pv);
     }
     const BOut<PREC, NT> out((T *)L.out + roff,
                                 L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
     out.store4(is, o);
-    if constexpr (MODE == EPI_NORM || MODE == EPI_HREC) {
+    if constexpr (MODE == EPI_NORM || HREC) {
 #pragma unroll
       for (int k = 0; k < 4; k++) red += (double)norm2(o[k]);
     } else if constexpr (MODE == EPI_DOTW) {
@@ -1025,7 +1065,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     double *P = L.partial + (long)rhs * TL.pstride;
     if (threadIdx.x == 0) P[blockIdx.x] = tot;
     if (blockIdx.x == 0)
-      for (unsigned k = gridDim.x + threadIdx.x; k < TL.pstride; k += BLK) P[k] = 0.0;
+      for (unsigned k = nbl + threadIdx.x; k < TL.pstride; k += BLK) P[k] = 0.0;
   }
 }
 
@@ -1241,11 +1281,15 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
   THR_CHECK(L.prec != P16 || L.mode != EPI_DOTW, THR_ERR_ARG, "fp16 dot epilogue unsupported");
   THR_CHECK(L.mode != EPI_HREC || (L.b_ptr && (L.prec != P16 || L.out_norm)), THR_ERR_ARG,
             "recurrence epilogue needs its scalar (and fp16 scales)");
+  THR_CHECK(L.mode != EPI_HPREC || (L.prec == P64 && !L.dagger && L.x), THR_ERR_ARG,
+            "direction epilogue: FP64, with its vector");
+  THR_CHECK(!L.scal || (c.site && L.prec == P64 && L.nrhs == 1 && L.fsum && L.sst), THR_ERR_ARG,
+            "scalar step on a launch that cannot carry it");
   THR_CHECK(4 * L.d.v5() < (1L << 31), THR_ERR_SIZE, "lattice too large for 32-bit indexing");
   unsigned nblocks = 0;
   const Tiling TL = make_tiling(L.d, c, &nblocks);
   THR_CHECK(nblocks <= TL.pstride, THR_ERR_ARG, "dslash grid exceeds partial stride");
-  dim3 grid(nblocks, (unsigned)L.nrhs);
+  dim3 grid(nblocks + (L.scal ? 1u : 0u), (unsigned)L.nrhs);
   dim3 block(TL.yl ? 2 * BLK : BLK);
   const bool shuf = c.laneshift != 0;
   // a wave is exactly one s-line when Ls = 64, two when Ls = 32, four when
@@ -1280,6 +1324,7 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
     case EPI_NORM: THR_SITE(P, D, EPI_NORM); break;          \
     case EPI_DOTW: THR_SITE(P, D, EPI_DOTW); break;          \
     case EPI_HREC: THR_SITE(P, D, EPI_HREC); break;          \
+    case EPI_HPREC: THR_SITE(P64, false, EPI_HPREC); break;  \
     default: THR_SITE(P, D, EPI_CG); break;                  \
   }
 #define THR_SITE2(P) \
@@ -1334,6 +1379,7 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
     case EPI_NORM: THR_LAUNCH(P, D, S, EPI_NORM); break;   \
     case EPI_DOTW: THR_LAUNCH(P, D, S, EPI_DOTW); break;   \
     case EPI_HREC: THR_LAUNCH(P, D, S, EPI_HREC); break;   \
+    case EPI_HPREC: THR_LAUNCH(P64, false, S, EPI_HPREC); break; \
     default: THR_LAUNCH(P, D, S, EPI_CG); break;           \
   }
 #define THR_LAUNCH2(P, D) \
@@ -1478,6 +1524,7 @@ int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *be
   for (int v = 0; v < 4 && !rc; v++) {
     DslashConfig c;
     c.site = 1;
+    c.tchunk = 1;
     c.box = v & 1;
     c.nt_stores = (v >> 1) & 1;
     for (int k = 0; k < 2 && !rc; k++) rc = launch(c);  // warm

@@ -13,7 +13,12 @@ enum EpiMode {
   EPI_DOTW = 2,      // out = M r ; partial += Re <w, out>
   EPI_CG = 3,        // (CG dagger step) r -= a*out ; x += b*p ; partial += |r|^2 ; out not stored
   EPI_HREC = 4,      // out = M r + b*out (in place) ; partial += |out|^2  (h = M p by recurrence)
+  EPI_HPREC = 5,     // EPI_HREC and x = r + b*x (the direction p itself); b is 0, and the old x
+                     // not used, where b_ptr is null (FP64)
 };
+
+// scalar step carried by a launch (krylov_scalars.h)
+enum ScalKind { SCAL_NONE = 0, SCAL_MS_ALPHA = 1, SCAL_MS_LAMBDA = 2, SCAL_CG_ALPHA = 3, SCAL_CG_BETA = 4 };
 
 struct DslashLaunch {
   Dims d;
@@ -51,7 +56,14 @@ struct DslashLaunch {
   const double *fsum;  // null: read a_ptr / b_ptr
   int fsum_n, fsum_stride;
   const double *fdelta;
-  double *frec;
+  double *frec;        // null: not stored
+  // scalar step run by one more block of the launch on the same sum (the
+  // kernels of dslash_fuses_scalars and the Wilson kernel; one right-hand
+  // side): the state's recurrences need the sum, the field work does not need
+  // them, so they overlap with it instead of being a launch in between
+  int scal;            // ScalKind
+  void *sst;           // its state
+  double *sslot;       // SCAL_MS_LAMBDA, SCAL_CG_BETA: where the new delta / |r|^2 goes
   double *partial;     // [nrhs][nblocks]
   const int *done;     // optional early-exit flag, done[rhs*done_stride] (device)
   int done_stride;
@@ -94,6 +106,8 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s);
 // partial-sum entries per right-hand side written by every Dslash epilogue
 // (the row stride of the partial buffer; entries past a launch's grid are 0)
 long dslash_blocks(const Dims &d);
+// whether a launch with configuration c may carry a scalar step (FP64)
+inline bool dslash_fuses_scalars(const DslashConfig &c) { return c.site != 0; }
 // blocks per right-hand side of a launch with configuration c: the partial
 // entries that launch fills with its sums
 long dslash_grid_blocks(const Dims &d, const DslashConfig &c);

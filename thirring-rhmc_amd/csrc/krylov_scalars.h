@@ -1,0 +1,207 @@
+// Scalar recurrences of the reference-order Krylov solvers, device side.
+//
+// Each step runs in one block of BLK threads on the sum of the operator's
+// partial dot products.  It runs as a kernel of its own (k_scalar and others in
+// solvers.hip) or in an extra block of the operator launch that follows
+// (DslashLaunch::scal), where it overlaps with that launch's field work: every
+// other block derives the one scalar it needs from the same sum.
+#pragma once
+#include "solvers.h"
+
+namespace thr {
+
+// iterations per block of the blocked shift updates (k_ms_flush)
+constexpr int MSR = 32;
+
+// CG state (measure_module.F90:41-120); lam: |r|^2 of the last two iterations
+// by parity, so that a step never writes what its launch's other blocks read
+struct CgState {
+  double alpha, alphan, betacg, lam[2];
+  float resid;
+  int niterc, nx, itercg, stop, iterations;
+};
+
+// multishift state (multishift_module.F90:71-282); dl: delta of the last two
+// iterations by parity
+struct MsState {
+  double delta, alpha, lambda, omega, omega_save, minus_omega, gammag, dl[2];
+  double zeta_i[MAXSHIFT], zeta_ii[MAXSHIFT], zeta_iii[MAXSHIFT], omegas[MAXSHIFT],
+      gammas[MAXSHIFT], corr[MAXSHIFT], aden[MAXSHIFT];
+  int flags[MAXSHIFT], cg_returns[MAXSHIFT];
+  int n, mini, maxi, umin, umax, cg_return, maxcg, stop, done, plain;
+  int nonfinite;  // a dot product came out NaN/Inf: the solve stopped there
+  float res;
+  double resd;  // threshold used by the convergence test
+  // blocked shift updates: the scalars of iteration j of the block for every
+  // shift updated in it, how many iterations of the block updated shift i,
+  // and the block's iterations so far
+  double rec_om[MSR][MAXSHIFT], rec_ga[MSR][MAXSHIFT], rec_ze[MSR][MAXSHIFT];
+  int cnt[MAXSHIFT], jcount;
+  // the block's coefficients for its flush: p_i = ca P_i + sum cb R,
+  // x_i = X_i + cc P_i + sum cd R
+  double ca[MAXSHIFT], cc[MAXSHIFT], cb[MAXSHIFT][MSR], cd[MAXSHIFT][MSR];
+  int fcnt[MAXSHIFT], fact[MAXSHIFT], fjc;
+};
+
+namespace {
+
+// value that thread 0 holds, for every thread of the block
+__device__ inline double block_value(double v) {
+  __shared__ double s;
+  if (threadIdx.x == 0) s = v;
+  __syncthreads();
+  const double r = s;
+  __syncthreads();
+  return r;
+}
+
+// alpha of a CG iteration from |M p|^2
+__device__ inline void cg_alpha_step(CgState *st, double alphad) {
+  if (threadIdx.x == 0) {
+    st->nx += 1;
+    st->itercg += 1;
+    st->alpha = st->alphan / alphad;
+    // a non-finite |M p|^2 (NaN or Inf in the source, the guess or the links)
+    // can never meet the stopping rule: end the solve here instead of at niterc
+    if (!isfinite(alphad) || !isfinite(st->alpha)) {
+      st->stop = 3;
+      st->iterations = st->nx;
+    }
+  }
+}
+
+// beta and the stopping rule from |r|^2; slot: where lam of this iteration goes
+__device__ inline void cg_beta_step(CgState *st, double *slot, double bn) {
+  if (threadIdx.x == 0) {
+    st->betacg = st->nx == 1 ? 0.0 : bn / st->alphan;
+    st->alphan = bn;
+    *slot = bn;
+    if (!isfinite(bn)) {
+      st->stop = 3;
+      st->iterations = st->nx;
+    } else if (bn < (double)st->resid) {
+      st->stop = 1;
+      st->iterations = st->nx;
+    } else if (st->nx >= st->niterc) {
+      // the Fortran loop ends with nx = niterc + 1
+      st->iterations = st->niterc + 1;
+      st->stop = 2;
+    }
+  }
+}
+
+// The shift recurrences take one thread per shift (MAXSHIFT <= 64: all in
+// wave 0); each shift's arithmetic is the serial loop's.  One thread walking
+// 25 shifts took 5.9 (alpha) and 11.7 us (lambda) per launch at 16^3 x 48,
+// most of it the memory latency of one shift after another; so 2.6 and 3.4.
+__device__ inline void ms_alpha_step(MsState *st, double sum) {
+  const double al = block_value(sum), os = st->omega, gg = st->gammag, om = -st->delta / al;
+  const bool ok = isfinite(om);
+  const int i = threadIdx.x;
+  if (ok && i >= st->mini - 1 && i < st->maxi) {
+    const double z1 = st->zeta_i[i], z2 = st->zeta_ii[i];
+    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - st->aden[i] * om));
+    st->zeta_iii[i] = z3;
+    st->omegas[i] = om * z3 / z2;
+  }
+  __syncthreads();  // every thread has read the scalars before thread 0 writes them
+  if (threadIdx.x == 0) {
+    st->cg_return += 1;
+    st->alpha = al;
+    st->omega_save = os;
+    st->omega = om;
+    st->minus_omega = -om;
+    if (!ok) {
+      // nothing downstream of a non-finite omega is meaningful: stop before
+      // any vector of this iteration is updated
+      st->nonfinite = 1;
+      st->stop = 1;
+      st->done = 1;
+    }
+  }
+}
+
+// REC: record the iteration's shift scalars for the block's flush; slot: where
+// the next iteration's delta goes beside the state's
+template <bool REC>
+__device__ inline void ms_lambda_step(MsState *st, double *slot, double sum) {
+  __shared__ int s_nmin, s_nmax;
+  const double lam = block_value(sum);
+  if (!isfinite(lam)) {
+    if (threadIdx.x == 0) {
+      st->nonfinite = 1;
+      st->stop = 1;
+      st->done = 1;
+    }
+    return;
+  }
+  const int i = threadIdx.x, mini = st->mini, maxi = st->maxi, n = st->n, j = st->jcount;
+  const double delta = st->delta, gg = lam / delta, om = st->omega, resd = st->resd;
+  const int cg = st->cg_return, maxcg = st->maxcg;
+  if (i < 64) {  // wave 0: the ballot spans every shift
+    const bool mine = i >= mini - 1 && i < maxi;
+    double z2 = 0.0, z3 = 0.0;
+    bool on = false;
+    if (i < n) {
+      z2 = st->zeta_ii[i];
+      if (mine) {
+        z3 = st->zeta_iii[i];
+        const double omi = st->omegas[i], ga = gg * z3 * omi / (z2 * om);
+        st->gammas[i] = ga;
+        st->cg_returns[i] = cg;
+        if constexpr (REC) {
+          st->rec_om[j][i] = omi;
+          st->rec_ga[j][i] = ga;
+          st->rec_ze[j][i] = z3;
+          st->cnt[i] = j + 1;
+        }
+      }
+      on = st->flags[i] && !(sqrt(delta * z2 * z2) * st->corr[i] < resd);
+      if (!on) st->flags[i] = 0;
+    }
+    const unsigned long long live = __ballot(on);
+    const int nmax = live ? 64 - __clzll(live) : 0, nmin = live ? __ffsll((long long)live) : n + 1;
+    // the window only shrinks, so its shifts have their zeta in registers
+    if (i >= nmin - 1 && i < nmax) {
+      st->zeta_i[i] = z2;
+      st->zeta_ii[i] = z3;
+    }
+    if (i == 0) {
+      s_nmin = nmin;
+      s_nmax = nmax;
+    }
+  }
+  __syncthreads();  // also: every thread has read the scalars
+  if (threadIdx.x == 0) {
+    st->lambda = lam;
+    st->gammag = gg;
+    st->umin = mini;
+    st->umax = maxi;
+    st->mini = s_nmin;
+    st->maxi = s_nmax;
+    st->delta = lam;
+    if (REC) {
+      *slot = lam;
+      st->jcount = j + 1;
+    }
+    if (!(s_nmax > s_nmin - 1 && cg < maxcg)) st->stop = 1;
+  }
+}
+
+// the step that DslashLaunch::scal names
+__device__ inline const int *scalar_stop(int kind, const void *st) {
+  return kind <= SCAL_MS_LAMBDA ? &((const MsState *)st)->stop : &((const CgState *)st)->stop;
+}
+__device__ inline void scalar_step(int kind, void *st, double *slot, double sum) {
+  if (kind == SCAL_MS_ALPHA)
+    ms_alpha_step((MsState *)st, sum);
+  else if (kind == SCAL_MS_LAMBDA)
+    ms_lambda_step<true>((MsState *)st, slot, sum);
+  else if (kind == SCAL_CG_ALPHA)
+    cg_alpha_step((CgState *)st, sum);
+  else
+    cg_beta_step((CgState *)st, slot, sum);
+}
+
+}  // namespace
+}  // namespace thr

@@ -86,11 +86,13 @@ int thr_congrad_dev_noalloc(const void *phi, void *x, const void *links64, const
   char *p = (char *)base;
   const size_t spinor = align256(sizeof(double2) * (size_t)d.nspinor());
   CgBuffers B{};
-  B.x1 = (double2 *)p;
+  B.h = (double2 *)p;
   B.r = (double2 *)(p + spinor);
   B.p = (double2 *)(p + 2 * spinor);
   B.state = p + 3 * spinor;
   B.partial = (double *)(p + 3 * spinor + align256(cg_state_bytes()));
+  const size_t sums = align256(sizeof(double) * (size_t)dslash_blocks(d));
+  if (need + sums <= NOALLOC_SCRATCH_BYTES) B.partial2 = (double *)((char *)B.partial + sums);
   OpDesc op{};
   op.d = d;
   op.kernel = 0;

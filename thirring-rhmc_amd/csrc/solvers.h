@@ -51,9 +51,10 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
 // allocated (then only the Shamir kernel is allowed: the Wilson kernel's
 // unfused epilogue needs library scratch).
 struct CgBuffers {
-  double2 *x1, *r, *p;
+  double2 *h, *r, *p;
   void *state;
   double *partial;
+  double *partial2;  // as partial; without it the scalar steps are launches of their own
 };
 size_t cg_state_bytes();
 int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float res, int niterc,

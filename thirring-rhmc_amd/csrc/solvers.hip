@@ -17,6 +17,7 @@
 #include <mutex>
 #include <vector>
 
+#include "krylov_scalars.h"
 #include "solvers.h"
 
 namespace thr {
@@ -220,10 +221,13 @@ __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o
       } else if (mode == EPI_DOTW) {
         const cx<double> wv = ldc(w, e);
         red += wv.r * ov.r + wv.i * ov.i;
-      } else if (mode == EPI_HREC) {
-        const cx<double> hv = ov + (*b) * ldc(x, e);
-        st(x, e, hv);
+      } else if (mode == EPI_HREC || mode == EPI_HPREC) {
+        // r: h, in place; EPI_HPREC also x = p + b x (p the operator's input)
+        const double bv = b ? *b : 0.0;
+        const cx<double> hv = ov + bv * ldc(r, e);
+        st(ro, e, hv);
         red += norm2(hv);
+        if (mode == EPI_HPREC) st(x, e, b ? ldc(p, e) + bv * ldc(x, e) : ldc(p, e));
       } else if (mode == EPI_CG) {
         const cx<double> rv = ldc(r, e) - (*a) * ov;
         st(ro, e, rv);
@@ -236,115 +240,33 @@ __global__ __launch_bounds__(BLK) void k_epi(long v5, int mode, const double2 *o
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// ---------------------------------------------------------------------------
-// CG state (measure_module.F90:41-120)
-// ---------------------------------------------------------------------------
-struct CgState {
-  double alpha, alpha_x, alphan, betacgd, betacgn, betacg;
-  float resid;
-  int niterc, nx, itercg, stop, iterations;
-};
-
+// the scalar steps as kernels of their own (one block), where no operator
+// launch carries them (DslashLaunch::scal)
 __global__ void k_cg_init(CgState *st, float resid, int niterc) {
   st->alpha = 1.0;
-  st->alpha_x = 0.0;
   st->alphan = 0.0;
-  st->betacgd = 1.0;
-  st->betacgn = 0.0;
   st->betacg = 0.0;
+  st->lam[0] = st->lam[1] = 1.0;
   st->resid = resid;
   st->niterc = niterc;
-  st->nx = 0;
-  st->itercg = 0;
+  // iteration 1 (r = phi - M^+M x, no scalar of its own) always runs
+  st->nx = niterc < 1 ? 0 : 1;
+  st->itercg = st->nx;
   st->stop = niterc < 1 ? 1 : 0;
   st->iterations = niterc < 1 ? 1 : 0;
 }
 
-__global__ __launch_bounds__(BLK) void k_cg_alpha(CgState *st, const double *partial, int nb) {
-  if (st->stop) return;
-  const double alphad = fin_sum(partial, nb);
-  if (threadIdx.x == 0) {
-    st->nx += 1;
-    st->itercg += 1;
-    if (st->nx != 1) {
-      st->alpha = st->alphan / alphad;
-      st->alpha_x = st->alpha;
-    } else {
-      st->alpha_x = 0.0;
-    }
-    // a non-finite |M p|^2 (NaN or Inf in the source, the guess or the links)
-    // can never meet the stopping rule: end the solve here instead of at niterc
-    if (!isfinite(alphad) || !isfinite(st->alpha)) {
-      st->stop = 3;
-      st->iterations = st->nx;
-    }
-  }
+__global__ __launch_bounds__(BLK) void k_scalar(int kind, void *st, double *slot,
+                                                const double *partial, int nb) {
+  if (*scalar_stop(kind, st)) return;
+  scalar_step(kind, st, slot, partial_sum(partial, nb));
 }
-
-__global__ __launch_bounds__(BLK) void k_cg_beta(CgState *st, const double *partial, int nb) {
-  if (st->stop) return;
-  const double bn = fin_sum(partial, nb);
-  if (threadIdx.x == 0) {
-    st->betacgn = bn;
-    st->betacg = bn / st->betacgd;
-    st->betacgd = bn;
-    st->alphan = bn;
-    if (st->nx == 1) st->betacg = 0.0;
-    if (!isfinite(bn)) {
-      st->stop = 3;
-      st->iterations = st->nx;
-    } else if (bn < (double)st->resid) {
-      st->stop = 1;
-      st->iterations = st->nx;
-    } else if (st->nx >= st->niterc) {
-      // p = r + beta p still runs; the Fortran loop then ends with nx = niterc + 1
-      st->iterations = st->niterc + 1;
-      st->stop = 2;
-    }
-  }
-}
-
-// the p update of the final capped iteration must still run: stop == 2 lets
-// it (stop 1: converged, 3: non-finite scalars)
-__global__ __launch_bounds__(BLK) void k_cg_p(long n, const double2 *r, double2 *p,
-                                              const CgState *S) {
-  if (S->stop == 1 || S->stop == 3) return;
-  const long i = (long)blockIdx.x * BLK + threadIdx.x;
-  if (i >= n) return;
-  st(p, i, ldc(r, i) + S->betacg * ldc(p, i));
-}
-
-// ---------------------------------------------------------------------------
-// multishift state (multishift_module.F90:71-282)
-// ---------------------------------------------------------------------------
-// iterations per block of the blocked shift updates (k_ms_flush)
-constexpr int MSR = 32;
-
-struct MsState {
-  double delta, alpha, lambda, omega, omega_save, gammag;
-  double zeta_i[MAXSHIFT], zeta_ii[MAXSHIFT], zeta_iii[MAXSHIFT], omegas[MAXSHIFT],
-      gammas[MAXSHIFT], corr[MAXSHIFT], aden[MAXSHIFT];
-  int flags[MAXSHIFT], cg_returns[MAXSHIFT];
-  int n, mini, maxi, umin, umax, cg_return, maxcg, stop, done, plain;
-  int nonfinite;  // a dot product came out NaN/Inf: the solve stopped there
-  float res;
-  double resd;  // threshold used by the convergence test
-  // blocked shift updates: the scalars of iteration j of the block for every
-  // shift updated in it, how many iterations of the block updated shift i,
-  // and the block's iterations so far
-  double rec_om[MSR][MAXSHIFT], rec_ga[MSR][MAXSHIFT], rec_ze[MSR][MAXSHIFT];
-  int cnt[MAXSHIFT], jcount;
-  double minus_omega;
-  // the block's coefficients for its flush: p_i = ca P_i + sum cb R,
-  // x_i = X_i + cc P_i + sum cd R
-  double ca[MAXSHIFT], cc[MAXSHIFT], cb[MAXSHIFT][MSR], cd[MAXSHIFT][MSR];
-  int fcnt[MAXSHIFT], fact[MAXSHIFT], fjc;
-};
 
 __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *partial, int nb) {
   const double d = fin_sum(partial, nb);
   if (threadIdx.x == 0) {
     st->delta = d;
+    st->dl[0] = d;
     st->omega = 1.0;
     st->alpha = 0.0;
     st->gammag = 0.0;
@@ -371,111 +293,17 @@ __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *part
   }
 }
 
-// The shift recurrences take one thread per shift (MAXSHIFT <= 64: all in
-// wave 0); each shift's arithmetic is the serial loop's.  One thread walking
-// 25 shifts took 5.9 (alpha) and 11.7 us (lambda) per launch at 16^3 x 48,
-// most of it the memory latency of one shift after another.
+// the per-iteration updates' scalars: done also ends k_ms_update
 __global__ __launch_bounds__(BLK) void k_ms_alpha(MsState *st, const double *partial, int nb) {
   if (st->stop) {
     if (threadIdx.x == 0) st->done = 1;
     return;
   }
-  __shared__ double s_al;
-  const double sum = fin_sum(partial, nb);
-  if (threadIdx.x == 0) s_al = sum;
-  __syncthreads();
-  const double al = s_al, os = st->omega, gg = st->gammag, om = -st->delta / al;
-  const bool ok = isfinite(om);
-  const int i = threadIdx.x;
-  if (ok && i >= st->mini - 1 && i < st->maxi) {
-    const double z1 = st->zeta_i[i], z2 = st->zeta_ii[i];
-    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - st->aden[i] * om));
-    st->zeta_iii[i] = z3;
-    st->omegas[i] = om * z3 / z2;
-  }
-  __syncthreads();  // every thread has read the scalars before thread 0 writes them
-  if (threadIdx.x == 0) {
-    st->cg_return += 1;
-    st->alpha = al;
-    st->omega_save = os;
-    st->omega = om;
-    st->minus_omega = -om;
-    if (!ok) {
-      // nothing downstream of a non-finite omega is meaningful: stop before
-      // any vector of this iteration is updated
-      st->nonfinite = 1;
-      st->stop = 1;
-      st->done = 1;
-    }
-  }
+  ms_alpha_step(st, partial_sum(partial, nb));
 }
-
-// REC: record the iteration's shift scalars for the block's flush
-template <bool REC>
 __global__ __launch_bounds__(BLK) void k_ms_lambda(MsState *st, const double *partial, int nb) {
   if (st->stop) return;
-  __shared__ double s_lam;
-  __shared__ int s_nmin, s_nmax;
-  const double sum = fin_sum(partial, nb);
-  if (threadIdx.x == 0) s_lam = sum;
-  __syncthreads();
-  const double lam = s_lam;
-  if (!isfinite(lam)) {
-    if (threadIdx.x == 0) {
-      st->nonfinite = 1;
-      st->stop = 1;
-      st->done = 1;
-    }
-    return;
-  }
-  const int i = threadIdx.x, mini = st->mini, maxi = st->maxi, n = st->n, j = st->jcount;
-  const double delta = st->delta, gg = lam / delta, om = st->omega, resd = st->resd;
-  const int cg = st->cg_return, maxcg = st->maxcg;
-  if (i < 64) {  // wave 0: the ballot spans every shift
-    const bool mine = i >= mini - 1 && i < maxi;
-    double z2 = 0.0, z3 = 0.0;
-    bool on = false;
-    if (i < n) {
-      z2 = st->zeta_ii[i];
-      if (mine) {
-        z3 = st->zeta_iii[i];
-        const double omi = st->omegas[i], ga = gg * z3 * omi / (z2 * om);
-        st->gammas[i] = ga;
-        st->cg_returns[i] = cg;
-        if constexpr (REC) {
-          st->rec_om[j][i] = omi;
-          st->rec_ga[j][i] = ga;
-          st->rec_ze[j][i] = z3;
-          st->cnt[i] = j + 1;
-        }
-      }
-      on = st->flags[i] && !(sqrt(delta * z2 * z2) * st->corr[i] < resd);
-      if (!on) st->flags[i] = 0;
-    }
-    const unsigned long long live = __ballot(on);
-    const int nmax = live ? 64 - __clzll(live) : 0, nmin = live ? __ffsll((long long)live) : n + 1;
-    // the window only shrinks, so its shifts have their zeta in registers
-    if (i >= nmin - 1 && i < nmax) {
-      st->zeta_i[i] = z2;
-      st->zeta_ii[i] = z3;
-    }
-    if (i == 0) {
-      s_nmin = nmin;
-      s_nmax = nmax;
-    }
-  }
-  __syncthreads();  // also: every thread has read the scalars
-  if (threadIdx.x == 0) {
-    st->lambda = lam;
-    st->gammag = gg;
-    st->umin = mini;
-    st->umax = maxi;
-    st->mini = s_nmin;
-    st->maxi = s_nmax;
-    st->delta = lam;
-    if (REC) st->jcount = j + 1;
-    if (!(s_nmax > s_nmin - 1 && cg < maxcg)) st->stop = 1;
-  }
+  ms_lambda_step<false>(st, nullptr, partial_sum(partial, nb));
 }
 
 // The block's coefficients from its recorded scalars, one thread per shift.
@@ -484,7 +312,12 @@ __global__ __launch_bounds__(BLK) void k_ms_lambda(MsState *st, const double *pa
 // the product of the later g, and in x it is -z_j G_j with
 // G_{j-1} = o_j + g_j G_j.  O(c) per shift and block, instead of updating c
 // coefficients in every iteration.
-__global__ __launch_bounds__(64) void k_ms_coef(MsState *st) {
+// The block's last lambda (its iteration's partial sums) is taken here too.
+__global__ __launch_bounds__(BLK) void k_ms_coef(MsState *st, const double *partial, int nb) {
+  if (!st->stop) {  // uniform: nothing writes it before every thread has read it
+    ms_lambda_step<true>(st, st->dl, partial_sum(partial, nb));
+    __syncthreads();
+  }
   const int i = threadIdx.x, n = st->n;
   if (i < n) {
     const int c = st->cnt[i];
@@ -684,7 +517,8 @@ static int apply_op_epi(const OpDesc &op, DslashLaunch L, const DslashConfig &cf
   if (op.kernel == 1 && op.d.ls <= 64) return launch_wilson_epi(L, s);
   if (op.kernel == 1) {
     // the operator's passes are not gated by the stop flag, the epilogue is
-    const bool direct = L.out && L.mode != EPI_HREC;  // HREC reads the old out
+    const bool hrec = L.mode == EPI_HREC || L.mode == EPI_HPREC;  // these read the old out
+    const bool direct = L.out && !hrec;
     double2 *o = direct ? (double2 *)L.out : (double2 *)workspace(2, sizeof(double2) * op.d.nspinor());
     double2 *tmp = (double2 *)workspace(1, sizeof(double2) * op.d.nspinor());
     THR_CHECK(o && tmp, THR_ERR_HIP, "workspace allocation failed");
@@ -692,15 +526,19 @@ static int apply_op_epi(const OpDesc &op, DslashLaunch L, const DslashConfig &cf
                                 op.u64, tmp, s));
     if (L.mode != EPI_STORE) {
       hipLaunchKernelGGL(k_epi, dim3(nblk(op.d.v5())), dim3(BLK), 0, s, op.d.v5(), L.mode, o,
-                         (const double2 *)L.w, (const double2 *)L.r,
-                         (double2 *)(L.r_out ? L.r_out : L.r),
-                         (double2 *)(L.mode == EPI_HREC ? L.out : L.x), (const double2 *)L.p,
-                         L.a_ptr, L.b_ptr, L.done, L.partial);
+                         (const double2 *)L.w, (const double2 *)(hrec ? L.out : L.r),
+                         (double2 *)(hrec ? L.out : L.r_out ? L.r_out : L.r), (double2 *)L.x,
+                         (const double2 *)(hrec ? L.in : L.p), L.a_ptr, L.b_ptr, L.done, L.partial);
       THR_HIP(hipGetLastError());
     }
     return THR_OK;
   }
   return launch_dslash_cfg(L, cfg, s);
+}
+
+// whether the operator's launches may carry the solver's scalar steps
+static bool op_fuses_scalars(const OpDesc &op, const DslashConfig &cfg) {
+  return op.kernel == 1 ? op.d.ls <= 64 : dslash_fuses_scalars(cfg);
 }
 
 // the partial sums that an operator's epilogue writes, all of them
@@ -709,19 +547,20 @@ static int op_partials(const OpDesc &op, const DslashConfig &cfg) {
 }
 
 // poll a device int every `batch` iterations; batches grow to bound host syncs.
-// host_flag: where the flag is read back (NULL: a pinned int allocated here)
+// one_iteration(k, first, last): iteration k (from 1), the first / last of its
+// batch.  host_flag: where the flag is read back (NULL: the context's pinned int)
 template <typename F>
 static int run_batched(F &&one_iteration, const int *dev_flag, hipStream_t s, long max_iters,
                        int *host_flag = nullptr) {
-  int *h = host_flag;
-  if (!h) THR_HIP(hipHostMalloc((void **)&h, sizeof(int), hipHostMallocDefault));
+  int *h = host_flag ? host_flag : (int *)host_workspace(21, sizeof(int));
+  THR_CHECK(h, THR_ERR_HIP, "host workspace allocation failed");
   *h = 0;
   int batch = 4;
   long done_iters = 0;
   int rc = THR_OK;
   for (;;) {
     for (int k = 0; k < batch; k++) {
-      rc = one_iteration();
+      rc = one_iteration(done_iters + k + 1, k == 0, k + 1 == batch);
       if (rc) break;
     }
     if (rc) break;
@@ -740,7 +579,6 @@ static int run_batched(F &&one_iteration, const int *dev_flag, hipStream_t s, lo
     }
     if (batch < 64) batch *= 2;
   }
-  if (!host_flag) (void)hipHostFree(h);
   return rc;
 }
 
@@ -750,71 +588,103 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
                  int *itercg, int *iterations, hipStream_t s) {
   const Dims &d = op.d;
   const long n = d.nspinor();
+  const int np = (int)std::max(dslash_blocks(d), wilson_blocks(d));
   CgBuffers B{};
-  B.x1 = (double2 *)workspace(10, sizeof(double2) * n);
+  B.h = (double2 *)workspace(10, sizeof(double2) * n);
   B.r = (double2 *)workspace(11, sizeof(double2) * n);
   B.p = (double2 *)workspace(12, sizeof(double2) * n);
   B.state = workspace(13, sizeof(CgState));
-  B.partial = partial_buffer((int)std::max(dslash_blocks(d), wilson_blocks(d)));
-  THR_CHECK(B.x1 && B.r && B.p && B.state && B.partial, THR_ERR_HIP,
-            "workspace allocation failed");
+  B.partial = partial_buffer(2 * np);
+  THR_CHECK(B.h && B.r && B.p && B.state && B.partial, THR_ERR_HIP, "workspace allocation failed");
+  B.partial2 = B.partial + np;
   return cg_reference_bufs(op, phi, x, res, niterc, itercg, iterations, s, B, nullptr);
 }
 
+// The reference's CG with h = M p by recurrence (h_new = M r + beta h; M is
+// linear), so the p update rides on the M pass and an iteration is two
+// operator passes and two scalar steps.  Where the passes may carry the
+// scalar steps (small launches) they do, and those cost no launches; the last
+// step of a batch runs by itself, so the poll sees its verdict.  12^3 x 24: 27
+// us per iteration with five launches, 15 with two.
 int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float res, int niterc,
                       int *itercg, int *iterations, hipStream_t s, const CgBuffers &B,
                       int *host_flag) {
   const Dims &d = op.d;
-  const long n = d.nspinor();
   const DslashConfig cfg = dslash_config(d, P64);
   const int nb = op_partials(op, cfg);
-  double2 *x1 = B.x1, *r = B.r, *p = B.p;
+  double2 *h = B.h, *r = B.r, *p = B.p;
   CgState *st = (CgState *)B.state;
-  double *partial = B.partial;
-  THR_CHECK(x1 && r && p && st && partial, THR_ERR_ARG, "congrad: missing buffers");
+  THR_CHECK(h && r && p && st && B.partial, THR_ERR_ARG, "congrad: missing buffers");
   THR_CHECK(op.kernel == 0 || !host_flag, THR_ERR_ARG,
             "congrad on caller buffers runs the Shamir kernel only");
+  const bool fused = B.partial2 && op_fuses_scalars(op, cfg);
+  double *apart = B.partial, *lpart = fused ? B.partial2 : B.partial;  // |h|^2 and |r|^2 sums
   // resid = 4*ksize*ksize*ksizet*kthird*res*res in default real (measure_module.F90:41)
   const long nsite4 = 4L * d.lx * d.ly * d.lt * d.ls;
   const float resid = ((float)nsite4 * res) * res;
-  THR_HIP(hipMemcpyAsync(p, x, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
-  THR_HIP(hipMemcpyAsync(r, phi, sizeof(double2) * n, hipMemcpyDeviceToDevice, s));
   hipLaunchKernelGGL(k_cg_init, dim3(1), dim3(1), 0, s, st, resid, niterc);
-  const int *stop = &st->stop;
-  auto iter = [&]() -> int {
+  auto scalar = [&](int kind, long k, const double *partial) {
+    hipLaunchKernelGGL(k_scalar, dim3(1), dim3(BLK), 0, s, kind, (void *)st, &st->lam[k & 1], partial,
+                       nb);
+  };
+  // iteration k of the Fortran loop; first, last: of a batch
+  auto iter = [&](long k, bool first, bool last) -> int {
     DslashLaunch a{};
-    a.in = p;
-    a.out = x1;
-    a.mode = EPI_NORM;
-    a.partial = partial;
-    a.done = stop;
+    a.in = k == 1 ? x : r;
+    a.out = h;
+    a.partial = apart;
+    a.done = &st->stop;
+    if (k == 1) {
+      a.mode = EPI_STORE;  // alpha = 1, x stays (measure_module.F90:60-66)
+    } else {
+      a.mode = EPI_HPREC;
+      a.x = p;
+      a.b_ptr = k == 2 ? nullptr : &st->betacg;  // p = r after the first iteration
+      if (fused && !first) {
+        a.fsum = lpart;
+        a.fsum_n = nb;
+        a.fdelta = &st->lam[k & 1];  // |r|^2 of iteration k - 2
+        a.scal = SCAL_CG_BETA;
+        a.sst = st;
+        a.sslot = &st->lam[(k - 1) & 1];
+      }
+    }
     TRY_RC(apply_op_epi(op, a, cfg, s));
-    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     DslashLaunch c{};
     c.dagger = 1;
-    c.in = x1;
+    c.in = h;
     c.mode = EPI_CG;
-    c.r = r;
-    c.x = x;
-    c.p = p;
+    c.r = k == 1 ? const_cast<double2 *>(phi) : r;
+    c.r_out = r;
     c.a_ptr = &st->alpha;
-    c.b_ptr = &st->alpha_x;
-    c.partial = partial;
-    c.done = stop;
+    c.partial = lpart;
+    c.done = &st->stop;
+    if (k > 1) {
+      c.x = x;
+      c.p = p;
+      c.b_ptr = &st->alpha;
+      if (fused) {
+        c.fsum = apart;
+        c.fsum_n = nb;
+        c.fdelta = &st->lam[(k - 1) & 1];
+        c.scal = SCAL_CG_ALPHA;
+        c.sst = st;
+      } else {
+        scalar(SCAL_CG_ALPHA, k, apart);
+      }
+    }
     TRY_RC(apply_op_epi(op, c, cfg, s));
-    hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(BLK), 0, s, st, partial, nb);
-    hipLaunchKernelGGL(k_cg_p, dim3(nblk(n)), dim3(BLK), 0, s, n, r, p, st);
+    if (!fused || last) scalar(SCAL_CG_BETA, k, lpart);
     THR_HIP(hipGetLastError());
     return THR_OK;
   };
-  int rc = run_batched(iter, stop, s, niterc, host_flag);
-  if (rc) return rc;
-  CgState h;
-  THR_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+  TRY_RC(run_batched(iter, &st->stop, s, niterc, host_flag));
+  CgState hs;
+  THR_HIP(hipMemcpyAsync(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
   THR_HIP(hipStreamSynchronize(s));
-  *itercg = h.itercg;
-  if (iterations) *iterations = h.iterations;
-  THR_CHECK(h.stop != 3, THR_ERR_NONFINITE,
+  *itercg = hs.itercg;
+  if (iterations) *iterations = hs.iterations;
+  THR_CHECK(hs.stop != 3, THR_ERR_NONFINITE,
             "congrad: non-finite dot product (NaN or Inf in the source, guess or links)");
   return THR_OK;
 }
@@ -868,13 +738,16 @@ static int ms_result(const MsState *st, int n, int *cg_return, int *cg_returns, 
 // linear), and the M^+ pass updates r in its epilogue, into the next slot of
 // the residual ring.  16^3 x 48, 25 poles: 195 us per iteration with the shift
 // updates in every iteration (four streams per active shift: 120 us), of which
-// this leaves the two operator passes and (MSR + 4 k) / MSR streams.
+// this leaves the two operator passes and (MSR + 4 k) / MSR streams.  On small
+// launches and with the Wilson kernel the passes also carry the scalar steps.
 static int multishift_blocked(const OpDesc &op, int n, const double2 *input, double2 *out,
-                              MsState *st, double2 *h, double2 *ring, double2 *P, double *partial,
-                              int maxcg, const DslashConfig &cfg, hipStream_t s) {
+                              MsState *st, double2 *h, double2 *ring, double2 *P, double *apart,
+                              double *lpart, int maxcg, const DslashConfig &cfg, hipStream_t s) {
   const Dims &d = op.d;
   const long ns = d.nspinor();
   const int nbl = op_partials(op, cfg);
+  // the passes carry the scalar steps: each takes the sum that the other left
+  const bool fused = op_fuses_scalars(op, cfg);
   int *stop = (int *)host_workspace(21, sizeof(int));
   THR_CHECK(stop, THR_ERR_HIP, "host workspace allocation failed");
   for (long t0 = 0;; t0 += MSR) {
@@ -885,10 +758,17 @@ static int multishift_blocked(const OpDesc &op, int n, const double2 *input, dou
       a.out = h;
       a.mode = t == 0 ? EPI_NORM : EPI_HREC;
       a.b_ptr = t == 0 ? nullptr : &st->gammag;
-      a.partial = partial;
+      a.partial = apart;
       a.done = &st->stop;
+      if (fused && t > t0) {
+        a.fsum = lpart;
+        a.fsum_n = nbl;
+        a.fdelta = &st->dl[(t - 1) & 1];
+        a.scal = SCAL_MS_LAMBDA;
+        a.sst = st;
+        a.sslot = &st->dl[t & 1];
+      }
       TRY_RC(apply_op_epi(op, a, cfg, s));
-      hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
       DslashLaunch b{};
       b.dagger = 1;
       b.in = h;
@@ -896,12 +776,24 @@ static int multishift_blocked(const OpDesc &op, int n, const double2 *input, dou
       b.r = const_cast<double2 *>(rin);
       b.r_out = ring + (t % MSR) * ns;
       b.a_ptr = &st->minus_omega;
-      b.partial = partial;
+      b.partial = lpart;
       b.done = &st->stop;
+      if (fused) {
+        b.fsum = apart;
+        b.fsum_n = nbl;
+        b.fdelta = &st->dl[t & 1];
+        b.scal = SCAL_MS_ALPHA;
+        b.sst = st;
+      } else {
+        hipLaunchKernelGGL(k_scalar, dim3(1), dim3(BLK), 0, s, (int)SCAL_MS_ALPHA, (void *)st,
+                           (double *)nullptr, apart, nbl);
+      }
       TRY_RC(apply_op_epi(op, b, cfg, s));
-      hipLaunchKernelGGL(k_ms_lambda<true>, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
+      if (!fused && t + 1 < t0 + MSR)
+        hipLaunchKernelGGL(k_scalar, dim3(1), dim3(BLK), 0, s, (int)SCAL_MS_LAMBDA, (void *)st, st->dl,
+                           lpart, nbl);
     }
-    hipLaunchKernelGGL(k_ms_coef, dim3(1), dim3(64), 0, s, st);
+    hipLaunchKernelGGL(k_ms_coef, dim3(1), dim3(BLK), 0, s, st, lpart, nbl);
     hipLaunchKernelGGL(k_ms_flush, dim3(nblk(ns)), dim3(BLK), 0, s, ns, st, input, ring, out, P,
                        t0 == 0 ? 1 : 0);
     THR_HIP(hipGetLastError());
@@ -921,7 +813,8 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   double2 *h = (double2 *)workspace(21, sizeof(double2) * ns);
   double2 *ps = (double2 *)workspace(24, sizeof(double2) * ns * n);
   MsState *st = (MsState *)workspace(25, sizeof(MsState));
-  double *partial = partial_buffer((int)std::max<long>(nb, wilson_blocks(d)));
+  const int np = (int)std::max<long>(nb, wilson_blocks(d));
+  double *partial = partial_buffer(2 * np);
   THR_CHECK(h && ps && st && partial, THR_ERR_HIP, "workspace allocation failed");
   // Blocked updates keep MSR residuals (16 GiB at most here: 512 MiB fields;
   // 32^3 x 64 takes 4.3); larger fields, and contexts where the ring does not
@@ -939,7 +832,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   hipLaunchKernelGGL(k_ms_init, dim3(1), dim3(BLK), 0, s, st, partial, nb);
   THR_HIP(hipGetLastError());
   if (ring) {
-    TRY_RC(multishift_blocked(op, n, input, out, st, h, ring, ps, partial, maxcg, cfg, s));
+    TRY_RC(multishift_blocked(op, n, input, out, st, h, ring, ps, partial, partial + np, maxcg, cfg, s));
     return ms_result(st, n, cg_return, cg_returns, s);
   }
   double2 *r = (double2 *)workspace(20, sizeof(double2) * ns);
@@ -953,7 +846,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   THR_HIP(hipGetLastError());
   const int *stop = &st->stop;
   const int nbl = op_partials(op, cfg);
-  auto iter = [&]() -> int {
+  auto iter = [&](long, bool, bool) -> int {
     DslashLaunch a{};
     a.in = p;
     a.out = h;
@@ -972,7 +865,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
     hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nbl);
     hipLaunchKernelGGL(k_axpy_norm<P64>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, sv, &st->omega,
                        stop, partial);
-    hipLaunchKernelGGL(k_ms_lambda<false>, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+    hipLaunchKernelGGL(k_ms_lambda, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_ms_update<P64>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, r, p, out, ps, st);
     THR_HIP(hipGetLastError());
     return THR_OK;
@@ -1025,7 +918,7 @@ int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const d
   L.done = stop;
   L.done_stride = 1;
   L.partial = partial;
-  auto iter = [&]() -> int {
+  auto iter = [&](long, bool, bool) -> int {
     DslashLaunch a = L;
     a.dagger = 0;
     a.in = p;
@@ -1044,7 +937,7 @@ int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const d
     hipLaunchKernelGGL(k_ms_alpha, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_axpy_norm<P32>, dim3(nb), dim3(BLK), 0, s, d.v5(), r, sv, &st->omega,
                        stop, partial);
-    hipLaunchKernelGGL(k_ms_lambda<false>, dim3(1), dim3(BLK), 0, s, st, partial, nb);
+    hipLaunchKernelGGL(k_ms_lambda, dim3(1), dim3(BLK), 0, s, st, partial, nb);
     hipLaunchKernelGGL(k_ms_update<P32>, dim3(nblk(ns)), dim3(BLK), 0, s, ns, r, p, xs, ps, st);
     THR_HIP(hipGetLastError());
     return THR_OK;

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "dslash_site.h"
+#include "krylov_scalars.h"
 
 namespace thr {
 
@@ -115,18 +116,37 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
   const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   const unsigned nl = BLK / wseg, nb2 = (v2 + nl - 1) / nl;  // lines per block, blocks per t
+  const unsigned nbl = nb2 * lt;  // field blocks; one more carries the scalar step
   const unsigned t = blockIdx.x / nb2, lb = blockIdx.x - t * nb2;
   const unsigned line = threadIdx.x / wseg, s = threadIdx.x - line * wseg;
   const unsigned col = lb * nl + line;  // 2-D site x + lx y
-  const bool valid = s < ls && col < v2;
+  const bool valid = s < ls && col < v2 && t < lt;
   const unsigned lane0 = (threadIdx.x & 63) - s;
   const long off = (long)rhs * 4 * v5;
+  constexpr bool HREC = MODE == EPI_HREC || MODE == EPI_HPREC;
+  constexpr bool SUM = MODE == EPI_CG || HREC;
+  const bool fsum = SUM && L.fsum;
   const unsigned i = s + ls * col + v3 * t;
-  Site<P64> c{}, f[3]{}, b[3]{}, old{};  // old: the epilogue's h or r
+  Site<P64> c{}, f[3]{}, b[3]{}, old{}, pold{};  // old: the epilogue's h or r
   cx<double> uf[3]{}, ub[3]{};
-  const double ea = MODE == EPI_CG ? L.a_ptr[(long)rhs * L.sc_stride] : 0.0;
-  const double eb = (MODE == EPI_HREC || (MODE == EPI_CG && L.b_ptr))
-                        ? L.b_ptr[(long)rhs * L.sc_stride] : 0.0;
+  // the epilogue's scalars: delta of a fused one, else a (EPI_CG) or b; the
+  // partial sums of a fused one
+  const double *sp = fsum ? L.fdelta : MODE == EPI_CG ? L.a_ptr : L.b_ptr;
+  const double *bp = MODE == EPI_CG && L.b_ptr ? L.b_ptr : sp;
+  const bool first = MODE == EPI_HPREC && !L.b_ptr;  // b = 0
+  constexpr int NP = 4;
+  double part[NP] = {}, sc = 0.0, sb = 0.0;
+  if constexpr (SUM) {
+    if (sp) {
+      sc = sp[(long)rhs * L.sc_stride];
+      sb = bp[(long)rhs * L.sc_stride];
+    }
+    if (fsum) {
+#pragma unroll
+      for (int k = 0; k < NP; k++)
+        part[k] = L.fsum[min((int)threadIdx.x + k * BLK, L.fsum_n - 1)];
+    }
+  }
   if (valid) {
     const double2 *in = (const double2 *)L.in + off, *u = (const double2 *)L.links;
     const unsigned x = col % lx, y = col / lx;
@@ -146,9 +166,27 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
     ub[1] = conj(ldc(u, v4 + x + lx * yb + v2 * t));
     uf[2] = ldc(u, 2 * v4 + col + v2 * t);
     ub[2] = conj(ldc(u, 2 * v4 + col + v2 * tb));
-    if constexpr (MODE == EPI_HREC) ld_spinor((const double2 *)L.out + off, v5, i, old.v);
+    if constexpr (HREC) ld_spinor((const double2 *)L.out + off, v5, i, old.v);
+    if constexpr (MODE == EPI_HPREC) ld_spinor((const double2 *)L.x + off, v5, i, pold.v);
     if constexpr (MODE == EPI_CG) ld_spinor((const double2 *)L.r + off, v5, i, old.v);
   }
+  asm volatile("" ::: "memory");  // the loads stay above the barriers
+  if constexpr (SUM) {
+    if (fsum) {  // the order of partial_sum
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < NP; k++)
+        if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
+      for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += L.fsum[k];
+      v = block_value(block_sum(v));
+      if (blockIdx.x == nbl) {
+        scalar_step(L.scal, L.sst, L.sslot, v);
+        return;
+      }
+      sc = MODE == EPI_CG ? sc / v : v / sc;  // alpha = delta / |h|^2, gamma = lambda / delta
+    }
+  }
+  const double ea = sc, eb = MODE == EPI_CG ? (fsum ? sc : sb) : first ? 0.0 : sc;
   const double diag = (double)(3.0f + (-L.am3));
   cx<double> o[4];
   if constexpr (!DAG) {
@@ -202,9 +240,11 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
           st(xo, e, ldc(xo, e) + eb * ldc((const double2 *)L.p + off, e));
         }
       } else {
-        if constexpr (MODE == EPI_HREC) o[a] = o[a] + eb * old.v[a];
+        if constexpr (HREC) o[a] = o[a] + eb * old.v[a];
         st(out, e, o[a]);
-        if constexpr (MODE == EPI_NORM || MODE == EPI_HREC) red += norm2(o[a]);
+        if constexpr (MODE == EPI_HPREC)
+          st((double2 *)L.x + off, e, first ? c.v[a] : c.v[a] + eb * pold.v[a]);
+        if constexpr (MODE == EPI_NORM || HREC) red += norm2(o[a]);
         if constexpr (MODE == EPI_DOTW) {
           const cx<double> wv = ldc((const double2 *)L.w + off, e);
           red += wv.r * o[a].r + wv.i * o[a].i;
@@ -214,7 +254,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
   }
   if constexpr (MODE != EPI_STORE) {
     const double tot = block_sum(red);
-    if (threadIdx.x == 0) L.partial[(long)rhs * gridDim.x + blockIdx.x] = tot;
+    if (threadIdx.x == 0) L.partial[(long)rhs * nbl + blockIdx.x] = tot;
   }
 }
 
@@ -740,7 +780,10 @@ int launch_wilson_epi(DslashLaunch L, hipStream_t s) {
   // -am | -i am at s = 1 (dirac.F90:274-278, 602-606), -am | +i am at s = Ls
   // (287-291, 615-619)
   const WallCoef w = L.imass == 1 ? WallCoef{-m, 0.0, -m, 0.0} : WallCoef{0.0, -m, 0.0, m};
-  const dim3 grid((unsigned)wilson_blocks(L.d), (unsigned)L.nrhs);
+  THR_CHECK(!L.scal == !L.fsum && (!L.scal || (L.nrhs == 1 && L.sst)), THR_ERR_ARG,
+            "Wilson kernel: a fused sum comes with its scalar step");
+  THR_CHECK(L.mode != EPI_HPREC || (!L.dagger && L.x), THR_ERR_ARG, "direction epilogue: M with its vector");
+  const dim3 grid((unsigned)wilson_blocks(L.d) + (L.scal ? 1u : 0u), (unsigned)L.nrhs);
   const unsigned seg = segment(L.d.ls);
 #define THR_GO(D, M) hipLaunchKernelGGL((k_wilson<D, M>), grid, dim3(BLK), 0, s, L, seg, w)
 #define THR_DAG(M)         \
@@ -755,6 +798,7 @@ int launch_wilson_epi(DslashLaunch L, hipStream_t s) {
     case EPI_NORM: THR_DAG(EPI_NORM); break;
     case EPI_DOTW: THR_DAG(EPI_DOTW); break;
     case EPI_HREC: THR_DAG(EPI_HREC); break;
+    case EPI_HPREC: THR_GO(false, EPI_HPREC); break;
     default: THR_DAG(EPI_CG); break;
   }
 #undef THR_DAG
