@@ -119,20 +119,57 @@ __device__ inline cx<float> ldh(const __half2 *p, long i, float scale) {
 
 constexpr int BLK = 256;  // threads per block for every streaming kernel
 
-// deterministic block reduction over NTH threads: wave shuffles, then a
-// fixed-order LDS sum; the result is valid in thread 0
-template <int NTH>
-__device__ inline double block_sum_n(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// v of another lane of its 16-lane row, by DPP control CTRL
+template <int CTRL> __device__ inline double dpp_value(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// v of lane i plus v of lane i ^ 32 (HALF) or i ^ 16: a row swap of two copies
+// leaves the one in the first and the other in the second
+template <bool HALF> __device__ inline double swap_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)(b & 0xffffffffLL), hi = (unsigned)(b >> 32);
+  const auto l = HALF ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                      : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = HALF ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                      : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  return __longlong_as_double(((long long)h0 << 32) | l0) +
+         __longlong_as_double(((long long)h1 << 32) | l1);
+}
+// sum over the wave, valid in every lane: the butterfly over lanes ^ 32, 16, 8,
+// 4, 2, 1.  Register moves; wave shuffles go through LDS, and six of them one
+// after another cost 0.3 us, as much as the loads of a small Dslash.
+__device__ inline double wave_sum(double v) {
+  v = swap_add<true>(v);
+  v = swap_add<false>(v);
+  v += dpp_value<0x128>(v);  // lane ^ 8: rotation of the row by 8
+  v += dpp_value<0x124>(v);  // by 4: lane ^ 4 or ^ 12, equal by now
+  v += dpp_value<0x4E>(v);   // lane ^ 2
+  v += dpp_value<0xB1>(v);   // lane ^ 1
+  return v;
+}
+
+// deterministic block reduction over NTH threads: wave sums, then a
+// fixed-order LDS sum; the result is valid in every thread.  One barrier; the
+// LDS buffer is TAG's, so sums of different tags may follow each other freely
+// and sums of one tag need a barrier in between (block_sum_n has it).
+template <int NTH, int TAG>
+__device__ inline double block_sum_once(double v) {
   __shared__ double sm[NTH / 64];
+  v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
   __syncthreads();
   double t = 0.0;
-  if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < NTH / 64; k++) t += sm[k];
-  }
+  for (int k = 0; k < NTH / 64; k++) t += sm[k];
+  return t;
+}
+template <int NTH>
+__device__ inline double block_sum_n(double v) {
+  const double t = block_sum_once<NTH, 0>(v);
   __syncthreads();
   return t;
 }
@@ -159,7 +196,7 @@ __device__ inline double partial_thread(const double *p, int n) {
 }
 
 // sum of n per-block partial sums by BLK threads (partial_thread, then
-// block_sum): the result, valid in thread 0, depends only on the values and n
+// block_sum): the result depends only on the values and n
 __device__ inline double partial_sum(const double *p, int n) {
   return block_sum(partial_thread(p, n));
 }

@@ -837,6 +837,11 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   using C = typename Store<PREC>::C;
   using T = typename Store<PREC>::T;
   const int rhs = blockIdx.y;
+  // one batch of argument loads: they lie in seven cache lines, and fetched as
+  // the code comes to need them each line is a wait of its own
+  asm volatile("" ::"s"(L.done), "s"(L.fsum), "s"(L.fdelta), "s"(L.b_ptr), "s"(L.r), "s"(L.in),
+               "s"(L.out), "s"(L.links), "s"(L.partial), "s"(L.d.lx), "s"(L.am3), "s"(TL.nb3),
+               "s"(TL.bt));
   const int dn = L.done ? L.done[(long)rhs * L.done_stride] : 0;
   const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
@@ -929,6 +934,14 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     const BAcc<PREC> po((const T *)L.x + roff, nullptr, v5);
     pold = load_site(po, i);
   }
+  Site<PREC> xold{};
+  const bool xup = MODE == EPI_CG && PREC != P16 && L.b_ptr;
+  if constexpr (MODE == EPI_CG && PREC != P16) {
+    if (xup) {
+      pold = load_site(BAcc<PREC>((const T *)L.p + roff, nullptr, v5), i);
+      xold = load_site(BAcc<PREC>((const T *)L.x + roff, nullptr, v5), i);
+    }
+  }
   if constexpr (MODE == EPI_CG) {
     const BAcc<PREC> ro((const T *)L.r + roff, L.r_norm ? L.r_norm + (long)rhs * v5 : nullptr, v5);
     old = load_site(ro, i);
@@ -945,24 +958,19 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
         if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
       const double *p = L.fsum + (long)rhs * L.fsum_stride;
       for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += p[k];
-      __shared__ double s_fs;
-      v = block_sum(v);
-      if (threadIdx.x == 0) {
-        s_fs = v;
-        if (L.frec && blockIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
-      }
-      __syncthreads();
+      v = block_sum_once<BLK, 1>(v);
+      if (L.frec && blockIdx.x == 0 && threadIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
       if constexpr (PREC == P64) {
         if (L.scal && blockIdx.x == nbl) {
-          scalar_step(L.scal, L.sst, L.sslot, s_fs);
+          scalar_step(L.scal, L.sst, L.sslot, v);
           return;
         }
       }
       if constexpr (MODE == EPI_CG) {
-        const double om = -sc / s_fs;  // omega = -delta / alpha
+        const double om = -sc / v;  // omega = -delta / alpha
         sc = -om;
       } else {
-        sc = s_fs / sc;  // gamma = lambda / delta
+        sc = v / sc;  // gamma = lambda / delta
       }
     }
     if constexpr (MODE == EPI_CG) {
@@ -1021,15 +1029,15 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     float *rn = L.r_out ? L.r_out_norm : const_cast<float *>(L.r_norm);
     const BOut<PREC, NT> rout(ro, rn ? rn + (long)rhs * v5 : nullptr, v5);
     rout.store4(is, rv);
-    if (L.b_ptr && valid) {
-      const Acc<PREC> pp{(const T *)L.p + roff, nullptr, v5}, xx{(const T *)L.x + roff, nullptr, v5};
-      cx<C> pv[4], xv[4];
-      pp.load4(i, pv);
-      xx.load4(i, xv);
+    if constexpr (PREC != P16) {
+      if (xup) {
+        cx<C> xv[4];
 #pragma unroll
-      for (int k = 0; k < 4; k++) xv[k] = xv[k] + eb * pv[k];
-      const Out<PREC> xo{(T *)L.x + roff, nullptr, v5};
-      xo.store4(i, xv);
+        for (int k = 0; k < 4; k++)
+          xv[k] = spin_value(spin_of(xold, k)) + eb * spin_value(spin_of(pold, k));
+        const BOut<PREC, NT> xout((T *)L.x + roff, nullptr, v5);
+        xout.store4(is, xv);
+      }
     }
   } else {
     if constexpr (HREC) {
@@ -1061,7 +1069,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     }
   }
   if constexpr (MODE != EPI_STORE) {
-    const double tot = block_sum(valid ? red : 0.0);
+    const double tot = block_sum_once<BLK, 2>(valid ? red : 0.0);
     double *P = L.partial + (long)rhs * TL.pstride;
     if (threadIdx.x == 0) P[blockIdx.x] = tot;
     if (blockIdx.x == 0)

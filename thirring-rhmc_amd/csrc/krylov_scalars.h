@@ -1,7 +1,7 @@
 // Scalar recurrences of the reference-order Krylov solvers, device side.
 //
-// Each step runs in one block of BLK threads on the sum of the operator's
-// partial dot products.  It runs as a kernel of its own (k_scalar and others in
+// Each step runs in one block of BLK threads on the sum (in every thread) of the
+// operator's partial dot products.  It runs as a kernel of its own (k_scalar and others in
 // solvers.hip) or in an extra block of the operator launch that follows
 // (DslashLaunch::scal), where it overlaps with that launch's field work: every
 // other block derives the one scalar it needs from the same sum.
@@ -45,16 +45,6 @@ struct MsState {
 
 namespace {
 
-// value that thread 0 holds, for every thread of the block
-__device__ inline double block_value(double v) {
-  __shared__ double s;
-  if (threadIdx.x == 0) s = v;
-  __syncthreads();
-  const double r = s;
-  __syncthreads();
-  return r;
-}
-
 // alpha of a CG iteration from |M p|^2
 __device__ inline void cg_alpha_step(CgState *st, double alphad) {
   if (threadIdx.x == 0) {
@@ -94,8 +84,8 @@ __device__ inline void cg_beta_step(CgState *st, double *slot, double bn) {
 // wave 0); each shift's arithmetic is the serial loop's.  One thread walking
 // 25 shifts took 5.9 (alpha) and 11.7 us (lambda) per launch at 16^3 x 48,
 // most of it the memory latency of one shift after another; so 2.6 and 3.4.
-__device__ inline void ms_alpha_step(MsState *st, double sum) {
-  const double al = block_value(sum), os = st->omega, gg = st->gammag, om = -st->delta / al;
+__device__ inline void ms_alpha_step(MsState *st, double al) {
+  const double os = st->omega, gg = st->gammag, om = -st->delta / al;
   const bool ok = isfinite(om);
   const int i = threadIdx.x;
   if (ok && i >= st->mini - 1 && i < st->maxi) {
@@ -124,9 +114,8 @@ __device__ inline void ms_alpha_step(MsState *st, double sum) {
 // REC: record the iteration's shift scalars for the block's flush; slot: where
 // the next iteration's delta goes beside the state's
 template <bool REC>
-__device__ inline void ms_lambda_step(MsState *st, double *slot, double sum) {
+__device__ inline void ms_lambda_step(MsState *st, double *slot, double lam) {
   __shared__ int s_nmin, s_nmax;
-  const double lam = block_value(sum);
   if (!isfinite(lam)) {
     if (threadIdx.x == 0) {
       st->nonfinite = 1;

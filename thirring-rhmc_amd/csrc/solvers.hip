@@ -546,40 +546,23 @@ static int op_partials(const OpDesc &op, const DslashConfig &cfg) {
   return (int)(op.kernel == 1 ? wilson_blocks(op.d) : dslash_grid_blocks(op.d, cfg));
 }
 
-// poll a device int every `batch` iterations; batches grow to bound host syncs.
-// one_iteration(k, first, last): iteration k (from 1), the first / last of its
-// batch.  host_flag: where the flag is read back (NULL: the context's pinned int)
+// poll a device int every `batch` iterations; batches grow to bound host syncs
 template <typename F>
-static int run_batched(F &&one_iteration, const int *dev_flag, hipStream_t s, long max_iters,
-                       int *host_flag = nullptr) {
-  int *h = host_flag ? host_flag : (int *)host_workspace(21, sizeof(int));
+static int run_batched(F &&one_iteration, const int *dev_flag, hipStream_t s, long max_iters) {
+  int *h = (int *)host_workspace(21, sizeof(int));
   THR_CHECK(h, THR_ERR_HIP, "host workspace allocation failed");
   *h = 0;
   int batch = 4;
   long done_iters = 0;
-  int rc = THR_OK;
   for (;;) {
-    for (int k = 0; k < batch; k++) {
-      rc = one_iteration(done_iters + k + 1, k == 0, k + 1 == batch);
-      if (rc) break;
-    }
-    if (rc) break;
+    for (int k = 0; k < batch; k++) TRY_RC(one_iteration());
     done_iters += batch;
-    if (hipMemcpyAsync(h, dev_flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-      set_error("stream synchronisation failed in solver loop");
-      rc = THR_ERR_HIP;
-      break;
-    }
-    if (*h) break;
-    if (done_iters > max_iters + 8) {
-      set_error("solver did not raise its stop flag");
-      rc = THR_ERR_STATE;
-      break;
-    }
+    THR_HIP(hipMemcpyAsync(h, dev_flag, sizeof(int), hipMemcpyDeviceToHost, s));
+    THR_HIP(hipStreamSynchronize(s));
+    if (*h) return THR_OK;
+    THR_CHECK(done_iters <= max_iters + 8, THR_ERR_STATE, "solver did not raise its stop flag");
     if (batch < 64) batch *= 2;
   }
-  return rc;
 }
 
 size_t cg_state_bytes() { return sizeof(CgState); }
@@ -678,10 +661,27 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
     THR_HIP(hipGetLastError());
     return THR_OK;
   };
-  TRY_RC(run_batched(iter, &st->stop, s, niterc, host_flag));
-  CgState hs;
-  THR_HIP(hipMemcpyAsync(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-  THR_HIP(hipStreamSynchronize(s));
+  // Batches between polls: each poll drains the stream (15 us), each iteration
+  // enqueued past the end is two launches that find the stop flag (6 us).  From
+  // the third poll on the next batch is most of what the mean rate of decay
+  // since the last poll leaves to do.
+  CgState local;
+  CgState *pinned = host_flag ? nullptr : (CgState *)host_workspace(22, sizeof(CgState));
+  CgState &hs = pinned ? *pinned : local;
+  int batch = 4;
+  double was = 0.0;
+  for (long k = 0;;) {
+    for (int b = 0; b < batch; b++) TRY_RC(iter(k + b + 1, b == 0, b + 1 == batch));
+    k += batch;
+    THR_HIP(hipMemcpyAsync(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+    THR_HIP(hipStreamSynchronize(s));
+    if (hs.stop) break;
+    THR_CHECK(k <= (long)niterc + 8, THR_ERR_STATE, "solver did not raise its stop flag");
+    const double now = std::log(hs.lam[k & 1] / (double)resid);
+    const double left = was > now ? now / (was - now) * batch : 128.0;
+    batch = was == 0.0 ? 8 : (int)std::max(4.0, std::min(std::min(64.0, 2.0 * batch), 0.8 * left));
+    was = now;
+  }
   *itercg = hs.itercg;
   if (iterations) *iterations = hs.iterations;
   THR_CHECK(hs.stop != 3, THR_ERR_NONFINITE,
@@ -846,7 +846,7 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   THR_HIP(hipGetLastError());
   const int *stop = &st->stop;
   const int nbl = op_partials(op, cfg);
-  auto iter = [&](long, bool, bool) -> int {
+  auto iter = [&]() -> int {
     DslashLaunch a{};
     a.in = p;
     a.out = h;
@@ -918,7 +918,7 @@ int multishift_reference_sp(const OpDesc &op, int n, const double *aden, const d
   L.done = stop;
   L.done_stride = 1;
   L.partial = partial;
-  auto iter = [&](long, bool, bool) -> int {
+  auto iter = [&]() -> int {
     DslashLaunch a = L;
     a.dagger = 0;
     a.in = p;

@@ -112,7 +112,10 @@ template <bool DAG, int MODE>
 __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigned wseg,
                                                    const WallCoef wall) {
   const int rhs = blockIdx.y;
-  if (L.done && L.done[(long)rhs * L.done_stride]) return;
+  // one batch of argument loads (see k_dslash_site)
+  asm volatile("" ::"s"(L.done), "s"(L.fsum), "s"(L.fdelta), "s"(L.b_ptr), "s"(L.r), "s"(L.in),
+               "s"(L.out), "s"(L.links), "s"(L.partial), "s"(L.d.lx), "s"(L.am3), "s"(wseg));
+  const int done = L.done ? L.done[(long)rhs * L.done_stride] : 0;
   const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   const unsigned nl = BLK / wseg, nb2 = (v2 + nl - 1) / nl;  // lines per block, blocks per t
@@ -170,7 +173,8 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
     if constexpr (MODE == EPI_HPREC) ld_spinor((const double2 *)L.x + off, v5, i, pold.v);
     if constexpr (MODE == EPI_CG) ld_spinor((const double2 *)L.r + off, v5, i, old.v);
   }
-  asm volatile("" ::: "memory");  // the loads stay above the barriers
+  asm volatile("" ::: "memory");  // the loads stay above the branch and the barriers
+  if (done) return;
   if constexpr (SUM) {
     if (fsum) {  // the order of partial_sum
       double v = 0.0;
@@ -178,7 +182,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
       for (int k = 0; k < NP; k++)
         if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
       for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += L.fsum[k];
-      v = block_value(block_sum(v));
+      v = block_sum_once<BLK, 1>(v);
       if (blockIdx.x == nbl) {
         scalar_step(L.scal, L.sst, L.sslot, v);
         return;
@@ -253,7 +257,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
     }
   }
   if constexpr (MODE != EPI_STORE) {
-    const double tot = block_sum(red);
+    const double tot = block_sum_once<BLK, 2>(red);
     if (threadIdx.x == 0) L.partial[(long)rhs * nbl + blockIdx.x] = tot;
   }
 }
