@@ -190,3 +190,28 @@ def test_congrad_batches_at_the_cap(G, niterc, pinned):
     o = O.congrad(phi, xo, u, dims, res=1e-9, am=0.1, imass=3, niterc=niterc)
     assert g == o
     assert rel(O.interior(xg), O.interior(xo)) <= 1e-11
+
+
+# the marching kernel (32 < Ls <= 64, Lx % 4 == 0): whole groups of 8 pairs and
+# pairs left over, more than one launch of 32 pairs, t chunks with a remainder;
+# and the one-step kernel with a block count that is no multiple of 8
+@pytest.mark.parametrize("dims,npair", [((4, 3, 5, 33), 3), ((4, 3, 5, 48), 9), ((8, 6, 21, 64), 40),
+                                        ((3, 5, 3, 20), 33), ((16, 16, 9, 40), 32)])
+def test_derivs_batch_splits(G, dims, npair):
+    """Against the single derivs of each pair, summed: the same terms in another
+    order of additions, 1e-13 of the sum's norm."""
+    from hiprt import DeviceArray
+    lx, ly, lt, ls = dims
+    rng = np.random.default_rng(40)
+    nsp = 4 * lx * ly * lt * ls
+    few = [DeviceArray.from_host(rng.standard_normal((nsp, 2))) for _ in range(6)]
+    rs = [few[k % 6] for k in range(npair)]
+    xs = [few[(k + 1 + k // 6) % 6] for k in range(npair)]
+    an, fl = 0.1 + rng.random(npair), [k % 2 for k in range(npair)]
+    base = rng.standard_normal(3 * lx * ly * lt)
+    one, all_ = DeviceArray.from_host(base), DeviceArray.from_host(base)
+    print("case: derivs batch splits", dims, npair, flush=True)
+    for k in range(npair):
+        G.derivs_dev(rs[k], xs[k], an[k], fl[k], dims, one)
+    G.derivs_batch_dev(rs, xs, an, fl, dims, all_)
+    assert rel(all_.to_host(), one.to_host()) <= 1e-13

@@ -853,13 +853,13 @@ int thr_derivs_batch_dev(const void *const *r, const void *const *x2, const doub
     THR_CHECK(iflag[k] == 0 || iflag[k] == 1, THR_ERR_ARG, "iflag must be 0 or 1");
     ph[k] = derivs_pair((const double2 *)r[k], (const double2 *)x2[k], anum[k], iflag[k]);
   }
-  DerivPair *pd = (DerivPair *)workspace(456, sizeof(DerivPair) * npair);
   double *part = (double *)workspace(457, sizeof(double) * 3 * d.v4() * npair);
-  THR_CHECK(pd && part, THR_ERR_HIP, "workspace allocation failed");
+  THR_CHECK(part, THR_ERR_HIP, "workspace allocation failed");
   hipStream_t s = pick(stream);
-  // launch_derivs_batch waits for the pair copy, so ph may go out of scope after it
-  return done_if_default(stream,
-                         launch_derivs_batch(d, npair, ph.data(), pd, part, (double *)dsdpi, s));
+  TRY(launch_derivs_batch(d, npair, ph.data(), part, (double *)dsdpi, s));
+  // part is the context's: the next call, on whatever stream, writes it again
+  THR_HIP(hipStreamSynchronize(s));
+  return THR_OK;
 }
 
 int thr_multishift_dev(const void *links64, const int dims[4], float am, int imass, float am3,

@@ -152,11 +152,10 @@ struct DerivPair {
   double w1, w2;
 };
 DerivPair derivs_pair(const double2 *R, const double2 *X2, double anum, int iflag);
-// dSdpi += the Shamir derivs of every pair, in one pass (Ls <= 64);
-// pairs_dev: device buffer of npair entries (filled from pairs_host); part:
-// device buffer of npair * 3 V4 doubles (the pairs' terms before their sum)
-int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs_host,
-                        DerivPair *pairs_dev, double *part, double *dsdpi, hipStream_t s);
+// dSdpi += the Shamir derivs of every pair (a host array), in one pass (Ls <= 64);
+// part: device buffer of npair * 3 V4 doubles (the pairs' terms before their sum)
+int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs, double *part,
+                        double *dsdpi, hipStream_t s);
 // fermion force (derivs_module.F90:99-196), FP64, accumulates into dsdpi [mu][t][y][x]
 int launch_derivs(const Dims &d, const double2 *R, const double2 *X2, double anum, int iflag,
                   double *dsdpi, hipStream_t s);

@@ -195,10 +195,9 @@ int qmrherm_device(const OpDesc &op, const double2 *phi, double2 *x, float res, 
     // loop below; dSdpi receives their sum once)
     double2 *mx = (double2 *)workspace(454, sizeof(double2) * ns * n);
     double2 *mr = iflag == 3 ? (double2 *)workspace(455, sizeof(double2) * ns * n) : nullptr;
-    DerivPair *pd = (DerivPair *)workspace(456, sizeof(DerivPair) * 2 * n);
-    DerivPair *ph = (DerivPair *)host_workspace(11, sizeof(DerivPair) * 2 * n);
+    DerivPair ph[2 * MAXRHS];
     double *part = (double *)workspace(457, sizeof(double) * 3 * d.v4() * 2 * n);
-    THR_CHECK(mx && pd && ph && part && (iflag == 2 || mr), THR_ERR_HIP,
+    THR_CHECK(mx && part && (iflag == 2 || mr), THR_ERR_HIP,
               "workspace allocation failed");
     DslashLaunch L{};
     L.d = d;
@@ -228,7 +227,7 @@ int qmrherm_device(const OpDesc &op, const double2 *phi, double2 *x, float res, 
         ph[np++] = derivs_pair(mr + (long)k * ns, x1 + (long)k * ns, coeff, 1);
       }
     }
-    return launch_derivs_batch(d, np, ph, pd, part, dsdpi, s);
+    return launch_derivs_batch(d, np, ph, part, dsdpi, s);
   }
   double2 *x2 = (double2 *)workspace(452, sizeof(double2) * ns);
   THR_CHECK(x2, THR_ERR_HIP, "workspace allocation failed");

@@ -348,29 +348,58 @@ template <int MU>
 __device__ inline double derivs_term(const cx<double> R0[4], const cx<double> X0[4],
                                      const cx<double> R1[4], const cx<double> X1[4], double w1,
                                      double w2) {
-  // gamval(mu, a) / akappa (gammamatrices.F90:27-75) and gamin(mu, a) - 1
-  constexpr double gre[3][4] = {{0, 0, 0, 0}, {-1, 1, 1, -1}, {0, 0, 0, 0}};
-  constexpr double gim[3][4] = {{-1, -1, 1, 1}, {0, 0, 0, 0}, {-1, 1, 1, -1}};
-  constexpr int gin[3][4] = {{3, 2, 1, 0}, {3, 2, 1, 0}, {2, 3, 0, 1}};
+  // gamval(mu, a) / akappa is one of +-1, +-i (kGamE): of the complex product
+  // only the part that it turns into an imaginary one is formed.  Written as
+  // full complex products (the compiler keeps products with a literal 0) the
+  // term took twice the FP64 operations: 5 of 160 us of the batched kernel.
   double sw = 0.0, sd = 0.0;
 #pragma unroll
   for (int a = 0; a < 4; a++) {
-    const int b = gin[MU][a];
-    sw += cjmul(R0[a], X1[a]).i - cjmul(R1[a], X0[a]).i;
-    const cx<double> g{0.5 * gre[MU][a], 0.5 * gim[MU][a]};
-    sd += cmul(g, cjmul(R0[a], X1[b]) + cjmul(R1[a], X0[b])).i;
+    const int b = kGamP[MU][a], e = kGamE[MU][a];
+    sw += R0[a].r * X1[a].i;
+    sw -= R0[a].i * X1[a].r;
+    sw -= R1[a].r * X0[a].i;
+    sw += R1[a].i * X0[a].r;
+    double z;
+    if (e < 2) {  // +-1: Im (R0_a^* X1_b + R1_a^* X0_b)
+      z = R0[a].r * X1[b].i;
+      z -= R0[a].i * X1[b].r;
+      z += R1[a].r * X0[b].i;
+      z -= R1[a].i * X0[b].r;
+    } else {      // +-i: Re
+      z = R0[a].r * X1[b].r;
+      z += R0[a].i * X1[b].i;
+      z += R1[a].r * X0[b].r;
+      z += R1[a].i * X0[b].i;
+    }
+    sd = (e & 1) ? sd - z : sd + z;
   }
-  return w1 * sw + w2 * sd;
+  return w1 * sw + (0.5 * w2) * sd;
 }
 
-// LDS x exchange of the batched derivs: with 64-lane segments (32 < Ls <=
-// 64) and Lx % 4 == 0 a block's 4 waves are 4 consecutive x of one (y, t),
-// so the x+1 neighbour of waves 0-2 is the centre of the next wave: each wave
-// stores its centre (R and X2, 8 complex numbers per lane, 32 KB per block)
-// and reads the next wave's instead of loading it; wave 3 loads its own.
-// 32^3 x 64, 25 poles: 1.74 against 1.82 ms; 16^3 x 48 even.  The same in
-// the single derivs march (two barriers per t step, 156 against 128 VGPRs:
-// 3 waves per SIMD instead of 4) was slower (84 against 78 us at 32^3 x 64).
+// sum of v over each segment of w lanes (a power of two), valid in all of its
+// lanes: the butterfly of lane exchanges with register moves down to
+// 16 lanes (rotations of a row by 8 and 4 reach lane ^ 8 and ^ 4 when the step
+// before has made the lanes ^ 8 equal)
+__device__ inline double segment_sum(double v, unsigned w) {
+  if (w >= 64) v = swap_add<true>(v);
+  if (w >= 32) v = swap_add<false>(v);
+  if (w >= 16) {
+    v += dpp_value<0x128>(v);
+    v += dpp_value<0x124>(v);
+  } else if (w >= 8) {
+    v += __shfl_xor(v, 4, 64);
+  }
+  if (w >= 4) v += dpp_value<0x4E>(v);
+  if (w >= 2) v += dpp_value<0xB1>(v);
+  return v;
+}
+
+// LDS x exchange of the marching batched derivs: a block's 4 waves are 4
+// consecutive x of one y, so the x+1 neighbour of waves 0-2 is the centre of the
+// next wave: each wave stores its centre (R and X2, 8 complex numbers per lane,
+// 32 KB per block) and reads the next wave's instead of loading it; wave 3
+// loads its own.
 struct DXBuf {
   double2 (*b)[8][64];
   __device__ inline void put(unsigned w, unsigned ln, const cx<double> R[4],
@@ -469,17 +498,22 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg(const Dims d, const doubl
         X0[a] = Xt[a];
       }
     }
-    // every lane of the wave takes part in the shuffles (idle lanes add 0)
-    for (unsigned off = wseg >> 1; off > 0; off >>= 1) {
+    // every lane of the wave takes part (idle lanes add 0)
 #pragma unroll
-      for (int mu = 0; mu < 3; mu++) v[mu] += __shfl_xor(v[mu], (int)off, 64);
-    }
+    for (int mu = 0; mu < 3; mu++) v[mu] = segment_sum(v[mu], wseg);
     if (s == 0 && col < v2) {
 #pragma unroll
       for (int mu = 0; mu < 3; mu++) ds[(long)mu * v4 + col + v2 * t] += v[mu];
     }
   }
 }
+
+// pairs of one batched launch, passed by value: no copy to the device, and no
+// wait for one
+constexpr int DPAIRS = 32;
+struct DerivPairs {
+  DerivPair p[DPAIRS];
+};
 
 // k_derivs_seg over several (R, X2) pairs in one launch, one t step per
 // thread: blockIdx.y is the pair, so the GPU sweeps the pairs in order with
@@ -491,19 +525,25 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg(const Dims d, const doubl
 // (qmrherm_module.F90:143-181); one launch over all of them reads each
 // pair's fields once like separate calls but fills the GPU on lattices whose
 // single call cannot (25 MB per pair at 16^3 x 48).
-template <bool XL>
-__global__ __launch_bounds__(BLK, 3) void k_derivs_seg_batch(const Dims d,
-                                                          const DerivPair *__restrict__ pairs,
-                                                          unsigned wseg, double *part) {
+// Bound by memory: 629 MB for 25 pairs there, 101 us at the copy rate.  Blocks
+// go to the XCDs round robin, so XCD k takes the k-th eighth of a pair's
+// (t, y, x): neighbours in y and most in t are lines of its own L2 (in launch
+// order every line was fetched by up to four XCDs: 191 us at 16^3 x 48 with 25
+// pairs, so 156; k_derivs_march_batch takes 143).
+__global__ __launch_bounds__(BLK, 3) void k_derivs_seg_batch(const Dims d, const DerivPairs pairs,
+                                                          unsigned wseg, unsigned nb, double *part) {
   const unsigned lx = d.lx, ly = d.ly, lt = d.lt, ls = d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   const unsigned nl = BLK / wseg;           // lines per block
   const unsigned nb2 = (v2 + nl - 1) / nl;  // blocks per t slice
-  const unsigned t = blockIdx.x / nb2, lb = blockIdx.x - t * nb2;
+  // gridDim.x is nb rounded up to a multiple of 8
+  const unsigned b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (b >= nb) return;
+  const unsigned t = b / nb2, lb = b - t * nb2;
   const unsigned line = threadIdx.x / wseg, s = threadIdx.x - line * wseg;
   const unsigned col = lb * nl + line;  // 2-D site x + lx y
-  const bool valid = s < ls && col < v2 && t < lt;
-  const DerivPair P = pairs[blockIdx.y];
+  const bool valid = s < ls && col < v2;
+  const DerivPair P = pairs.p[blockIdx.y];
   unsigned x = 0, y = 0;
   if (col < v2) {
     x = col % lx;
@@ -514,55 +554,136 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg_batch(const Dims d,
   const unsigned j = s + ls * col + v3 * t, jx = s + ls * (xf + lx * y) + v3 * t;
   const unsigned jy = s + ls * (x + lx * yf) + v3 * t, jt = s + ls * col + v3 * tf;
   double v[3] = {0.0, 0.0, 0.0};
-  const unsigned w = threadIdx.x >> 6, ln = threadIdx.x & 63;
   cx<double> R0[4], X0[4], Rx[4], Xx[4], Ry[4], Xy[4], Rt[4], Xt[4];
   if (valid) {
     ld_spinor(P.r, v5, j, R0);
     ld_spinor(P.x2, v5, j, X0);
-    if (!XL || w == 3) {
-      ld_spinor(P.r, v5, jx, Rx);
-      ld_spinor(P.x2, v5, jx, Xx);
-    }
+    ld_spinor(P.r, v5, jx, Rx);
+    ld_spinor(P.x2, v5, jx, Xx);
     ld_spinor(P.r, v5, jy, Ry);
     ld_spinor(P.x2, v5, jy, Xy);
     ld_spinor(P.r, v5, jt, Rt);
     ld_spinor(P.x2, v5, jt, Xt);
-  }
-  if constexpr (XL) {
-    // x+1 of waves 0-2 from the next wave's centre (wseg = 64 and full
-    // blocks: every wave takes the barrier)
-    __shared__ double2 xraw[4][8][64];
-    const DXBuf xb{xraw};
-    if (valid) xb.put(w, ln, R0, X0);
-    __syncthreads();
-    if (valid && w < 3) xb.get(w + 1, ln, Rx, Xx);
   }
   if (valid) {
     v[0] = derivs_term<0>(R0, X0, Rx, Xx, P.w1, P.w2);
     v[1] = derivs_term<1>(R0, X0, Ry, Xy, P.w1, P.w2);
     v[2] = derivs_term<2>(R0, X0, Rt, Xt, P.w1, P.w2);
   }
-  // every lane of the wave takes part in the shuffles (idle lanes add 0)
-  for (unsigned off = wseg >> 1; off > 0; off >>= 1) {
+  // every lane of the wave takes part (idle lanes add 0)
 #pragma unroll
-    for (int mu = 0; mu < 3; mu++) v[mu] += __shfl_xor(v[mu], (int)off, 64);
-  }
-  if (s == 0 && col < v2 && t < lt) {
+  for (int mu = 0; mu < 3; mu++) v[mu] = segment_sum(v[mu], wseg);
+  if (s == 0 && col < v2) {
     double *o = part + (long)blockIdx.y * 3 * v4;
 #pragma unroll
     for (int mu = 0; mu < 3; mu++) o[(long)mu * v4 + col + v2 * t] = v[mu];
   }
 }
 
-// dSdpi[e] += sum over the pairs, in pair order, of part[pair][e]
-__global__ __launch_bounds__(BLK) void k_derivs_sum_pairs(long n, int npair,
-                                                          const double *__restrict__ part,
-                                                          double *ds) {
-  const long e = (long)blockIdx.x * BLK + threadIdx.x;
+// The same for 64-lane segments (32 < Ls <= 64) with Lx % 4 == 0: a block is 4
+// consecutive x of one y, so x+1 of waves 0-2 comes through LDS, and it marches
+// tchunk t steps, the t+1 line of a step being the centre of the next: 2.25
+// instead of 3.25 lines loaded per line.  XCD k takes pair 8 g + k of each
+// group of 8 whole (no line is fetched twice across XCDs), and the k-th eighth
+// of each pair left over.  25 pairs, one call: 32^3 x 64 1.89 -> 1.53 ms, 16^3 x
+// 48 185 -> 180 us against k_derivs_seg_batch with the LDS exchange, which it
+// replaces.  Without the exchange (other Ls) the march did not pay: 24^3 x 32
+// 382 and 388 us.
+__global__ __launch_bounds__(BLK, 3) void k_derivs_march_batch(const Dims d, const DerivPairs pairs,
+                                                            unsigned nb, unsigned npair,
+                                                            unsigned tchunk, double *part) {
+  const unsigned lx = d.lx, ly = d.ly, lt = d.lt, ls = d.ls;
+  const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
+  const unsigned nb2 = v2 / 4;  // blocks per t chunk
+  // whole groups of 8 pairs: XCD k takes pair 8 g + k; the others: XCD k takes
+  // the k-th eighth of each pair
+  const unsigned xcd = blockIdx.x & 7, q = blockIdx.x >> 3, whole = npair & ~7u;
+  unsigned b, pair;
+  if (q < (whole >> 3) * nb) {
+    pair = q / nb;
+    b = q - pair * nb;
+    pair = pair * 8 + xcd;
+  } else {
+    const unsigned per = (nb + 7) / 8, q2 = q - (whole >> 3) * nb;
+    pair = q2 / per;
+    b = xcd * per + (q2 - pair * per);
+    pair += whole;
+    if (b >= nb) return;
+  }
+  const unsigned chunk = b / nb2, lb = b - chunk * nb2;
+  const unsigned t0 = chunk * tchunk, t1 = min(t0 + tchunk, lt);
+  const unsigned w = threadIdx.x >> 6, s = threadIdx.x & 63;
+  const unsigned col = lb * 4 + w;  // 2-D site x + lx y
+  const bool valid = s < ls;
+  const DerivPair P = pairs.p[pair];
+  const unsigned x = col % lx, y = col / lx;
+  const unsigned xf = (x + 1 == lx) ? 0 : x + 1, yf = (y + 1 == ly) ? 0 : y + 1;
+  const unsigned j = s + ls * col, jx = s + ls * (xf + lx * y), jy = s + ls * (x + lx * yf);
+  __shared__ double2 xraw[4][8][64];
+  const DXBuf xb{xraw};
+  cx<double> R0[4], X0[4];
+  if (valid) {
+    ld_spinor(P.r, v5, j + v3 * t0, R0);
+    ld_spinor(P.x2, v5, j + v3 * t0, X0);
+  }
+  double *o = part + (long)pair * 3 * v4;
+  for (unsigned t = t0; t < t1; t++) {
+    const unsigned tf = (t + 1 == lt) ? 0 : t + 1;
+    double v[3] = {0.0, 0.0, 0.0};
+    cx<double> Rx[4], Xx[4], Ry[4], Xy[4], Rt[4], Xt[4];
+    if (valid) {
+      if (w == 3) {
+        ld_spinor(P.r, v5, jx + v3 * t, Rx);
+        ld_spinor(P.x2, v5, jx + v3 * t, Xx);
+      }
+      ld_spinor(P.r, v5, jy + v3 * t, Ry);
+      ld_spinor(P.x2, v5, jy + v3 * t, Xy);
+      ld_spinor(P.r, v5, j + v3 * tf, Rt);
+      ld_spinor(P.x2, v5, j + v3 * tf, Xt);
+    }
+    if (t > t0) __syncthreads();  // the reads of the step before are done
+    if (valid) xb.put(w, s, R0, X0);
+    __syncthreads();
+    if (valid && w < 3) xb.get(w + 1, s, Rx, Xx);
+    if (valid) {
+      v[0] = derivs_term<0>(R0, X0, Rx, Xx, P.w1, P.w2);
+      v[1] = derivs_term<1>(R0, X0, Ry, Xy, P.w1, P.w2);
+      v[2] = derivs_term<2>(R0, X0, Rt, Xt, P.w1, P.w2);
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        R0[a] = Rt[a];
+        X0[a] = Xt[a];
+      }
+    }
+    // every lane of the wave takes part (idle lanes add 0)
+#pragma unroll
+    for (int mu = 0; mu < 3; mu++) v[mu] = wave_sum(v[mu]);
+    if (s == 0) {
+#pragma unroll
+      for (int mu = 0; mu < 3; mu++) o[(long)mu * v4 + col + v2 * t] = v[mu];
+    }
+  }
+}
+
+// dSdpi[e] += sum over the pairs, in pair order, of part[pair][e]; 8 loads in
+// flight per thread (one after another they took 11 us for 25 pairs at 16^3)
+__global__ __launch_bounds__(64) void k_derivs_sum_pairs(long n, int npair,
+                                                         const double *__restrict__ part,
+                                                         double *ds) {
+  const long e = (long)blockIdx.x * 64 + threadIdx.x;
   if (e >= n) return;
+  constexpr int U = 8;
+  const double d0 = ds[e];
   double v = 0.0;
-  for (int k = 0; k < npair; k++) v += part[(long)k * n + e];
-  ds[e] += v;
+  for (int k0 = 0; k0 < npair; k0 += U) {
+    double a[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) a[u] = part[(long)min(k0 + u, npair - 1) * n + e];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k0 + u < npair) v += a[u];
+  }
+  ds[e] = d0 + v;
 }
 
 __global__ __launch_bounds__(BLK) void k_derivs_march(const Dims d, const double2 *__restrict__ R,
@@ -874,7 +995,7 @@ DerivPair derivs_pair(const double2 *R, const double2 *X2, double anum, int ifla
   return DerivPair{R, X2, (double)(tzi * 0.5f), (double)tzi * (iflag == 0 ? 1.0 : -1.0)};
 }
 
-// the batched derivs' LDS x exchange applies with 64-lane segments (32 < Ls
+// the batched derivs' march with the LDS x exchange applies with 64-lane segments (32 < Ls
 // <= 64) when a block's 4 lines are 4 consecutive x of one y (Lx % 4 == 0);
 // THR_DERIVS_LDSX=0 switches it off
 static bool derivs_lds_x(const Dims &d, unsigned wseg) {
@@ -883,30 +1004,39 @@ static bool derivs_lds_x(const Dims &d, unsigned wseg) {
   return wseg == 64 && d.lx % 4 == 0;
 }
 
-int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs_host,
-                        DerivPair *pairs_dev, double *part, double *dsdpi, hipStream_t s) {
+int launch_derivs_batch(const Dims &d, int npair, const DerivPair *pairs, double *part,
+                        double *dsdpi, hipStream_t s) {
   THR_CHECK(npair >= 1 && npair <= 65535, THR_ERR_ARG, "derivs batch: 1..65535 pairs");
   THR_CHECK(d.v5() * 4 < (1L << 31), THR_ERR_SIZE, "derivs: 4*V5 must be below 2^31");
   THR_CHECK(d.ls <= 64, THR_ERR_ARG, "derivs batch: Ls above 64");
-  THR_CHECK(pairs_dev && part, THR_ERR_ARG, "derivs batch: NULL buffer");
+  THR_CHECK(part, THR_ERR_ARG, "derivs batch: NULL buffer");
   const long n = 3 * d.v4();
-  THR_HIP(hipMemcpyAsync(pairs_dev, pairs_host, sizeof(DerivPair) * npair, hipMemcpyHostToDevice,
-                         s));
   const unsigned w = segment(d.ls);
   const unsigned nl = BLK / w;
   const unsigned v2 = (unsigned)(d.lx * d.ly);
-  const unsigned nb = ((v2 + nl - 1) / nl) * (unsigned)d.lt;
-  if (derivs_lds_x(d, w))
-    hipLaunchKernelGGL(k_derivs_seg_batch<true>, dim3(nb, npair), dim3(BLK), 0, s, d,
-                       (const DerivPair *)pairs_dev, w, part);
-  else
-    hipLaunchKernelGGL(k_derivs_seg_batch<false>, dim3(nb, npair), dim3(BLK), 0, s, d,
-                       (const DerivPair *)pairs_dev, w, part);
-  hipLaunchKernelGGL(k_derivs_sum_pairs, dim3((unsigned)((n + BLK - 1) / BLK)), dim3(BLK), 0, s, n,
-                     npair, (const double *)part, dsdpi);
+  const bool march = derivs_lds_x(d, w);
+  for (int k0 = 0; k0 < npair; k0 += DPAIRS) {
+    const int np = std::min(DPAIRS, npair - k0);
+    DerivPairs P{};
+    std::copy(pairs + k0, pairs + k0 + np, P.p);
+    double *out = part + (long)k0 * n;
+    if (march) {
+      // t steps per block: up to 8 as long as the launch keeps 2048 blocks
+      const long steps = (long)(v2 / 4) * d.lt * np;
+      const unsigned tc = (unsigned)std::max(1L, std::min({8L, (long)d.lt, steps / 2048}));
+      const unsigned nb = (v2 / 4) * ((d.lt + tc - 1) / tc);
+      const unsigned grid = 8 * ((unsigned)(np / 8) * nb + (unsigned)(np % 8) * ((nb + 7) / 8));
+      hipLaunchKernelGGL(k_derivs_march_batch, dim3(grid), dim3(BLK), 0, s, d, P, nb, (unsigned)np,
+                         tc, out);
+    } else {
+      const unsigned nb = ((v2 + nl - 1) / nl) * (unsigned)d.lt;
+      hipLaunchKernelGGL(k_derivs_seg_batch, dim3((nb + 7) / 8 * 8, (unsigned)np), dim3(BLK), 0, s,
+                         d, P, w, nb, out);
+    }
+  }
+  hipLaunchKernelGGL(k_derivs_sum_pairs, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, n, npair,
+                     (const double *)part, dsdpi);
   THR_HIP(hipGetLastError());
-  // the host pair array must outlive the copy
-  THR_HIP(hipStreamSynchronize(s));
   return THR_OK;
 }
 
