@@ -15,8 +15,11 @@
 // dimension neighbours s+-1 are the adjacent lanes' centre loads and hit in
 // L1; the spin projection and gamma algebra are register arithmetic (no
 // MFMA: the operator is a sparse stencil, not a dense contraction).
+#include <unistd.h>
+
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -1131,6 +1134,14 @@ struct TuneKey {
 std::mutex g_tune_mu;
 std::map<TuneKey, DslashConfig> g_tuned;
 
+// whether any override is in the environment: one pass over it instead of ten
+// (every launch without a pinned shape asks)
+bool dslash_env_set() {
+  for (char **e = environ; e && *e; e++)
+    if (std::strncmp(*e, "THR_DSLASH_", 11) == 0) return true;
+  return false;
+}
+
 // The default shape of a launch, from the times of every shape over 17
 // lattices (8^4 to 32^3 x 64), 1 to 16 right-hand sides and all precisions on
 // fields that rotate beyond the Infinity Cache (us, one right-hand side
@@ -1174,6 +1185,7 @@ DslashConfig default_config(const Dims &d, int prec, int nrhs) {
   c.laneshift = (64 % d.ls) == 0 ? 1 : 0;
   c.uniform_links = lines ? 1 : 0;
   c.lds_x = c.uniform_links;
+  if (!dslash_env_set()) return c;
   if (const char *e = std::getenv("THR_DSLASH_SITE")) c.site = std::atoi(e) ? 1 : 0;
   if (const char *e = std::getenv("THR_DSLASH_TCHUNK")) c.tchunk = std::max(1, std::atoi(e));
   if (const char *e = std::getenv("THR_DSLASH_REMAP")) c.remap = std::atoi(e) ? 1 : 0;

@@ -152,8 +152,30 @@ def _p(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+_I4 = ctypes.c_int * 4
+
+
 def _dims(dims):
-    return (ctypes.c_int * 4)(*[int(d) for d in dims])
+    return _I4(*[int(d) for d in dims])
+
+
+def _addr(a):
+    """_p as a plain integer (or None), which a c_void_p argument takes as it
+    is: a device call of a few microseconds makes five of these."""
+    if a is None or type(a) is int:
+        return a
+    ptr = getattr(a, "data_ptr", None)
+    return ptr() if ptr is not None else _p(a).value
+
+
+def _masses(am, nrhs):
+    """One float per right-hand side from a number or a sequence of them."""
+    if nrhs == 1 and type(am) in (float, int):
+        return (F32 * 1)(am)
+    if type(am) in (list, tuple) and len(am) == nrhs:
+        return (F32 * nrhs)(*am)
+    ams = np.ascontiguousarray(np.broadcast_to(np.asarray(am, dtype=np.float32), (nrhs,)))
+    return (F32 * nrhs)(*ams.tolist())
 
 
 def halo5(a):
@@ -463,11 +485,9 @@ def hamilton(phi, res2, am, imass, beta, theta, pp, u, dims, coeffs, am3=1.0,
 # ---- device-resident API --------------------------------------------------
 
 def _stream(stream):
-    if stream is None:
-        return None
-    if isinstance(stream, int):
-        return ctypes.c_void_p(stream)
-    return ctypes.c_void_p(stream.ptr)
+    if stream is None or isinstance(stream, int):
+        return stream
+    return stream.ptr
 
 
 def coef_dev(links64, theta_dev, dims, ibound=-1, stream=None):
@@ -508,10 +528,10 @@ def norms_dev(x, nvec, n, stream=None):
 def dslash_dev(out, inp, links, dims, am, imass=3, am3=1.0, dagger=False, prec="f64",
                in_norm=None, out_norm=None, nrhs=1, stream=None):
     init()
-    ams = np.ascontiguousarray(np.broadcast_to(np.asarray(am, dtype=np.float32), (nrhs,)))
-    _check(lib().thr_dslash_dev(_p(out), _p(out_norm), _p(inp), _p(in_norm), _p(links),
-                                _dims(dims), int(nrhs), _p(ams), int(imass), am3,
-                                int(bool(dagger)), PREC[prec], _stream(stream)), "dslash_dev")
+    _check(lib().thr_dslash_dev(_addr(out), _addr(out_norm), _addr(inp), _addr(in_norm),
+                                _addr(links), _dims(dims), int(nrhs), _masses(am, int(nrhs)),
+                                int(imass), am3, int(bool(dagger)), PREC[prec],
+                                _stream(stream)), "dslash_dev")
 
 
 SHAPE_XCD_REMAP, SHAPE_UNIFORM_LINKS, SHAPE_LANESHIFT, SHAPE_XCD_BOXES, SHAPE_LDS_X = 1, 2, 4, 8, 16
@@ -566,8 +586,8 @@ def derivs_dev(r, x2, anum, iflag, dims, dsdpi, am=0.0, imass=3, kernel="shamir"
     """derivs on device fields (R, X2 spinors, dsdpi [mu][t][y][x] float64,
     accumulated in place)."""
     init()
-    _check(lib().thr_derivs_dev(_p(r), _p(x2), float(anum), int(iflag), _dims(dims), am,
-                                int(imass), KERNEL[kernel], _p(dsdpi), _stream(stream)),
+    _check(lib().thr_derivs_dev(_addr(r), _addr(x2), float(anum), int(iflag), _dims(dims), am,
+                                int(imass), KERNEL[kernel], _addr(dsdpi), _stream(stream)),
            "derivs_dev")
     return dsdpi
 
@@ -579,11 +599,11 @@ def derivs_batch_dev(rs, x2s, anums, iflags, dims, dsdpi, stream=None):
     n = len(rs)
     if not (len(x2s) == len(anums) == len(iflags) == n):
         raise ValueError("rs, x2s, anums and iflags must have the same length")
-    rp = (ctypes.c_void_p * n)(*[_p(a).value for a in rs])
-    xp = (ctypes.c_void_p * n)(*[_p(a).value for a in x2s])
+    rp = (ctypes.c_void_p * n)(*[_addr(a) for a in rs])
+    xp = (ctypes.c_void_p * n)(*[_addr(a) for a in x2s])
     an = np.ascontiguousarray(anums, dtype=np.float64)
     fl = np.ascontiguousarray(iflags, dtype=np.int32)
-    _check(lib().thr_derivs_batch_dev(rp, xp, _p(an), _p(fl), int(n), _dims(dims), _p(dsdpi),
+    _check(lib().thr_derivs_batch_dev(rp, xp, _p(an), _p(fl), int(n), _dims(dims), _addr(dsdpi),
                                       _stream(stream)), "derivs_batch_dev")
     return dsdpi
 
