@@ -510,8 +510,8 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
   bool valid;
   if (TL.mode == TILE_BOXES) {
     const unsigned k = blockIdx.x & 7, l = blockIdx.x >> 3;
-    const unsigned rx = k % TL.px, ry = (k / TL.px) % TL.py, rt = k / (TL.px * TL.py);
-    const unsigned chunk = l / TL.nb3;
+    const unsigned kx = k / TL.dpx, rx = k - kx * TL.px, rt = kx / TL.dpy, ry = kx - rt * TL.py;
+    const unsigned chunk = l / TL.dnb3;
     t0 = rt * TL.bt + chunk * TL.tchunk;
     t1 = min(t0 + TL.tchunk, rt * TL.bt + TL.bt);
     if constexpr (YL) {
@@ -523,10 +523,10 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
     } else {
       const unsigned jr = (l - chunk * TL.nb3) * BLK + threadIdx.x;
       valid = jr < ls * TL.bx * TL.by && chunk * TL.tchunk < TL.bt;
-      s = jr % ls;
-      const unsigned q = jr / ls;
-      x = rx * TL.bx + q % TL.bx;
-      y = ry * TL.by + q / TL.bx;
+      const unsigned q = jr / TL.dls, qy = q / TL.dnx;
+      s = jr - q * ls;
+      x = rx * TL.bx + (q - qy * TL.bx);
+      y = ry * TL.by + qy;
     }
     j = s + ls * (x + lx * y);
   } else {
@@ -536,7 +536,7 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
       const unsigned nbl = gridDim.x, per = nbl >> 3, full = per << 3;
       if (b < full) b = (b & 7) * per + (b >> 3);
     }
-    const unsigned chunk = b / TL.nb3;
+    const unsigned chunk = b / TL.dnb3;
     t0 = chunk * TL.tchunk;
     t1 = min(t0 + TL.tchunk, lt);
     if constexpr (YL) {
@@ -549,10 +549,10 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
     } else {
       j = (b - chunk * TL.nb3) * BLK + threadIdx.x;
       valid = j < v3 && t0 < lt;
-      s = j % ls;
-      const unsigned xy = j / ls;
-      x = xy % lx;
-      y = xy / lx;
+      const unsigned xy = j / TL.dls;
+      s = j - xy * ls;
+      y = xy / TL.dnx;
+      x = xy - y * lx;
     }
   }
   double red = 0.0;
@@ -881,10 +881,10 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   bool valid;
   if (TL.mode == TILE_BOXES) {
     const unsigned k = blockIdx.x & 7, l = blockIdx.x >> 3;
-    const unsigned rx = k % TL.px, ry = (k / TL.px) % TL.py, rt = k / (TL.px * TL.py);
-    const unsigned chunk = l / TL.nb3, jr = (l - chunk * TL.nb3) * BLK + threadIdx.x;
+    const unsigned kx = k / TL.dpx, rx = k - kx * TL.px, rt = kx / TL.dpy, ry = kx - rt * TL.py;
+    const unsigned chunk = l / TL.dnb3, jr = (l - chunk * TL.nb3) * BLK + threadIdx.x;
     valid = jr < ls * TL.bx * TL.by;
-    const unsigned q = jr / ls;
+    const unsigned q = jr / TL.dls, qy = q / TL.dnx;
     s = jr - q * ls;
     x = rx * TL.bx + q % TL.bx;
     y = ry * TL.by + q / TL.bx;
@@ -895,12 +895,12 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
       const unsigned per = nbl >> 3, full = per << 3;
       if (b < full) b = (b & 7) * per + (b >> 3);
     }
-    t = b / TL.nb3;
+    t = b / TL.dnb3;
     const unsigned j = (b - t * TL.nb3) * BLK + threadIdx.x;
     valid = j < v3;
-    const unsigned xy = j / ls;
+    const unsigned xy = j / TL.dls;
     s = j - xy * ls;
-    y = xy / lx;
+    y = xy / TL.dnx;
     x = xy - y * lx;
   }
   if (t >= lt) t = 0;  // the scalar block: no site of its own
@@ -1270,6 +1270,11 @@ static size_t lds_pad(const void *kern, int cap) {
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) !=
             hipSuccess ||
+  TL.dnb3 = fast_div(TL.nb3);
+  TL.dls = fast_div((unsigned)d.ls);
+  TL.dpx = fast_div(px);
+  TL.dpy = fast_div(py);
+  TL.dnx = fast_div(TL.mode == TILE_BOXES ? TL.bx : (unsigned)d.lx);
         hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) !=
             hipSuccess) {
       lds_cu = lds_blk = 0;

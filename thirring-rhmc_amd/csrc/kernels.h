@@ -91,6 +91,22 @@ struct DslashConfig {
   int site = 0;           // one site per thread, all loads issued at once (small launches)
 };
 
+// division by a launch constant: n / d = (2 n m >> 32) >> l for n < 2^31, with
+// l = ceil(log2 d) and m = ceil(2^(31 + l) / d) (m d - 2^(31 + l) < d <= 2^l, so
+// the quotient's error stays below n / 2^31 < 1 / d).  Three instructions; a
+// division by a kernel argument is about twenty, and an index takes six.
+struct FastDiv {
+  unsigned m, l;
+};
+inline FastDiv fast_div(unsigned d) {
+  unsigned l = 0;
+  while ((1ull << l) < d) l++;
+  return FastDiv{(unsigned)(((1ull << (31 + l)) + d - 1) / d), l};
+}
+__host__ __device__ inline unsigned operator/(unsigned n, const FastDiv &d) {
+  return (unsigned)(((unsigned long long)(2u * n) * d.m) >> 32) >> d.l;
+}
+
 // block -> lattice mapping of one Dslash launch (see dslash.hip)
 enum TileMode { TILE_LINEAR = 0, TILE_REMAP = 1, TILE_BOXES = 2 };
 struct Tiling {
@@ -98,6 +114,7 @@ struct Tiling {
   unsigned tchunk, nb3, pstride;
   unsigned px, py;      // boxes: split of x and y (t split = 8 / (px py))
   unsigned bx, by, bt;  // boxes: box extents
+  FastDiv dnb3, dls, dpx, dpy, dnx;  // by nb3, Ls, px, py and the sites per row (bx or Lx)
   unsigned yl, ntx;     // 4 x 2-line blocks (lds_y); tiles per row of the slab or box
 };
 
