@@ -886,8 +886,8 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     valid = jr < ls * TL.bx * TL.by;
     const unsigned q = jr / TL.dls, qy = q / TL.dnx;
     s = jr - q * ls;
-    x = rx * TL.bx + q % TL.bx;
-    y = ry * TL.by + q / TL.bx;
+    x = rx * TL.bx + (q - qy * TL.bx);
+    y = ry * TL.by + qy;
     t = rt * TL.bt + chunk;
   } else {
     unsigned b = blockIdx.x;
