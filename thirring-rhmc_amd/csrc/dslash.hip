@@ -835,8 +835,20 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
 // waited for.  The neighbours along s wrap around the line, which is where the
 // wall terms read from, so the s hops and the walls need no loads of their own
 // behind branches.
+//
+// The FP64 passes that carry a solver's epilogue hold up to three fields more.
+// With all of it loaded up front they took 216 to 248 registers, two waves per
+// SIMD, and a launch of 768 blocks ran as one full round of 512 and one half
+// full; so they load the s neighbours and the epilogue's fields behind the
+// first hops, in the registers of the x neighbours, and three waves fit
+// (16^3 x 48: M + beta 13.4 -> 12.6 us, M^+ + r update 10.4 -> 9.6; the whole
+// multishift there 8.79 -> 8.32 ms, 24^3 x 40 31.3 -> 28.6, 24^3 x 60 50.9 ->
+// 44.5, 12^3 x 24, where every block is resident either way, 3.22 -> 3.24).
+constexpr bool site_late(int prec, int mode) {
+  return prec == P64 && (mode == EPI_CG || mode == EPI_HREC || mode == EPI_HPREC);
+}
 template <int PREC, bool DAG, int MODE, bool NT>
-__global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, const Tiling TL) {
+__global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_site(const DslashLaunch L, const Tiling TL) {
   using C = typename Store<PREC>::C;
   using T = typename Store<PREC>::T;
   const int rhs = blockIdx.y;
@@ -850,8 +862,16 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   constexpr bool HREC = MODE == EPI_HREC || MODE == EPI_HPREC;
   constexpr bool SUM = MODE == EPI_CG || HREC;
-  // the launch's field blocks; one more carries the scalar step
-  const unsigned nbl = gridDim.x - (SUM && PREC == P64 && L.scal ? 1u : 0u);
+  constexpr bool LATE = site_late(PREC, MODE);
+  // the launch's field blocks, after those of a scalar step
+  const unsigned lead = SUM && PREC == P64 && L.scal ? SCAL_LEAD : 0;
+  if constexpr (SUM && PREC == P64) {
+    if (blockIdx.x < lead) {
+      scalar_block(L);
+      return;
+    }
+  }
+  const unsigned bid = blockIdx.x - lead, nbl = gridDim.x - lead;
   // the first 4 * BLK partial sums of the previous pass
   const bool fsum = SUM && L.fsum;
   constexpr int NP = 4;
@@ -880,7 +900,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   unsigned s, x, y, t;
   bool valid;
   if (TL.mode == TILE_BOXES) {
-    const unsigned k = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const unsigned k = bid & 7, l = bid >> 3;
     const unsigned kx = k / TL.dpx, rx = k - kx * TL.px, rt = kx / TL.dpy, ry = kx - rt * TL.py;
     const unsigned chunk = l / TL.dnb3, jr = (l - chunk * TL.nb3) * BLK + threadIdx.x;
     valid = jr < ls * TL.bx * TL.by;
@@ -890,7 +910,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     y = ry * TL.by + qy;
     t = rt * TL.bt + chunk;
   } else {
-    unsigned b = blockIdx.x;
+    unsigned b = bid;
     if (TL.mode == TILE_REMAP) {
       const unsigned per = nbl >> 3, full = per << 3;
       if (b < full) b = (b & 7) * per + (b >> 3);
@@ -903,7 +923,6 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
     y = xy / TL.dnx;
     x = xy - y * lx;
   }
-  if (t >= lt) t = 0;  // the scalar block: no site of its own
   if (!valid) s = x = y = 0;  // loads a site that exists; nothing is stored
   const unsigned xy = x + lx * y, l4 = v2 * t;
   const unsigned xf = (x + 1 == lx) ? 0 : x + 1, xb = (x == 0) ? lx - 1 : x - 1;
@@ -922,32 +941,42 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   const Site<PREC> rtf = load_site(in, s + ls * xy + v3 * tf);
   const Site<PREC> rtb = load_site(in, s + ls * xy + v3 * tb);
   Spin<PREC> su[2], sd[2];
-  load_pair(in, s + 1 == ls ? col : i + 1, up0, su);
-  load_pair(in, s == 0 ? col + ls - 1 : i - 1, dn0, sd);
+  const auto load_s = [&] {
+    load_pair(in, s + 1 == ls ? col : i + 1, up0, su);
+    load_pair(in, s == 0 ? col + ls - 1 : i - 1, dn0, sd);
+  };
+  if constexpr (!LATE) load_s();
   const cx<C> uxf = lk(xy + l4), uxb = conj(lk(xb + lx * y + l4));
   const cx<C> uyf = lk(v4 + xy + l4), uyb = conj(lk(v4 + x + lx * yb + l4));
   const cx<C> utf = lk(2 * v4 + xy + l4), utb = conj(lk(2 * v4 + xy + v2 * tb));
-  Site<PREC> old{}, pold{};
-  if constexpr (HREC) {
-    const BAcc<PREC> ho((const T *)L.out + roff,
-                        L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
-    old = load_site(ho, i);
-  }
-  if constexpr (MODE == EPI_HPREC) {
-    const BAcc<PREC> po((const T *)L.x + roff, nullptr, v5);
-    pold = load_site(po, i);
-  }
-  Site<PREC> xold{};
+  Site<PREC> old{}, pold{}, xold{};
   const bool xup = MODE == EPI_CG && PREC != P16 && L.b_ptr;
-  if constexpr (MODE == EPI_CG && PREC != P16) {
-    if (xup) {
-      pold = load_site(BAcc<PREC>((const T *)L.p + roff, nullptr, v5), i);
-      xold = load_site(BAcc<PREC>((const T *)L.x + roff, nullptr, v5), i);
+  const auto load_old = [&] {
+    if constexpr (HREC) {
+      const BAcc<PREC> ho((const T *)L.out + roff,
+                          L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr, v5);
+      old = load_site(ho, i);
     }
-  }
-  if constexpr (MODE == EPI_CG) {
-    const BAcc<PREC> ro((const T *)L.r + roff, L.r_norm ? L.r_norm + (long)rhs * v5 : nullptr, v5);
-    old = load_site(ro, i);
+    if constexpr (MODE == EPI_HPREC) {
+      const BAcc<PREC> po((const T *)L.x + roff, nullptr, v5);
+      pold = load_site(po, i);
+    }
+    if constexpr (MODE == EPI_CG) {
+      const BAcc<PREC> ro((const T *)L.r + roff, L.r_norm ? L.r_norm + (long)rhs * v5 : nullptr, v5);
+      old = load_site(ro, i);
+    }
+  };
+  const auto load_px = [&] {
+    if constexpr (MODE == EPI_CG && PREC != P16) {
+      if (xup) {
+        pold = load_site(BAcc<PREC>((const T *)L.p + roff, nullptr, v5), i);
+        xold = load_site(BAcc<PREC>((const T *)L.x + roff, nullptr, v5), i);
+      }
+    }
+  };
+  if constexpr (!LATE) {
+    load_px();
+    load_old();
   }
   asm volatile("" ::: "memory");  // the loads stay above the branch and the barriers
   if (dn) return;
@@ -962,13 +991,7 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
       const double *p = L.fsum + (long)rhs * L.fsum_stride;
       for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += p[k];
       v = block_sum_once<BLK, 1>(v);
-      if (L.frec && blockIdx.x == 0 && threadIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
-      if constexpr (PREC == P64) {
-        if (L.scal && blockIdx.x == nbl) {
-          scalar_step(L.scal, L.sst, L.sslot, v);
-          return;
-        }
-      }
+      if (L.frec && bid == 0 && threadIdx.x == 0) L.frec[(long)rhs * L.sc_stride] = v;
       if constexpr (MODE == EPI_CG) {
         const double om = -sc / v;  // omega = -delta / alpha
         sc = -om;
@@ -989,7 +1012,21 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   cx<C> o[4];
   centre(o, diag, cur);
   hop<0, DAG>(o, uxf, rxf, uxb, rxb);
+  if constexpr (LATE) {
+    // behind the x hop (its result is an operand, and memory): no earlier
+    asm volatile("" : "+v"(o[0].r), "+v"(o[0].i), "+v"(o[1].r), "+v"(o[1].i), "+v"(o[2].r),
+                 "+v"(o[2].i), "+v"(o[3].r), "+v"(o[3].i)::"memory");
+    load_s();
+    load_old();
+    asm volatile("" ::: "memory");
+  }
   hop<1, DAG>(o, uyf, ryf, uyb, ryb);
+  if constexpr (LATE && MODE == EPI_CG) {
+    asm volatile("" : "+v"(o[0].r), "+v"(o[0].i), "+v"(o[1].r), "+v"(o[1].i), "+v"(o[2].r),
+                 "+v"(o[2].i), "+v"(o[3].r), "+v"(o[3].i)::"memory");
+    load_px();
+    asm volatile("" ::: "memory");
+  }
   hop<2, DAG>(o, utf, rtf, utb, rtb);
   if (!L.wilson4d) {
 #pragma unroll
@@ -1074,8 +1111,8 @@ __global__ __launch_bounds__(BLK, 2) void k_dslash_site(const DslashLaunch L, co
   if constexpr (MODE != EPI_STORE) {
     const double tot = block_sum_once<BLK, 2>(valid ? red : 0.0);
     double *P = L.partial + (long)rhs * TL.pstride;
-    if (threadIdx.x == 0) P[blockIdx.x] = tot;
-    if (blockIdx.x == 0)
+    if (threadIdx.x == 0) P[bid] = tot;
+    if (bid == 0)
       for (unsigned k = nbl + threadIdx.x; k < TL.pstride; k += BLK) P[k] = 0.0;
   }
 }
@@ -1246,6 +1283,11 @@ static Tiling make_tiling(const Dims &d, const DslashConfig &c, unsigned *nblock
     TL.nb3 = TL.yl ? TL.ntx * (d.ly / 2) : ((unsigned)d.lx * d.ly * d.ls + BLK - 1) / BLK;
     *nblocks = TL.nb3 * ((d.lt + TL.tchunk - 1) / TL.tchunk);
   }
+  TL.dnb3 = fast_div(TL.nb3);
+  TL.dls = fast_div((unsigned)d.ls);
+  TL.dpx = fast_div(px);
+  TL.dpy = fast_div(py);
+  TL.dnx = fast_div(TL.mode == TILE_BOXES ? TL.bx : (unsigned)d.lx);
   return TL;
 }
 
@@ -1270,11 +1312,6 @@ static size_t lds_pad(const void *kern, int cap) {
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) !=
             hipSuccess ||
-  TL.dnb3 = fast_div(TL.nb3);
-  TL.dls = fast_div((unsigned)d.ls);
-  TL.dpx = fast_div(px);
-  TL.dpy = fast_div(py);
-  TL.dnx = fast_div(TL.mode == TILE_BOXES ? TL.bx : (unsigned)d.lx);
         hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) !=
             hipSuccess) {
       lds_cu = lds_blk = 0;
@@ -1314,7 +1351,7 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
   unsigned nblocks = 0;
   const Tiling TL = make_tiling(L.d, c, &nblocks);
   THR_CHECK(nblocks <= TL.pstride, THR_ERR_ARG, "dslash grid exceeds partial stride");
-  dim3 grid(nblocks + (L.scal ? 1u : 0u), (unsigned)L.nrhs);
+  dim3 grid(nblocks + (L.scal ? SCAL_LEAD : 0u), (unsigned)L.nrhs);
   dim3 block(TL.yl ? 2 * BLK : BLK);
   const bool shuf = c.laneshift != 0;
   // a wave is exactly one s-line when Ls = 64, two when Ls = 32, four when

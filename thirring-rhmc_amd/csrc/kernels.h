@@ -19,6 +19,7 @@ enum EpiMode {
 
 // scalar step carried by a launch (krylov_scalars.h)
 enum ScalKind { SCAL_NONE = 0, SCAL_MS_ALPHA = 1, SCAL_MS_LAMBDA = 2, SCAL_CG_ALPHA = 3, SCAL_CG_BETA = 4 };
+constexpr unsigned SCAL_LEAD = 8;  // blocks in front of the field blocks of such a launch
 
 struct DslashLaunch {
   Dims d;
@@ -57,7 +58,7 @@ struct DslashLaunch {
   int fsum_n, fsum_stride;
   const double *fdelta;
   double *frec;        // null: not stored
-  // scalar step run by one more block of the launch on the same sum (the
+  // scalar step run by the launch's first block on the same sum (the
   // kernels of dslash_fuses_scalars and the Wilson kernel; one right-hand
   // side): the state's recurrences need the sum, the field work does not need
   // them, so they overlap with it instead of being a launch in between

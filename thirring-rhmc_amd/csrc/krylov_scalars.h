@@ -45,36 +45,48 @@ struct MsState {
 
 namespace {
 
+// sum: the dot product, called after the state's loads are issued, so that the
+// step waits once for both (see scalar_block)
+
 // alpha of a CG iteration from |M p|^2
-__device__ inline void cg_alpha_step(CgState *st, double alphad) {
+template <class F> __device__ inline void cg_alpha_step(CgState *st, F sum) {
+  const int nx = st->nx, itercg = st->itercg;
+  const double alphan = st->alphan;
+  asm volatile("" ::: "memory");
+  const double alphad = sum();
   if (threadIdx.x == 0) {
-    st->nx += 1;
-    st->itercg += 1;
-    st->alpha = st->alphan / alphad;
+    st->nx = nx + 1;
+    st->itercg = itercg + 1;
+    st->alpha = alphan / alphad;
     // a non-finite |M p|^2 (NaN or Inf in the source, the guess or the links)
     // can never meet the stopping rule: end the solve here instead of at niterc
-    if (!isfinite(alphad) || !isfinite(st->alpha)) {
+    if (!isfinite(alphad) || !isfinite(alphan / alphad)) {
       st->stop = 3;
-      st->iterations = st->nx;
+      st->iterations = nx + 1;
     }
   }
 }
 
 // beta and the stopping rule from |r|^2; slot: where lam of this iteration goes
-__device__ inline void cg_beta_step(CgState *st, double *slot, double bn) {
+template <class F> __device__ inline void cg_beta_step(CgState *st, double *slot, F sum) {
+  const int nx = st->nx, niterc = st->niterc;
+  const double alphan = st->alphan;
+  const float resid = st->resid;
+  asm volatile("" ::: "memory");
+  const double bn = sum();
   if (threadIdx.x == 0) {
-    st->betacg = st->nx == 1 ? 0.0 : bn / st->alphan;
+    st->betacg = nx == 1 ? 0.0 : bn / alphan;
     st->alphan = bn;
     *slot = bn;
     if (!isfinite(bn)) {
       st->stop = 3;
-      st->iterations = st->nx;
-    } else if (bn < (double)st->resid) {
+      st->iterations = nx;
+    } else if (bn < (double)resid) {
       st->stop = 1;
-      st->iterations = st->nx;
-    } else if (st->nx >= st->niterc) {
+      st->iterations = nx;
+    } else if (nx >= niterc) {
       // the Fortran loop ends with nx = niterc + 1
-      st->iterations = st->niterc + 1;
+      st->iterations = niterc + 1;
       st->stop = 2;
     }
   }
@@ -84,19 +96,22 @@ __device__ inline void cg_beta_step(CgState *st, double *slot, double bn) {
 // wave 0); each shift's arithmetic is the serial loop's.  One thread walking
 // 25 shifts took 5.9 (alpha) and 11.7 us (lambda) per launch at 16^3 x 48,
 // most of it the memory latency of one shift after another; so 2.6 and 3.4.
-__device__ inline void ms_alpha_step(MsState *st, double al) {
-  const double os = st->omega, gg = st->gammag, om = -st->delta / al;
+template <class F> __device__ inline void ms_alpha_step(MsState *st, F sum) {
+  const int i = threadIdx.x, ic = min(i, MAXSHIFT - 1), mini = st->mini, maxi = st->maxi,
+            cg = st->cg_return;
+  const double os = st->omega, gg = st->gammag, delta = st->delta;
+  const double z1 = st->zeta_i[ic], z2 = st->zeta_ii[ic], aden = st->aden[ic];
+  asm volatile("" ::: "memory");
+  const double al = sum(), om = -delta / al;
   const bool ok = isfinite(om);
-  const int i = threadIdx.x;
-  if (ok && i >= st->mini - 1 && i < st->maxi) {
-    const double z1 = st->zeta_i[i], z2 = st->zeta_ii[i];
-    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - st->aden[i] * om));
+  if (ok && i >= mini - 1 && i < maxi) {
+    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - aden * om));
     st->zeta_iii[i] = z3;
     st->omegas[i] = om * z3 / z2;
   }
   __syncthreads();  // every thread has read the scalars before thread 0 writes them
   if (threadIdx.x == 0) {
-    st->cg_return += 1;
+    st->cg_return = cg + 1;
     st->alpha = al;
     st->omega_save = os;
     st->omega = om;
@@ -113,9 +128,16 @@ __device__ inline void ms_alpha_step(MsState *st, double al) {
 
 // REC: record the iteration's shift scalars for the block's flush; slot: where
 // the next iteration's delta goes beside the state's
-template <bool REC>
-__device__ inline void ms_lambda_step(MsState *st, double *slot, double lam) {
+template <bool REC, class F>
+__device__ inline void ms_lambda_step(MsState *st, double *slot, F sum) {
   __shared__ int s_nmin, s_nmax;
+  const int i = threadIdx.x, ic = min(i, MAXSHIFT - 1), mini = st->mini, maxi = st->maxi,
+            n = st->n, j = st->jcount, cg = st->cg_return, maxcg = st->maxcg, flag = st->flags[ic];
+  const double delta = st->delta, om = st->omega, resd = st->resd;
+  const double zeta2 = st->zeta_ii[ic], zeta3 = st->zeta_iii[ic], omi = st->omegas[ic],
+               corr = st->corr[ic];
+  asm volatile("" ::: "memory");
+  const double lam = sum();
   if (!isfinite(lam)) {
     if (threadIdx.x == 0) {
       st->nonfinite = 1;
@@ -124,18 +146,16 @@ __device__ inline void ms_lambda_step(MsState *st, double *slot, double lam) {
     }
     return;
   }
-  const int i = threadIdx.x, mini = st->mini, maxi = st->maxi, n = st->n, j = st->jcount;
-  const double delta = st->delta, gg = lam / delta, om = st->omega, resd = st->resd;
-  const int cg = st->cg_return, maxcg = st->maxcg;
+  const double gg = lam / delta;
   if (i < 64) {  // wave 0: the ballot spans every shift
     const bool mine = i >= mini - 1 && i < maxi;
     double z2 = 0.0, z3 = 0.0;
     bool on = false;
     if (i < n) {
-      z2 = st->zeta_ii[i];
+      z2 = zeta2;
       if (mine) {
-        z3 = st->zeta_iii[i];
-        const double omi = st->omegas[i], ga = gg * z3 * omi / (z2 * om);
+        z3 = zeta3;
+        const double ga = gg * z3 * omi / (z2 * om);
         st->gammas[i] = ga;
         st->cg_returns[i] = cg;
         if constexpr (REC) {
@@ -145,7 +165,7 @@ __device__ inline void ms_lambda_step(MsState *st, double *slot, double lam) {
           st->cnt[i] = j + 1;
         }
       }
-      on = st->flags[i] && !(sqrt(delta * z2 * z2) * st->corr[i] < resd);
+      on = flag && !(sqrt(delta * z2 * z2) * corr < resd);
       if (!on) st->flags[i] = 0;
     }
     const unsigned long long live = __ballot(on);
@@ -181,7 +201,7 @@ __device__ inline void ms_lambda_step(MsState *st, double *slot, double lam) {
 __device__ inline const int *scalar_stop(int kind, const void *st) {
   return kind <= SCAL_MS_LAMBDA ? &((const MsState *)st)->stop : &((const CgState *)st)->stop;
 }
-__device__ inline void scalar_step(int kind, void *st, double *slot, double sum) {
+template <class F> __device__ inline void scalar_step(int kind, void *st, double *slot, F sum) {
   if (kind == SCAL_MS_ALPHA)
     ms_alpha_step((MsState *)st, sum);
   else if (kind == SCAL_MS_LAMBDA)
@@ -190,6 +210,30 @@ __device__ inline void scalar_step(int kind, void *st, double *slot, double sum)
     cg_alpha_step((CgState *)st, sum);
   else
     cg_beta_step((CgState *)st, slot, sum);
+}
+
+// The blocks in front of a launch's field blocks when it carries a scalar step.
+// The step is a chain of waits, so its block is the launch's first and waits
+// for the sum and the state together: as the last block it started when the
+// field blocks made room, and the multishift at 16^3 x 48 (768 field blocks)
+// took 9.73 ms against 9.33.  SCAL_LEAD of them, so that field block b still
+// runs on XCD b % 8.
+__device__ inline void scalar_block(const DslashLaunch &L) {
+  if (blockIdx.x) return;
+  constexpr int NP = 4;
+  double part[NP];
+  const int dn = L.done ? *L.done : 0;
+#pragma unroll
+  for (int k = 0; k < NP; k++) part[k] = L.fsum[min((int)threadIdx.x + k * BLK, L.fsum_n - 1)];
+  if (dn) return;
+  scalar_step(L.scal, L.sst, L.sslot, [&] {
+    double v = 0.0;  // the field blocks' order of summation
+#pragma unroll
+    for (int k = 0; k < NP; k++)
+      if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
+    for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += L.fsum[k];
+    return block_sum_once<BLK, 3>(v);
+  });
 }
 
 }  // namespace

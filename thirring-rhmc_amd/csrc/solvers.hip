@@ -259,7 +259,7 @@ __global__ void k_cg_init(CgState *st, float resid, int niterc) {
 __global__ __launch_bounds__(BLK) void k_scalar(int kind, void *st, double *slot,
                                                 const double *partial, int nb) {
   if (*scalar_stop(kind, st)) return;
-  scalar_step(kind, st, slot, partial_sum(partial, nb));
+  scalar_step(kind, st, slot, [&] { return partial_sum(partial, nb); });
 }
 
 __global__ __launch_bounds__(BLK) void k_ms_init(MsState *st, const double *partial, int nb) {
@@ -299,11 +299,11 @@ __global__ __launch_bounds__(BLK) void k_ms_alpha(MsState *st, const double *par
     if (threadIdx.x == 0) st->done = 1;
     return;
   }
-  ms_alpha_step(st, partial_sum(partial, nb));
+  ms_alpha_step(st, [&] { return partial_sum(partial, nb); });
 }
 __global__ __launch_bounds__(BLK) void k_ms_lambda(MsState *st, const double *partial, int nb) {
   if (st->stop) return;
-  ms_lambda_step<false>(st, nullptr, partial_sum(partial, nb));
+  ms_lambda_step<false>(st, nullptr, [&] { return partial_sum(partial, nb); });
 }
 
 // The block's coefficients from its recorded scalars, one thread per shift.
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(BLK) void k_ms_lambda(MsState *st, const double *pa
 // The block's last lambda (its iteration's partial sums) is taken here too.
 __global__ __launch_bounds__(BLK) void k_ms_coef(MsState *st, const double *partial, int nb) {
   if (!st->stop) {  // uniform: nothing writes it before every thread has read it
-    ms_lambda_step<true>(st, st->dl, partial_sum(partial, nb));
+    ms_lambda_step<true>(st, st->dl, [&] { return partial_sum(partial, nb); });
     __syncthreads();
   }
   const int i = threadIdx.x, n = st->n;

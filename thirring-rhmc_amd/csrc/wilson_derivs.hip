@@ -119,15 +119,23 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
   const unsigned lx = L.d.lx, ly = L.d.ly, lt = L.d.lt, ls = L.d.ls;
   const unsigned v2 = lx * ly, v3 = v2 * ls, v4 = v2 * lt, v5 = v4 * ls;
   const unsigned nl = BLK / wseg, nb2 = (v2 + nl - 1) / nl;  // lines per block, blocks per t
-  const unsigned nbl = nb2 * lt;  // field blocks; one more carries the scalar step
-  const unsigned t = blockIdx.x / nb2, lb = blockIdx.x - t * nb2;
-  const unsigned line = threadIdx.x / wseg, s = threadIdx.x - line * wseg;
-  const unsigned col = lb * nl + line;  // 2-D site x + lx y
-  const bool valid = s < ls && col < v2 && t < lt;
-  const unsigned lane0 = (threadIdx.x & 63) - s;
-  const long off = (long)rhs * 4 * v5;
   constexpr bool HREC = MODE == EPI_HREC || MODE == EPI_HPREC;
   constexpr bool SUM = MODE == EPI_CG || HREC;
+  // the launch's field blocks, after those of a scalar step
+  const unsigned lead = SUM && L.scal ? SCAL_LEAD : 0;
+  if constexpr (SUM) {
+    if (blockIdx.x < lead) {
+      scalar_block(L);
+      return;
+    }
+  }
+  const unsigned bid = blockIdx.x - lead, nbl = nb2 * lt;
+  const unsigned t = bid / nb2, lb = bid - t * nb2;
+  const unsigned line = threadIdx.x / wseg, s = threadIdx.x - line * wseg;
+  const unsigned col = lb * nl + line;  // 2-D site x + lx y
+  const bool valid = s < ls && col < v2;
+  const unsigned lane0 = (threadIdx.x & 63) - s;
+  const long off = (long)rhs * 4 * v5;
   const bool fsum = SUM && L.fsum;
   const unsigned i = s + ls * col + v3 * t;
   Site<P64> c{}, f[3]{}, b[3]{}, old{}, pold{};  // old: the epilogue's h or r
@@ -183,10 +191,6 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
         if ((int)threadIdx.x + k * BLK < L.fsum_n) v += part[k];
       for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += L.fsum[k];
       v = block_sum_once<BLK, 1>(v);
-      if (blockIdx.x == nbl) {
-        scalar_step(L.scal, L.sst, L.sslot, v);
-        return;
-      }
       sc = MODE == EPI_CG ? sc / v : v / sc;  // alpha = delta / |h|^2, gamma = lambda / delta
     }
   }
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
   }
   if constexpr (MODE != EPI_STORE) {
     const double tot = block_sum_once<BLK, 2>(red);
-    if (threadIdx.x == 0) L.partial[(long)rhs * nbl + blockIdx.x] = tot;
+    if (threadIdx.x == 0) L.partial[(long)rhs * nbl + bid] = tot;
   }
 }
 
@@ -908,7 +912,7 @@ int launch_wilson_epi(DslashLaunch L, hipStream_t s) {
   THR_CHECK(!L.scal == !L.fsum && (!L.scal || (L.nrhs == 1 && L.sst)), THR_ERR_ARG,
             "Wilson kernel: a fused sum comes with its scalar step");
   THR_CHECK(L.mode != EPI_HPREC || (!L.dagger && L.x), THR_ERR_ARG, "direction epilogue: M with its vector");
-  const dim3 grid((unsigned)wilson_blocks(L.d) + (L.scal ? 1u : 0u), (unsigned)L.nrhs);
+  const dim3 grid((unsigned)wilson_blocks(L.d) + (L.scal ? SCAL_LEAD : 0u), (unsigned)L.nrhs);
   const unsigned seg = segment(L.d.ls);
 #define THR_GO(D, M) hipLaunchKernelGGL((k_wilson<D, M>), grid, dim3(BLK), 0, s, L, seg, w)
 #define THR_DAG(M)         \
