@@ -1368,7 +1368,12 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
                    (TL.mode != TILE_BOXES || TL.bx % 8 == 0);
   const bool xl4 = ul4 && c.lds_x && L.d.lx % 16 == 0 &&
                    (TL.mode != TILE_BOXES || TL.bx % 16 == 0);
-  const bool nt = c.nt_stores != 0;
+  // r of a single FP64 solve is what the next pass reads 7 sites of at each
+  // site, so it is stored to stay in cache (multishift at 16^3 x 48 8.03 ms
+  // against 8.31, 24^3 x 40 27.3 against 28.6, 24^3 x 60 43.6 against 44.5);
+  // batches pass more through the caches than they hold (a mixed solve of 8
+  // sources on 24^3 x 32 135.6 ms, without non-temporal stores 142.6)
+  const bool nt = c.nt_stores != 0 && !(L.mode == EPI_CG && L.prec == P64 && L.nrhs == 1);
   THR_CHECK(!TL.yl || xl, THR_ERR_STATE, "y exchange without the x exchange");
   THR_CHECK(4 * L.d.v5() * Store<P64>::bytes < (1L << 32), THR_ERR_SIZE,
             "spinor too large for 32-bit buffer offsets");
