@@ -111,6 +111,21 @@ __device__ inline cx<float> ldc(const float2 *p, long i) {
 }
 __device__ inline void st(double2 *p, long i, cx<double> v) { p[i] = make_double2(v.r, v.i); }
 __device__ inline void st(float2 *p, long i, cx<float> v) { p[i] = make_float2(v.r, v.i); }
+// non-temporal: data that is not read again before the caches have turned over
+typedef __attribute__((ext_vector_type(2))) double V2d;
+typedef __attribute__((ext_vector_type(2))) float V2f;
+__device__ inline cx<double> ldc_nt(const double2 *p, long i) {
+  const V2d v = __builtin_nontemporal_load((const V2d *)p + i);
+  return {v.x, v.y};
+}
+__device__ inline cx<float> ldc_nt(const float2 *p, long i) {
+  const V2f v = __builtin_nontemporal_load((const V2f *)p + i);
+  return {v.x, v.y};
+}
+__device__ inline void st_nt(double2 *p, long i, cx<double> c) {
+  const V2d v = {c.r, c.i};
+  __builtin_nontemporal_store(v, (V2d *)p + i);
+}
 
 __device__ inline cx<float> ldh(const __half2 *p, long i, float scale) {
   float2 f = __half22float2(p[i]);

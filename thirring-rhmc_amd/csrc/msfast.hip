@@ -43,7 +43,8 @@ template <int P> using CC = typename Store<P>::C;
 
 __device__ inline double fin_sum(const double *partial, int n) { return partial_sum(partial, n); }
 
-// one element of a source's field: FP64 stores spin planes (element
+// one element of a source's field, loaded non-temporally (the flush is the
+// last reader of a block's residuals): FP64 stores spin planes (element
 // e = spin * V5 + site), FP32 and FP16 the spins of a site together
 // ([site][spin], FP16 with a per-site scale)
 template <int P> struct VAcc {
@@ -56,9 +57,9 @@ template <int P> struct VAcc {
       const float sc = nrm[site];
       return {f.x * sc, f.y * sc};
     } else if constexpr (P == P32) {
-      return ldc(p, 4 * site + spin);
+      return ldc_nt(p, 4 * site + spin);
     } else {
-      return ldc(p, e);
+      return ldc_nt(p, e);
     }
   }
 };
@@ -104,14 +105,21 @@ __global__ __launch_bounds__(BLK) void k_msf_init(MsfState *st, int n, const dou
 // aden holds MAXSHIFT shifts per source.  Thread i updates shift i; every
 // shift's arithmetic is the serial recurrence's, so results do not depend on
 // the thread count.  Returns false (and stops the source) on a non-finite
-// omega.  Block-uniform: every thread of the block calls it.
-__device__ bool fin1_step(MsfState *S, const double *aden, double al) {
-  const double os = S->omega, gg = S->gammag;
-  const double om = -S->delta / al;
+// omega, and false for a source that has stopped.  Block-uniform: every thread
+// of the block calls it.  sum: alpha, called after the state's loads are
+// issued: one wait for both.
+template <class F> __device__ bool fin1_step(MsfState *S, const double *aden, F sum) {
+  const int i = threadIdx.x, ic = min(i, MAXSHIFT - 1), stop = S->stop, mini = S->mini,
+            maxi = S->maxi, cgr = S->cg_return, act = S->active[ic];
+  const double os = S->omega, gg = S->gammag, delta = S->delta;
+  const double z1 = S->zeta_i[ic], z2 = S->zeta_ii[ic], ad = aden[ic];
+  asm volatile("" ::: "memory");
+  if (stop) return false;
+  const double al = sum(), om = -delta / al;
+  __syncthreads();  // every thread has read the state before it changes
   if (!isfinite(om)) {
     // a non-finite alpha can never converge: stop this source before any of
     // its vectors is updated (its later launches exit on the stop flag)
-    __syncthreads();
     if (threadIdx.x == 0) {
       S->nonfinite = 1;
       S->stop = 1;
@@ -119,16 +127,13 @@ __device__ bool fin1_step(MsfState *S, const double *aden, double al) {
     __syncthreads();
     return false;
   }
-  const int i = threadIdx.x;
-  if (i >= S->mini - 1 && i < S->maxi && S->active[i]) {
-    S->zeta_iii[i] = (S->zeta_i[i] * S->zeta_ii[i] * os) /
-                     (om * gg * (S->zeta_i[i] - S->zeta_ii[i]) +
-                      S->zeta_i[i] * os * (1.0 - aden[i] * om));
-    S->omegas[i] = om * S->zeta_iii[i] / S->zeta_ii[i];
+  if (i >= mini - 1 && i < maxi && act) {
+    const double z3 = (z1 * z2 * os) / (om * gg * (z1 - z2) + z1 * os * (1.0 - ad * om));
+    S->zeta_iii[i] = z3;
+    S->omegas[i] = om * z3 / z2;
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
-    S->cg_return += 1;
+    S->cg_return = cgr + 1;
     S->alpha = al;
     S->omega_save = os;
     S->omega = om;
@@ -140,11 +145,34 @@ __device__ bool fin1_step(MsfState *S, const double *aden, double al) {
 
 // lambda, gamma, gamma_i; block coefficients; convergence (136-176, 230-275).
 // Returns false once the source stops (non-finite lambda, every shift
-// converged, or maxcg).  Block-uniform.
-__device__ bool fin2_step(MsfState *S, double L) {
-  __shared__ int s_nmax, s_nmin;
+// converged, or maxcg) and for one that has stopped.  Block-uniform.  sum:
+// lambda, as above.  A shift's row of coefficients is one wave wide (MSB), so
+// a wave takes every fourth row and has NR of them in registers before the sum
+// is there: 24^3 x 32 with 8 sources and 12 shifts 4.6 us a launch, 6.7 when
+// shift i's thread walked its row after the sum.
+static_assert(MSB == 64 && MAXSHIFT <= 64, "a wave spans a row and every shift");
+template <class F> __device__ bool fin2_step(MsfState *S, F sum) {
+  __shared__ int s_nmax, s_nmin, s_mine[MAXSHIFT];
+  __shared__ double s_om[MAXSHIFT], s_gi[MAXSHIFT];
+  constexpr int NW = BLK / 64, NR = 4;
+  const int i = threadIdx.x, ic = min(i, MAXSHIFT - 1), w = i >> 6, q = i & 63;
+  const int stop = S->stop, n = S->n, mini = S->mini, maxi = S->maxi, j = S->jcount,
+            cgr = S->cg_return, maxcg = S->maxcg, act = S->active[ic];
+  const double delta = S->delta, omega = S->omega, tol2 = S->tol2;
+  const double z2 = S->zeta_ii[ic], zt = S->zeta_iii[ic], om = S->omegas[ic], ca = S->ca[ic],
+               cc = S->cc[ic];
+  double cbr[NR], cdr[NR];
+#pragma unroll
+  for (int u = 0; u < NR; u++) {
+    const int r = min(w + NW * u, MAXSHIFT - 1);
+    cbr[u] = S->cb[r][q];
+    cdr[u] = S->cd[r][q];
+  }
+  asm volatile("" ::: "memory");
+  if (stop) return false;
+  const double L = sum();
+  __syncthreads();  // every thread has read the state before it changes
   if (!isfinite(L)) {
-    __syncthreads();
     if (threadIdx.x == 0) {
       S->nonfinite = 1;
       S->stop = 1;
@@ -152,61 +180,52 @@ __device__ bool fin2_step(MsfState *S, double L) {
     __syncthreads();
     return false;
   }
-  if (threadIdx.x == 0) {
-    s_nmax = 0;
-    s_nmin = S->n + 1;
-  }
-  __syncthreads();
-  const double gam = L / S->delta;
-  const double omega = S->omega, tol2 = S->tol2;
-  const int j = S->jcount, cgr = S->cg_return;
-  const int i = threadIdx.x;
-  const bool mine = i >= S->mini - 1 && i < S->maxi && S->active[i];
-  __syncthreads();  // every thread has read the scalars before thread 0 writes them
-  if (mine) {
-    const double zt = S->zeta_iii[i], om = S->omegas[i];
-    const double gi = gam * zt * om / (S->zeta_ii[i] * omega);
-    S->gammas[i] = gi;
-    // x_i -= omega_i p_i  with p_i = ca P + sum cb R ; then
-    // p_i = gamma_i p_i + zeta_i''' R_j.  The rows go in chunks of 16 slots:
-    // static indices keep a chunk in registers and make its loads independent
-    S->cc[i] -= om * S->ca[i];
-    S->ca[i] *= gi;
-    for (int q0 = 0; q0 < j; q0 += 16) {
-      double cbr[16], cdr[16];
-#pragma unroll
-      for (int u = 0; u < 16; u++) {
-        cbr[u] = S->cb[i][q0 + u];
-        cdr[u] = S->cd[i][q0 + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; u++) {
-        if (q0 + u < j) {
-          S->cd[i][q0 + u] = cdr[u] - om * cbr[u];
-          S->cb[i][q0 + u] = cbr[u] * gi;
-        }
+  const double gam = L / delta;
+  if (i < 64) {  // wave 0: the ballot spans every shift
+    const bool mine = i >= mini - 1 && i < maxi && act;
+    bool on = false;
+    if (mine) {
+      const double gi = gam * zt * om / (z2 * omega);
+      S->gammas[i] = gi;
+      // x_i -= omega_i p_i  with p_i = ca P + sum cb R ; then
+      // p_i = gamma_i p_i + zeta_i''' R_j
+      S->cc[i] = cc - om * ca;
+      S->ca[i] = ca * gi;
+      S->cb[i][j] = zt;
+      S->cd[i][j] = 0.0;
+      S->touched[i] = 1;
+      S->cg_returns[i] = cgr;
+      s_om[i] = om;
+      s_gi[i] = gi;
+      // shifted residual of the new iterate: |zeta'''| |r_new|
+      on = !(zt * zt * L <= tol2);
+      if (on) {  // the window only shrinks: a shift that stays was in it
+        S->zeta_i[i] = z2;
+        S->zeta_ii[i] = zt;
+      } else {
+        S->active[i] = 0;
       }
     }
-    S->cb[i][j] = zt;
-    S->cd[i][j] = 0.0;
-    S->touched[i] = 1;
-    S->cg_returns[i] = cgr;
-    // shifted residual of the new iterate: |zeta'''| |r_new|
-    if (zt * zt * L <= tol2) {
-      S->active[i] = 0;
-    } else {
-      atomicMax(&s_nmax, i + 1);
-      atomicMin(&s_nmin, i + 1);
+    if (i < MAXSHIFT) s_mine[i] = mine;
+    const unsigned long long live = __ballot(on);
+    if (i == 0) {
+      s_nmax = live ? 64 - __clzll(live) : 0;
+      s_nmin = live ? __ffsll((long long)live) : n + 1;
     }
   }
   __syncthreads();
   const int nmax = s_nmax, nmin = s_nmin;
-  if (i >= nmin - 1 && i < nmax && S->active[i]) {
-    S->zeta_i[i] = S->zeta_ii[i];
-    S->zeta_ii[i] = S->zeta_iii[i];
-  }
-  __syncthreads();
-  const bool go = !(nmax == 0 || cgr >= S->maxcg);
+  const auto row = [&](int r, double b, double d) {
+    if (q < j && s_mine[r]) {
+      S->cd[r][q] = d - s_om[r] * b;
+      S->cb[r][q] = b * s_gi[r];
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < NR; u++)
+    if (w + NW * u < n) row(w + NW * u, cbr[u], cdr[u]);
+  for (int r = w + NW * NR; r < n; r += NW) row(r, S->cb[r][q], S->cd[r][q]);
+  const bool go = !(nmax == 0 || cgr >= maxcg);
   if (threadIdx.x == 0) {
     S->lambda = L;
     S->gammag = gam;
@@ -222,24 +241,13 @@ __device__ bool fin2_step(MsfState *S, double L) {
 
 __global__ __launch_bounds__(BLK) void k_msf_fin1(MsfState *st, const double *adens,
                                                   const double *partial, int stride, int nb) {
-  MsfState *S = st + blockIdx.x;
-  if (S->stop) return;
-  __shared__ double s_al;
-  const double al = fin_sum(partial + (long)blockIdx.x * stride, nb);
-  if (threadIdx.x == 0) s_al = al;
-  __syncthreads();
-  fin1_step(S, adens + (long)blockIdx.x * MAXSHIFT, s_al);
+  fin1_step(st + blockIdx.x, adens + (long)blockIdx.x * MAXSHIFT,
+            [&] { return fin_sum(partial + (long)blockIdx.x * stride, nb); });
 }
 
 __global__ __launch_bounds__(BLK) void k_msf_fin2(MsfState *st, const double *partial, int stride,
                                                   int nb) {
-  MsfState *S = st + blockIdx.x;
-  if (S->stop) return;
-  __shared__ double s_lam;
-  const double lam = fin_sum(partial + (long)blockIdx.x * stride, nb);
-  if (threadIdx.x == 0) s_lam = lam;
-  __syncthreads();
-  fin2_step(S, s_lam);
+  fin2_step(st + blockIdx.x, [&] { return fin_sum(partial + (long)blockIdx.x * stride, nb); });
 }
 
 // The recurrences of a block's iterations replayed from the scalars the
@@ -259,8 +267,9 @@ __global__ __launch_bounds__(BLK) void k_msf_fin_block(MsfState *st, const doubl
   __syncthreads();
   const double *aden = adens + (long)blockIdx.x * MAXSHIFT;
   for (int j = 0; j < nit; j++) {
-    if (!fin1_step(S, aden, S->al_rec[j])) return;
-    if (!fin2_step(S, j + 1 < nit ? S->lam_rec[j] : s_last)) return;
+    const double al = S->al_rec[j], lam = j + 1 < nit ? S->lam_rec[j] : s_last;
+    if (!fin1_step(S, aden, [&] { return al; })) return;
+    if (!fin2_step(S, [&] { return lam; })) return;
   }
 }
 
@@ -274,7 +283,9 @@ __device__ inline cx<double> widen(cx<float> v) {
 }
 
 // apply the block's coefficients of ring slots [q0, q0 + QN) to x_i and p_i
-// (FP64), reading each residual once.  A 64-iteration block takes one launch
+// (FP64), reading each residual once, all of it non-temporal and with the next
+// shift's x_i, p_i loaded ahead (24^3 x 32, 8 sources, 12 shifts, 64 FP32 slots:
+// 15.4 GB in 2.89 ms, 5.3 TB/s; 3.19 ms through the caches).  A 64-iteration block takes one launch
 // with FP32/FP16 residuals (held as such, widened per use) and two with FP64
 // ones (q0 = 0, 32: the second adds its slots to the x_i, p_i the first
 // wrote).
@@ -339,7 +350,9 @@ __global__ __launch_bounds__(BLK) void k_msf_flush(long v5, int n, TT<P> *const 
       uint4 raw = make_uint4(0u, 0u, 0u, 0u);
       float sk = 0.0f;
       if (qb + spin < jc) {
-        raw = *(const uint4 *)(pk + off + 4 * site);
+        typedef __attribute__((ext_vector_type(4))) unsigned V4u;
+        const V4u v = __builtin_nontemporal_load((const V4u *)(pk + off + 4 * site));
+        raw = make_uint4(v.x, v.y, v.z, v.w);
         sk = nk[so];
       }
       __builtin_amdgcn_wave_barrier();
@@ -373,18 +386,27 @@ __global__ __launch_bounds__(BLK) void k_msf_flush(long v5, int n, TT<P> *const 
   const bool head = q0 == 0;
   const int first = S->first_block;
   const cx<double> bv = head && first ? ldc(b, off + e) : cx<double>{0.0, 0.0};
+  // the next shift's x and p are loaded before this one's are worked on
+  cx<double> xn{0.0, 0.0}, pn = bv;
+  const auto fetch = [&](int i) {
+    if (i < n && stouch[i] && !(head && first)) {
+      const long xo = ((long)src * n + i) * ns + e;
+      xn = ldc_nt(X, xo);
+      if (head || sact[i]) pn = ldc_nt(Pv, xo);
+    }
+  };
+  fetch(0);
   for (int i = 0; i < n; i++) {
+    const cx<double> base = pn;
+    cx<double> xs = xn, ps = {0.0, 0.0};
+    fetch(i + 1);
     if (!stouch[i]) continue;
     const long xo = ((long)src * n + i) * ns + e;
-    cx<double> xs, ps = {0.0, 0.0};
     if (head) {
-      const cx<double> base = first ? bv : ldc(Pv, xo);
-      xs = first ? cx<double>{0.0, 0.0} : ldc(X, xo);
       xs = xs + sc[i] * base;
       if (sact[i]) ps = sa[i] * base;
-    } else {
-      xs = ldc(X, xo);
-      if (sact[i]) ps = ldc(Pv, xo);
+    } else if (sact[i]) {
+      ps = base;
     }
     if (sact[i]) {
 #pragma unroll
@@ -394,13 +416,13 @@ __global__ __launch_bounds__(BLK) void k_msf_flush(long v5, int n, TT<P> *const 
           xs = xs + sd[i][q] * r;
           ps = ps + sb[i][q] * r;
         }
-      st(X, xo, xs);
-      st(Pv, xo, ps);
+      st_nt(X, xo, xs);
+      st_nt(Pv, xo, ps);
     } else {
 #pragma unroll
       for (int q = 0; q < QN; q++)
         if (q0 + q < jc) xs = xs + sd[i][q] * widen(R[q]);
-      st(X, xo, xs);
+      st_nt(X, xo, xs);
     }
   }
 }

@@ -359,17 +359,6 @@ __global__ __launch_bounds__(BLK) void k_ms_coef(MsState *st, const double *part
   }
 }
 
-// loads and stores past the caches' reuse order (k_ms_flush)
-typedef __attribute__((ext_vector_type(2))) double V2d;
-__device__ inline cx<double> ldc_nt(const double2 *p, long i) {
-  const V2d v = __builtin_nontemporal_load((const V2d *)p + i);
-  return {v.x, v.y};
-}
-__device__ inline void st_nt(double2 *p, long i, cx<double> c) {
-  const V2d v = {c.r, c.i};
-  __builtin_nontemporal_store(v, (V2d *)p + i);
-}
-
 // x_i, p_i of every shift that the block updated, from its residuals R_0 ..
 // R_{c-1}: ring slot q of residual j = t0 + q.  Bound by memory: one read of
 // each residual and, per shift, p and x read and written (c + 4 k field
