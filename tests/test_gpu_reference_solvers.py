@@ -215,3 +215,33 @@ def test_derivs_batch_splits(G, dims, npair):
         G.derivs_dev(rs[k], xs[k], an[k], fl[k], dims, one)
     G.derivs_batch_dev(rs, xs, an, fl, dims, all_)
     assert rel(all_.to_host(), one.to_host()) <= 1e-13
+
+
+# one site per thread (a remainder, one shift), the t march on whole lines
+# (2^18 sites in a batch) and off them (more than 2^20)
+@pytest.mark.parametrize("dims,nsrc,n", [((3, 5, 4, 12), 3, 1), ((5, 3, 7, 32), 2, 3),
+                                         ((16, 16, 16, 32), 2, 2), ((13, 5, 22, 64), 3, 1),
+                                         ((17, 16, 21, 47), 4, 1)])
+def test_true_residuals_of_any_x(G, nsrc, n, dims):
+    """|b - (M^+M + sigma_i) x_i| / |b| of random b and x against the oracle's
+    operator: no cancellation, sums of positive terms, so rounding only (1e-13
+    as the operator's own tolerance)."""
+    from hiprt import DeviceArray
+    rng, u = smooth(dims, 40)
+    v5 = int(np.prod(dims))
+    am = np.array([0.05, 0.3, 0.01, 0.1][:nsrc], dtype=np.float32)
+    sig = np.array([0.02, 1.5, 0.3][:n])
+    c = rng.standard_normal((nsrc, n + 1, 4 * v5, 2))
+    print("case: true residuals", dims, nsrc, n, flush=True)
+    lin = u[1:-1, 1:-1, 1:-1, :].reshape(-1, order="F")
+    l64 = DeviceArray.from_host(np.stack([lin.real, lin.imag], axis=-1))
+    got = G.true_residuals_dev(l64, dims, am, 3, sig,
+                               DeviceArray.from_host(np.ascontiguousarray(c[:, 0])),
+                               DeviceArray.from_host(np.ascontiguousarray(c[:, 1:])), nsrc=nsrc)
+    z = c[..., 0] + 1j * c[..., 1]
+    for k in range(nsrc):
+        for i in range(n):
+            a = O.dirac_op_shifted(D.from_vec(z[k, 1 + i], dims), u, dims, float(am[k]), 3,
+                                   shift=sig[i])
+            want = np.linalg.norm(z[k, 0] - D.interior_vec(a)) / np.linalg.norm(z[k, 0])
+            assert abs(got[k, i] - want) <= 1e-13 * want

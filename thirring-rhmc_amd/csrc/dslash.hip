@@ -454,6 +454,22 @@ template <int NW> struct XBuf<P16, NW> {
   }
 };
 
+// EPI_TRES at one site: |w - o - sigma x|^2.  Replaces a pass over four fields
+// behind an M^+ that stored its result (24^3 x 32, 8 sources: 105 + 119 us a
+// shift, 140 us this way).
+__device__ inline double true_res(const DslashLaunch &L, unsigned rhs, unsigned i, unsigned v5,
+                                  const cx<double> o[4]) {
+  const Acc<P64> wa{(const double2 *)L.w + (long)rhs * 4 * v5, nullptr, v5};
+  const Acc<P64> xa{(const double2 *)L.x + (long)rhs * L.x_stride, nullptr, v5};
+  cx<double> wv[4], xv[4];
+  wa.load4(i, wv);
+  xa.load4(i, xv);
+  double red = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) red += norm2(wv[k] - o[k] - L.sigma * xv[k]);
+  return red;
+}
+
 // One thread owns the s-x-y site (s fastest) of one t-chunk and marches
 // through it: R(t+1) loaded at step t is the centre at t+1 and the backward
 // t neighbour at t+2, so the t hops come from registers.  x and y hops are
@@ -569,7 +585,8 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
     using Lk = std::conditional_t<UL == 1, SLinks<C>,
                                   std::conditional_t<(UL > 1), SLinksN<C, (UL > 1 ? UL : 2)>,
                                                      BLinks<C>>>;
-    const In in((const T *)L.in + roff, L.in_norm ? L.in_norm + (long)rhs * v5 : nullptr, v5);
+    const long ioff = L.in_stride ? (long)rhs * L.in_stride : roff;
+    const In in((const T *)L.in + ioff, L.in_norm ? L.in_norm + (long)rhs * v5 : nullptr, v5);
     const Lk lk(L.links, 3 * v4);
     const C diag = L.wilson4d ? (C)(3.0f + (-L.am3)) : (C)((3.0f - L.am3) + 1.0f);
     const int up0 = DAG ? 0 : 2, dn0 = DAG ? 2 : 0;
@@ -774,6 +791,8 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
           Out<PREC> xo{(T *)L.x + roff, nullptr, v5};
           xo.store4(i, xv);
         }
+      } else if constexpr (MODE == EPI_TRES) {
+        red += true_res(L, rhs, i, v5, o);
       } else {
         const BOut<PREC, NT> out((T *)L.out + roff, L.out_norm ? L.out_norm + (long)rhs * v5 : nullptr,
                                  v5);
@@ -930,7 +949,8 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
   const unsigned tf = (t + 1 == lt) ? 0 : t + 1, tb = (t == 0) ? lt - 1 : t - 1;
   const unsigned col = ls * xy + v3 * t, i = s + col;
   const long roff = (long)rhs * 4 * v5;
-  const BAcc<PREC> in((const T *)L.in + roff, L.in_norm ? L.in_norm + (long)rhs * v5 : nullptr, v5);
+  const long ioff = L.in_stride ? (long)rhs * L.in_stride : roff;
+  const BAcc<PREC> in((const T *)L.in + ioff, L.in_norm ? L.in_norm + (long)rhs * v5 : nullptr, v5);
   const BLinks<C> lk(L.links, 3 * v4);
   constexpr int up0 = DAG ? 0 : 2, dn0 = DAG ? 2 : 0;
   const Site<PREC> cur = load_site(in, i);
@@ -1079,6 +1099,8 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
         xout.store4(is, xv);
       }
     }
+  } else if constexpr (MODE == EPI_TRES) {
+    red = true_res(L, rhs, i, v5, o);
   } else {
     if constexpr (HREC) {
 #pragma unroll
@@ -1345,6 +1367,8 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
             "recurrence epilogue needs its scalar (and fp16 scales)");
   THR_CHECK(L.mode != EPI_HPREC || (L.prec == P64 && !L.dagger && L.x), THR_ERR_ARG,
             "direction epilogue: FP64, with its vector");
+  THR_CHECK(L.mode != EPI_TRES || (L.prec == P64 && L.dagger && L.w && L.x && L.x_stride),
+            THR_ERR_ARG, "true-residual epilogue: FP64 M^+, with its fields");
   THR_CHECK(!L.scal || (c.site && L.prec == P64 && L.nrhs == 1 && L.fsum && L.sst), THR_ERR_ARG,
             "scalar step on a launch that cannot carry it");
   THR_CHECK(4 * L.d.v5() < (1L << 31), THR_ERR_SIZE, "lattice too large for 32-bit indexing");
@@ -1392,6 +1416,7 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
     case EPI_DOTW: THR_SITE(P, D, EPI_DOTW); break;          \
     case EPI_HREC: THR_SITE(P, D, EPI_HREC); break;          \
     case EPI_HPREC: THR_SITE(P64, false, EPI_HPREC); break;  \
+    case EPI_TRES: THR_SITE(P64, true, EPI_TRES); break;     \
     default: THR_SITE(P, D, EPI_CG); break;                  \
   }
 #define THR_SITE2(P) \
@@ -1447,6 +1472,7 @@ int launch_dslash_cfg(const DslashLaunch &L, DslashConfig c, hipStream_t s) {
     case EPI_DOTW: THR_LAUNCH(P, D, S, EPI_DOTW); break;   \
     case EPI_HREC: THR_LAUNCH(P, D, S, EPI_HREC); break;   \
     case EPI_HPREC: THR_LAUNCH(P64, false, S, EPI_HPREC); break; \
+    case EPI_TRES: THR_LAUNCH(P64, true, S, EPI_TRES); break; \
     default: THR_LAUNCH(P, D, S, EPI_CG); break;           \
   }
 #define THR_LAUNCH2(P, D) \

@@ -15,6 +15,8 @@ enum EpiMode {
   EPI_HREC = 4,      // out = M r + b*out (in place) ; partial += |out|^2  (h = M p by recurrence)
   EPI_HPREC = 5,     // EPI_HREC and x = r + b*x (the direction p itself); b is 0, and the old x
                      // not used, where b_ptr is null (FP64)
+  EPI_TRES = 6,      // partial += |w - M^+ in - sigma x|^2, nothing stored (FP64, M^+): the true
+                     // residual of a shift, in = M x
 };
 
 // scalar step carried by a launch (krylov_scalars.h)
@@ -30,13 +32,16 @@ struct DslashLaunch {
   float am3;
   float am[MAXRHS];  // per right-hand side (float32, as the reference's `real :: am`)
   const void *in;
+  long in_stride;  // elements between the right-hand sides of in (0: a field, 4 V5)
   const float *in_norm;
   void *out;
   float *out_norm;
   const void *links;  // double2 for P64, float2 otherwise
   // epilogue
   int mode;
-  const void *w;       // EPI_DOTW
+  const void *w;       // EPI_DOTW, EPI_TRES
+  double sigma;        // EPI_TRES
+  long x_stride;       // EPI_TRES: elements between the right-hand sides of x
   void *r, *x;         // EPI_CG: r read (and written unless r_out is set)
   const void *p;       // EPI_CG
   void *r_out;         // EPI_CG: optional separate destination of the updated r

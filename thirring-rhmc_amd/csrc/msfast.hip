@@ -444,25 +444,6 @@ __global__ void k_msf_reset(MsfState *st) {
   }
 }
 
-// partial |b - (M^+M + sigma) x|^2 per source: t holds M^+M x
-__global__ __launch_bounds__(BLK) void k_true_res(long v5, const double2 *b, const double2 *t,
-                                                  const double2 *x, double sigma, long xstride,
-                                                  double *partial) {
-  const int src = blockIdx.y;
-  const long i = (long)blockIdx.x * BLK + threadIdx.x;
-  double red = 0.0;
-  if (i < v5) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const long e = (long)src * 4 * v5 + k * v5 + i;
-      const cx<double> r = ldc(b, e) - ldc(t, e) - sigma * ldc(x, (long)src * xstride + k * v5 + i);
-      red += norm2(r);
-    }
-  }
-  const double tot = block_sum(red);
-  if (threadIdx.x == 0) partial[(long)src * gridDim.x + blockIdx.x] = tot;
-}
-
 // Reliable update of the base residual (the replacement of the iterated
 // residual by a true one, Sleijpen and van der Vorst): for each source with
 // rel[src] != 0, r' = (b - (M^+M + sigma) x) / zeta from the FP64 true
@@ -1116,18 +1097,15 @@ int msfast_true_residuals(const MsfArgs &A, double *relres, hipStream_t s) {
   const long v5 = d.v5(), nsp = 4 * v5;
   const int nb = (int)dslash_blocks(d);
   double2 *t1 = (double2 *)workspace(370, sizeof(double2) * nsp * ns_);
-  double2 *t2 = (double2 *)workspace(371, sizeof(double2) * nsp * ns_);
   double *partial = (double *)workspace(366, sizeof(double) * nb * ns_);
-  double *sums = (double *)workspace(368, sizeof(double) * ns_);
-  double2 *xs = (double2 *)workspace(372, sizeof(double2) * nsp * ns_);
-  THR_CHECK(t1 && t2 && partial && sums && xs, THR_ERR_HIP, "workspace allocation failed");
-  double *bn = (double *)host_workspace(3, sizeof(double) * ns_);
-  double *hsum = (double *)host_workspace(4, sizeof(double) * ns_);
-  THR_CHECK(bn && hsum, THR_ERR_HIP, "host workspace allocation failed");
+  // row 0: |b|^2, row 1 + i: shift i
+  const size_t nsum = (size_t)ns_ * (n + 1);
+  double *sums = (double *)workspace(368, sizeof(double) * nsum);
+  THR_CHECK(t1 && partial && sums, THR_ERR_HIP, "workspace allocation failed");
+  double *hsum = (double *)host_workspace(4, sizeof(double) * nsum);
+  THR_CHECK(hsum, THR_ERR_HIP, "host workspace allocation failed");
   hipLaunchKernelGGL(k_norm_src, dim3(nb, ns_), dim3(BLK), 0, s, v5, A.b, partial);
   hipLaunchKernelGGL(k_sum_rows, dim3(ns_), dim3(BLK), 0, s, partial, nb, sums);
-  THR_HIP(hipMemcpyAsync(bn, sums, sizeof(double) * ns_, hipMemcpyDeviceToHost, s));
-  THR_HIP(hipStreamSynchronize(s));
   DslashLaunch L{};
   L.d = d;
   L.nrhs = ns_;
@@ -1136,30 +1114,35 @@ int msfast_true_residuals(const MsfArgs &A, double *relres, hipStream_t s) {
   L.am3 = A.am3;
   for (int k = 0; k < ns_; k++) L.am[k] = A.am[k];
   L.links = A.u64;
-  L.mode = EPI_STORE;
   L.sc_stride = 1;
   L.done_stride = 1;
   for (int i = 0; i < n; i++) {
-    // gather shift i of every source into one batch
-    for (int k = 0; k < ns_; k++)
-      THR_HIP(hipMemcpyAsync(xs + k * nsp, A.x + ((long)k * n + i) * nsp, sizeof(double2) * nsp,
-                             hipMemcpyDeviceToDevice, s));
+    // shift i of every source: x of source k lies n fields behind that of k - 1
     DslashLaunch a = L;
-    a.in = xs;
+    a.mode = EPI_STORE;
+    a.in = A.x + (long)i * nsp;
+    a.in_stride = n * nsp;
     a.out = t1;
     TRY_RC(launch_dslash(a, s));
     DslashLaunch b = L;
+    b.mode = EPI_TRES;
     b.dagger = 1;
     b.in = t1;
-    b.out = t2;
+    b.w = A.b;
+    b.sigma = A.aden[i];
+    b.x = A.x + (long)i * nsp;
+    b.x_stride = n * nsp;
+    b.partial = partial;
     TRY_RC(launch_dslash(b, s));
-    hipLaunchKernelGGL(k_true_res, dim3(nb, ns_), dim3(BLK), 0, s, v5, A.b, t2, xs, A.aden[i],
-                       nsp, partial);
-    hipLaunchKernelGGL(k_sum_rows, dim3(ns_), dim3(BLK), 0, s, partial, nb, sums);
-    THR_HIP(hipMemcpyAsync(hsum, sums, sizeof(double) * ns_, hipMemcpyDeviceToHost, s));
-    THR_HIP(hipStreamSynchronize(s));
-    for (int k = 0; k < ns_; k++) relres[k * n + i] = std::sqrt(hsum[k] / bn[k]);
+    hipLaunchKernelGGL(k_sum_rows, dim3(ns_), dim3(BLK), 0, s, partial, nb,
+                       sums + (long)(1 + i) * ns_);
+    THR_HIP(hipGetLastError());
   }
+  THR_HIP(hipMemcpyAsync(hsum, sums, sizeof(double) * nsum, hipMemcpyDeviceToHost, s));
+  THR_HIP(hipStreamSynchronize(s));
+  for (int k = 0; k < ns_; k++)
+    for (int i = 0; i < n; i++)
+      relres[k * n + i] = std::sqrt(hsum[(long)(1 + i) * ns_ + k] / hsum[k]);
   return THR_OK;
 }
 

@@ -909,6 +909,7 @@ int launch_wilson_epi(DslashLaunch L, hipStream_t s) {
   // -am | -i am at s = 1 (dirac.F90:274-278, 602-606), -am | +i am at s = Ls
   // (287-291, 615-619)
   const WallCoef w = L.imass == 1 ? WallCoef{-m, 0.0, -m, 0.0} : WallCoef{0.0, -m, 0.0, m};
+  THR_CHECK(L.mode != EPI_TRES && !L.in_stride, THR_ERR_ARG, "Wilson kernel: no such epilogue");
   THR_CHECK(!L.scal == !L.fsum && (!L.scal || (L.nrhs == 1 && L.sst)), THR_ERR_ARG,
             "Wilson kernel: a fused sum comes with its scalar step");
   THR_CHECK(L.mode != EPI_HPREC || (!L.dagger && L.x), THR_ERR_ARG, "direction epilogue: M with its vector");
