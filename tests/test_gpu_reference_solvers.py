@@ -245,3 +245,40 @@ def test_true_residuals_of_any_x(G, nsrc, n, dims):
                                    shift=sig[i])
             want = np.linalg.norm(z[k, 0] - D.interior_vec(a)) / np.linalg.norm(z[k, 0])
             assert abs(got[k, i] - want) <= 1e-13 * want
+
+
+@pytest.mark.parametrize("tc,flags", [(1, 6), (2, 22), (3, 55), (4, 256 | 22)])
+@pytest.mark.parametrize("imass", [1, 3, 5])
+def test_dslash_f16_lines_of_64(G, imass, tc, flags):
+    """The FP16 march with a wave per s-line (scalar links and lane moves, with
+    and without the exchanges along x and y), where the s hops and the wall
+    terms go around the wave: against the oracle to 4e-3, and each end of the
+    line by itself, to 4e-3 of that slice."""
+    from hiprt import DeviceArray
+    dims = (4, 6, 5, 64)
+    rng, u = smooth(dims, 41)
+    v5 = int(np.prod(dims))
+    r = D.rand_spinor(dims, rng)
+    v = D.interior_vec(r)
+    sites = np.stack([v.real, v.imag], -1).reshape(4, v5, 2).transpose(1, 0, 2)
+    scale = np.abs(sites).max(axis=(1, 2)).astype(np.float32)
+    lin = u[1:-1, 1:-1, 1:-1, :].reshape(-1, order="F")
+    l32 = DeviceArray.from_host(np.stack([lin.real, lin.imag], axis=-1).astype(np.float32))
+    q = DeviceArray.from_host(np.ascontiguousarray((sites / scale[:, None, None])
+                                                   .astype(np.float16)))
+    out, on = DeviceArray(sites.shape, np.float16), DeviceArray(scale.shape, np.float32)
+    saved = G.dslash_get_config(dims, "f16")
+    print("case: FP16 lines of 64", imass, tc, flags, flush=True)
+    try:
+        G.dslash_set_config(dims, "f16", tc, flags)
+        for dagger, of in ((False, O.dslash), (True, O.dslashd)):
+            w = D.interior_vec(of(r, u, dims, 0.3, imass))
+            ref = np.stack([w.real, w.imag], -1).reshape(4, v5, 2).transpose(1, 0, 2)
+            G.dslash_dev(out, q, l32, dims, 0.3, imass=imass, dagger=dagger, prec="f16",
+                         in_norm=DeviceArray.from_host(scale), out_norm=on)
+            got = out.to_host().astype(np.float64) * on.to_host()[:, None, None]
+            assert rel(got, ref) <= 4e-3
+            for s in (0, 63):
+                assert rel(got[s::64], ref[s::64]) <= 4e-3
+    finally:
+        G.dslash_set_config(dims, "f16", *saved)

@@ -92,6 +92,17 @@ template <int PREC> struct Acc {
   }
 };
 
+// max |re|, |im| of a site's spins, 0 if all are NaN: four instructions (fmaxf
+// of fabsf takes fourteen, each operand through one that only quiets NaNs;
+// FP16 M^+ at 32^3 x 64 21.6 -> 21.3 us)
+__device__ inline float max_abs(const cx<float> v[4]) {
+  float m = 0.f;
+#pragma unroll
+  for (int a = 0; a < 4; a++)
+    asm("v_max3_f32 %0, %0, abs(%1), abs(%2)" : "+v"(m) : "v"(v[a].r), "v"(v[a].i));
+  return m;
+}
+
 template <int PREC> struct Out {
   using C = typename Store<PREC>::C;
   using T = typename Store<PREC>::T;
@@ -100,9 +111,7 @@ template <int PREC> struct Out {
   unsigned v5;
   __device__ inline void store4(unsigned site, const cx<C> v[4]) const {
     if constexpr (PREC == P16) {
-      float m = 0.f;
-#pragma unroll
-      for (int a = 0; a < 4; a++) m = fmaxf(m, fmaxf(fabsf(v[a].r), fabsf(v[a].i)));
+      const float m = max_abs(v);
       const float inv = m > 0.f ? 1.0f / m : 0.f;
       nrm[site] = m;
 #pragma unroll
@@ -161,9 +170,7 @@ template <int PREC, bool NT> struct BOut {
             o32 + 16u * h, 0, aux);
       }
     } else {
-      float m = 0.f;
-#pragma unroll
-      for (int a = 0; a < 4; a++) m = fmaxf(m, fmaxf(fabsf(v[a].r), fabsf(v[a].i)));
+      const float m = max_abs(v);
       const float inv = m > 0.f ? 1.0f / m : 0.f;
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m), rn, site * 4u, 0, aux);
       __attribute__((ext_vector_type(4))) unsigned q;
@@ -425,6 +432,10 @@ template <bool NEXT, int PREC> __device__ inline Spin<PREC> shift_spin(const Sit
   else
     return {lane_shift<NEXT>(S.v[a])};
 }
+// the same with the wave as a ring: lane 63's next is lane 0
+template <bool NEXT> __device__ inline unsigned lane_turn(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, NEXT ? 0x134 : 0x13C, 0xF, 0xF, false);
+}
 // one spin of the site held by lane k of the wave
 template <int PREC> __device__ inline Spin<PREC> lane_spin(const Site<PREC> &S, int a, int k) {
   if constexpr (PREC == P16)
@@ -624,6 +635,10 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
         eb = (C)L.b_ptr[(long)rhs * L.sc_stride];
     }
 
+    // FP16 with a wave per s-line: s hops and wall terms by one rule
+    constexpr bool RING = PREC == P16 && UL == 1;
+    const RingSpin rup = ring_spin(s + 1 == ls, shops, imass, (float)m, 1.0f),
+                   rdn = ring_spin(s == 0, shops, imass, (float)m, -1.0f);
     Site<PREC> prv, cur, nxt;
     const unsigned tb0 = (t0 == 0) ? lt - 1 : t0 - 1;
     prv = load_site(in, j + v3 * tb0);
@@ -702,7 +717,15 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
 
       // hops along s (dirac.F90:80-87 for M, 317-324 for M^dagger): spins that
       // hop from s+1 are {3,4} for M and {1,2} for M^dagger; the others from s-1.
-      if constexpr (SHUF) {
+      if constexpr (RING) {
+        const float su = __uint_as_float(lane_turn<true>(__float_as_uint(cur.sc)));
+        const float sd = __uint_as_float(lane_turn<false>(__float_as_uint(cur.sc)));
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          add_ring(o[up0 + k], lane_turn<true>(cur.h[up0 + k]), rup.kr * su, rup.ki * su, rup.sel);
+          add_ring(o[dn0 + k], lane_turn<false>(cur.h[dn0 + k]), rdn.kr * sd, rdn.ki * sd, rdn.sel);
+        }
+      } else if constexpr (SHUF) {
         Spin<PREC> u0 = shift_spin<true>(cur, up0), u1 = shift_spin<true>(cur, up0 + 1);
         Spin<PREC> d0 = shift_spin<false>(cur, dn0), d1 = shift_spin<false>(cur, dn0 + 1);
         if (UL == 0 && 64 % ls != 0) {
@@ -738,7 +761,7 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
       }
       // wall mass (dirac.F90:119-176 for M, 356-402 for M^dagger)
       const unsigned col = i - s;  // s = 0 of this (x,y,t)
-      if (imass == 1 || imass == 3) {
+      if (!RING && (imass == 1 || imass == 3)) {
         // top: s = Ls couples to s = 1 on the up0 spins; bottom: s = 1 couples to s = Ls
         Spin<PREC> w0[2], wL[2];
         if constexpr (UL == 1) {
@@ -1069,18 +1092,28 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
   }
   hop<2, DAG>(o, utf, rtf, utb, rtb);
   if (!L.wilson4d) {
+    if constexpr (PREC == P16) {
+      const RingSpin rup = ring_spin(s + 1 == ls, true, imass, m, 1.0f),
+                     rdn = ring_spin(s == 0, true, imass, m, -1.0f);
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-      // s + 1: the hop, or at s = Ls the wall term from s = 1
-      const cx<C> u = spin_value(su[k]), d = spin_value(sd[k]);
-      if (s + 1 < ls)
-        sub_spin(o[up0 + k], su[k]);
-      else if (imass != 5)
-        o[up0 + k] = o[up0 + k] + (imass == 1 ? m * u : m * muli(u));
-      if (s > 0)
-        sub_spin(o[dn0 + k], sd[k]);
-      else if (imass != 5)
-        o[dn0 + k] = o[dn0 + k] + (imass == 1 ? m * d : (-m) * muli(d));
+      for (int k = 0; k < 2; k++) {
+        add_ring(o[up0 + k], su[k].h, rup.kr * su[k].sc, rup.ki * su[k].sc, rup.sel);
+        add_ring(o[dn0 + k], sd[k].h, rdn.kr * sd[k].sc, rdn.ki * sd[k].sc, rdn.sel);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        // s + 1: the hop, or at s = Ls the wall term from s = 1
+        const cx<C> u = spin_value(su[k]), d = spin_value(sd[k]);
+        if (s + 1 < ls)
+          sub_spin(o[up0 + k], su[k]);
+        else if (imass != 5)
+          o[up0 + k] = o[up0 + k] + (imass == 1 ? m * u : m * muli(u));
+        if (s > 0)
+          sub_spin(o[dn0 + k], sd[k]);
+        else if (imass != 5)
+          o[dn0 + k] = o[dn0 + k] + (imass == 1 ? m * d : (-m) * muli(d));
+      }
     }
     if (imass == 5) {
       const C sg = DAG ? C(-1) : C(1);
