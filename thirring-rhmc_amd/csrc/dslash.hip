@@ -1272,7 +1272,11 @@ bool dslash_env_set() {
 //    18.8); above, Ls = 32 best at 2 on XCD boxes in every precision (within
 //    4% of the best of 45 shapes on 7 batches).  Ls = 64: FP64 8 (batches 4)
 //    on the XCD remap with at most 3 blocks per CU (32^3 x 64: 64.9; without
-//    the cap 70.9), FP32 4 on 4 x 2-line blocks, FP16 2 on the remap.
+//    the cap 70.9); FP32 8 on 4 x 2-line blocks under the same cap (4 without
+//    it: 32^3 x 64 41.0 against 37.3, four right-hand sides 134 and 128, 16^3 x
+//    64 times 8 39.3 and 37.0); FP16 2 on the remap, 8 from four right-hand
+//    sides on (24^3 x 64 times 8 78.9 against 74.6; 32^3 x 64 times 2 46 against
+//    50 that way).
 DslashConfig default_config(const Dims &d, int prec, int nrhs) {
   DslashConfig c;
   const long sites = d.v5() * nrhs;
@@ -1287,8 +1291,11 @@ DslashConfig default_config(const Dims &d, int prec, int nrhs) {
       c.tchunk = nrhs == 1 ? 8 : 4;
       c.occ_cap = 2;
     } else if (prec == P32) {
-      c.tchunk = 4;
+      c.tchunk = 8;
       c.lds_y = 1;
+      c.occ_cap = 2;
+    } else if (nrhs >= 4) {
+      c.tchunk = 8;
     }
   }
   c.tchunk = std::min(c.tchunk, d.lt);
