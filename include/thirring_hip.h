@@ -282,7 +282,9 @@ int thr_dslash_dev(void *out, float *out_norm, const void *in, const float *in_n
  *   THR_SHAPE_LDS_X          with uniform links and Lx % 4, 8, 16 == 0 (Ls =
  *                            64, 32, 16): the inner x neighbours of a block
  *                            come through LDS
- *   THR_SHAPE_NT_STORES      non-temporal output stores
+ *   THR_SHAPE_NT_STORES      non-temporal output stores (never for the
+ *                            residual of a single FP64 solve, which the next
+ *                            pass reads again from cache)
  *   k << THR_SHAPE_OCC_SHIFT occupancy cap, k = 1..3: at most k + 1 resident
  *                            blocks per CU (LDS padding; 0 = no cap)
  *   THR_SHAPE_LDS_Y          with THR_SHAPE_LDS_X at Ls = 64, Lx % 4 == 0 and
@@ -294,7 +296,10 @@ int thr_dslash_dev(void *out, float *out_norm, const void *in, const float *in_n
  * fields with the given links (complex128 for F64, complex64 otherwise) and
  * pins the fastest for the process; thr_dslash_set_config pins a given shape;
  * both apply to every later launch (solvers included) with these dims and
- * precision. */
+ * precision.  Without a pinned shape a launch takes a default by its size; on
+ * small launches that is one site per thread with every load up front, which
+ * the flags do not express: thr_dslash_get_config reports its tiling with
+ * tchunk 1, and pinning that pair selects the march. */
 #define THR_SHAPE_XCD_REMAP 1
 #define THR_SHAPE_UNIFORM_LINKS 2
 #define THR_SHAPE_LANESHIFT 4
