@@ -867,7 +867,7 @@ __global__ __launch_bounds__(YL ? 2 * BLK : BLK) void k_dslash(const DslashLaunc
         if constexpr (MODE == EPI_NORM) {
 #pragma unroll
           for (int k = 0; k < 4; k++) red += (double)norm2(o[k]);
-        } else if constexpr (MODE == EPI_DOTW) {
+        } else if constexpr (MODE == EPI_DOTW && PREC != P16) {  // FP16: refused (no scales of w)
           Acc<PREC> w{(const T *)L.w + roff, nullptr, v5};
           cx<C> wv[4];
           w.load4(i, wv);
@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
     if constexpr (MODE == EPI_NORM || HREC) {
 #pragma unroll
       for (int k = 0; k < 4; k++) red += (double)norm2(o[k]);
-    } else if constexpr (MODE == EPI_DOTW) {
+    } else if constexpr (MODE == EPI_DOTW && PREC != P16) {  // FP16: refused (no scales of w)
       const Acc<PREC> w{(const T *)L.w + roff, nullptr, v5};
       cx<C> wv[4];
       w.load4(i, wv);
