@@ -481,7 +481,7 @@ template <int NW> struct XBuf<P16, NW> {
 
 // EPI_TRES at one site: |w - o - sigma x|^2.  Replaces a pass over four fields
 // behind an M^+ that stored its result (24^3 x 32, 8 sources: 105 + 119 us a
-// shift, 140 us this way).
+// shift, 131 us this way).
 __device__ inline double true_res(const DslashLaunch &L, unsigned rhs, unsigned i, unsigned v5,
                                   const cx<double> o[4]) {
   const Acc<P64> wa{(const double2 *)L.w + (long)rhs * 4 * v5, nullptr, v5};
