@@ -1044,6 +1044,8 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
   asm volatile("" ::: "memory");  // the loads stay above the branch and the barriers
   if (dn) return;
   C ea = C(0), eb = C(0);
+  // a fused alpha that stops the solve (cg_alpha_step) must leave x as it is
+  bool xgo = xup;
   if constexpr (SUM) {
     if (fsum) {
       // the finalize kernels' order of summation (partial_thread, block_sum)
@@ -1058,6 +1060,7 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
       if constexpr (MODE == EPI_CG) {
         const double om = -sc / v;  // omega = -delta / alpha
         sc = -om;
+        xgo = xgo && isfinite(v) && isfinite(sc);
       } else {
         sc = v / sc;  // gamma = lambda / delta
       }
@@ -1143,7 +1146,7 @@ __global__ __launch_bounds__(BLK, site_late(PREC, MODE) ? 3 : 2) void k_dslash_s
     const BOut<PREC, NT> rout(ro, rn ? rn + (long)rhs * v5 : nullptr, v5);
     rout.store4(is, rv);
     if constexpr (PREC != P16) {
-      if (xup) {
+      if (xgo) {
         cx<C> xv[4];
 #pragma unroll
         for (int k = 0; k < 4; k++)

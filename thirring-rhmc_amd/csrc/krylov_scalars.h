@@ -59,7 +59,9 @@ template <class F> __device__ inline void cg_alpha_step(CgState *st, F sum) {
     st->itercg = itercg + 1;
     st->alpha = alphan / alphad;
     // a non-finite |M p|^2 (NaN or Inf in the source, the guess or the links)
-    // can never meet the stopping rule: end the solve here instead of at niterc
+    // can never meet the stopping rule: end the solve here instead of at
+    // niterc, with x as the iteration before left it (the field blocks of a
+    // launch that carries this step test the same two values)
     if (!isfinite(alphad) || !isfinite(alphan / alphad)) {
       st->stop = 3;
       st->iterations = nx + 1;
@@ -118,7 +120,9 @@ template <class F> __device__ inline void ms_alpha_step(MsState *st, F sum) {
     st->minus_omega = -om;
     if (!ok) {
       // nothing downstream of a non-finite omega is meaningful: stop before
-      // any vector of this iteration is updated
+      // any shift is updated.  Field blocks of a launch that carries this step
+      // may still write their part of r, into a ring slot that no flush reads:
+      // the iteration is not counted in jcount.
       st->nonfinite = 1;
       st->stop = 1;
       st->done = 1;

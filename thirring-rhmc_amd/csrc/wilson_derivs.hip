@@ -183,6 +183,8 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
   }
   asm volatile("" ::: "memory");  // the loads stay above the branch and the barriers
   if (done) return;
+  // a fused alpha that stops the solve (cg_alpha_step) must leave x as it is
+  bool xgo = MODE == EPI_CG && L.b_ptr;
   if constexpr (SUM) {
     if (fsum) {  // the order of partial_sum
       double v = 0.0;
@@ -192,6 +194,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
       for (int k = (int)threadIdx.x + NP * BLK; k < L.fsum_n; k += BLK) v += L.fsum[k];
       v = block_sum_once<BLK, 1>(v);
       sc = MODE == EPI_CG ? sc / v : v / sc;  // alpha = delta / |h|^2, gamma = lambda / delta
+      xgo = xgo && isfinite(v) && isfinite(sc);
     }
   }
   const double ea = sc, eb = MODE == EPI_CG ? (fsum ? sc : sb) : first ? 0.0 : sc;
@@ -243,7 +246,7 @@ __global__ __launch_bounds__(BLK, 2) void k_wilson(const DslashLaunch L, unsigne
         const cx<double> rv = old.v[a] - ea * o[a];
         st((double2 *)(L.r_out ? L.r_out : L.r) + off, e, rv);
         red += norm2(rv);
-        if (L.b_ptr) {
+        if (xgo) {
           double2 *xo = (double2 *)L.x + off;
           st(xo, e, ldc(xo, e) + eb * ldc((const double2 *)L.p + off, e));
         }
