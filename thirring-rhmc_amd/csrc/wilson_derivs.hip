@@ -351,37 +351,42 @@ __constant__ int kGin[3][4] = {{3, 2, 1, 0}, {3, 2, 1, 0}, {2, 3, 0, 1}};
 //                     + w2 sum_a Im(g_mu,a (R0_a^* X1_b + R1_a^* X0_b)),  b = gamin(mu, a)
 // with (R0, X0) at x and (R1, X1) at x+mu, w1 = fl32(tzi/2), w2 = +-tzi
 // (derivs_module.F90:131-187).
-template <int MU>
+//
+// Each spin's products are summed in pairs before they join the sum over the
+// spins (in one chain of 16 the error against 64 bits grew by 5%: 2.36e-16 ->
+// 2.48e-16 at 16^3 x 48).  gamval(mu, a) / akappa is one of +-1, +-i (kGamE),
+// and only the part of the product that it turns into an imaginary one counts.
+// FULL forms the whole complex product all the same (the compiler keeps
+// products with a literal 0): twice the FP64 operations, but in the single
+// Shamir force the compiler then needs 128 registers, four waves per SIMD,
+// against 152 and three (16^3 x 48 11.4 and 12.1 us, 24^3 x 32 19.6 and 20.2,
+// 32^3 x 64 73.2 and 74.9).  The batches and the Wilson kernel's force run at
+// three waves either way and take the short form (25 pairs at 16^3 x 48 212 and
+// 215 us with the call, 12 at 24^3 x 32 214 and 218; Wilson force at 15^2 x 21 x
+// 20 9.4 and 9.65).
+template <int MU, bool FULL>
 __device__ inline double derivs_term(const cx<double> R0[4], const cx<double> X0[4],
                                      const cx<double> R1[4], const cx<double> X1[4], double w1,
                                      double w2) {
-  // gamval(mu, a) / akappa is one of +-1, +-i (kGamE): of the complex product
-  // only the part that it turns into an imaginary one is formed.  Written as
-  // full complex products (the compiler keeps products with a literal 0) the
-  // term took twice the FP64 operations: 5 of 160 us of the batched kernel.
   double sw = 0.0, sd = 0.0;
 #pragma unroll
   for (int a = 0; a < 4; a++) {
     const int b = kGamP[MU][a], e = kGamE[MU][a];
-    sw += R0[a].r * X1[a].i;
-    sw -= R0[a].i * X1[a].r;
-    sw -= R1[a].r * X0[a].i;
-    sw += R1[a].i * X0[a].r;
-    double z;
-    if (e < 2) {  // +-1: Im (R0_a^* X1_b + R1_a^* X0_b)
-      z = R0[a].r * X1[b].i;
-      z -= R0[a].i * X1[b].r;
-      z += R1[a].r * X0[b].i;
-      z -= R1[a].i * X0[b].r;
-    } else {      // +-i: Re
-      z = R0[a].r * X1[b].r;
-      z += R0[a].i * X1[b].i;
-      z += R1[a].r * X0[b].r;
-      z += R1[a].i * X0[b].i;
+    if constexpr (FULL) {
+      const cx<double> g{e == 0 ? 0.5 : e == 1 ? -0.5 : 0.0, e == 2 ? 0.5 : e == 3 ? -0.5 : 0.0};
+      sw += cjmul(R0[a], X1[a]).i - cjmul(R1[a], X0[a]).i;
+      sd += cmul(g, cjmul(R0[a], X1[b]) + cjmul(R1[a], X0[b])).i;
+    } else {
+      sw += (R0[a].r * X1[a].i - R0[a].i * X1[a].r) - (R1[a].r * X0[a].i - R1[a].i * X0[a].r);
+      double z;
+      if (e < 2)  // +-1: Im (R0_a^* X1_b + R1_a^* X0_b)
+        z = (R0[a].r * X1[b].i - R0[a].i * X1[b].r) + (R1[a].r * X0[b].i - R1[a].i * X0[b].r);
+      else        // +-i: Re
+        z = (R0[a].r * X1[b].r + R0[a].i * X1[b].i) + (R1[a].r * X0[b].r + R1[a].i * X0[b].i);
+      sd = (e & 1) ? sd - z : sd + z;
     }
-    sd = (e & 1) ? sd - z : sd + z;
   }
-  return w1 * sw + (0.5 * w2) * sd;
+  return w1 * sw + (FULL ? w2 : 0.5 * w2) * sd;
 }
 
 // sum of v over each segment of w lanes (a power of two), valid in all of its
@@ -496,9 +501,9 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg(const Dims d, const doubl
       add_couplings(Xt, s, ls, lane0, wall);
     }
     if (valid) {
-      v[0] = derivs_term<0>(R0, X0, Rx, Xx, w1, w2);
-      v[1] = derivs_term<1>(R0, X0, Ry, Xy, w1, w2);
-      v[2] = derivs_term<2>(R0, X0, Rt, Xt, w1, w2);
+      v[0] = derivs_term<0, WK == 0>(R0, X0, Rx, Xx, w1, w2);
+      v[1] = derivs_term<1, WK == 0>(R0, X0, Ry, Xy, w1, w2);
+      v[2] = derivs_term<2, WK == 0>(R0, X0, Rt, Xt, w1, w2);
 #pragma unroll
       for (int a = 0; a < 4; a++) {
         R0[a] = Rt[a];
@@ -573,9 +578,9 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_seg_batch(const Dims d, const
     ld_spinor(P.x2, v5, jt, Xt);
   }
   if (valid) {
-    v[0] = derivs_term<0>(R0, X0, Rx, Xx, P.w1, P.w2);
-    v[1] = derivs_term<1>(R0, X0, Ry, Xy, P.w1, P.w2);
-    v[2] = derivs_term<2>(R0, X0, Rt, Xt, P.w1, P.w2);
+    v[0] = derivs_term<0, false>(R0, X0, Rx, Xx, P.w1, P.w2);
+    v[1] = derivs_term<1, false>(R0, X0, Ry, Xy, P.w1, P.w2);
+    v[2] = derivs_term<2, false>(R0, X0, Rt, Xt, P.w1, P.w2);
   }
   // every lane of the wave takes part (idle lanes add 0)
 #pragma unroll
@@ -653,9 +658,9 @@ __global__ __launch_bounds__(BLK, 3) void k_derivs_march_batch(const Dims d, con
     __syncthreads();
     if (valid && w < 3) xb.get(w + 1, s, Rx, Xx);
     if (valid) {
-      v[0] = derivs_term<0>(R0, X0, Rx, Xx, P.w1, P.w2);
-      v[1] = derivs_term<1>(R0, X0, Ry, Xy, P.w1, P.w2);
-      v[2] = derivs_term<2>(R0, X0, Rt, Xt, P.w1, P.w2);
+      v[0] = derivs_term<0, false>(R0, X0, Rx, Xx, P.w1, P.w2);
+      v[1] = derivs_term<1, false>(R0, X0, Ry, Xy, P.w1, P.w2);
+      v[2] = derivs_term<2, false>(R0, X0, Rt, Xt, P.w1, P.w2);
 #pragma unroll
       for (int a = 0; a < 4; a++) {
         R0[a] = Rt[a];
@@ -727,13 +732,13 @@ __global__ __launch_bounds__(BLK) void k_derivs_march(const Dims d, const double
       cx<double> R1[4], X1[4], Rt[4], Xt[4];
       ld_spinor(R, v5, jx + v3 * t, R1);
       ld_spinor(X2, v5, jx + v3 * t, X1);
-      terms[pb][0][threadIdx.x] = derivs_term<0>(R0, X0, R1, X1, w1, w2);
+      terms[pb][0][threadIdx.x] = derivs_term<0, true>(R0, X0, R1, X1, w1, w2);
       ld_spinor(R, v5, jy + v3 * t, R1);
       ld_spinor(X2, v5, jy + v3 * t, X1);
-      terms[pb][1][threadIdx.x] = derivs_term<1>(R0, X0, R1, X1, w1, w2);
+      terms[pb][1][threadIdx.x] = derivs_term<1, true>(R0, X0, R1, X1, w1, w2);
       ld_spinor(R, v5, j + v3 * tf, Rt);
       ld_spinor(X2, v5, j + v3 * tf, Xt);
-      terms[pb][2][threadIdx.x] = derivs_term<2>(R0, X0, Rt, Xt, w1, w2);
+      terms[pb][2][threadIdx.x] = derivs_term<2, true>(R0, X0, Rt, Xt, w1, w2);
 #pragma unroll
       for (int a = 0; a < 4; a++) {
         R0[a] = Rt[a];
