@@ -291,15 +291,20 @@ int thr_dslash_dev(void *out, float *out_norm, const void *in, const float *in_n
  *                            Ly % 2 == 0 (per XCD box with boxes): blocks of
  *                            4 x by 2 y s-lines (512 threads), the inner y
  *                            neighbours also through LDS
+ *   THR_SHAPE_ONE_SITE       one site per thread with every load up front
+ *                            instead of the march (the default of small
+ *                            launches): tchunk 1 and exactly this setting of
+ *                            UNIFORM_LINKS, LANESHIFT, LDS_X, LDS_Y and the
+ *                            occupancy cap, which it has no use for; the
+ *                            other flags keep their meaning
  * No counterpart in the reference (a tuning knob of this library).
  * thr_dslash_autotune times the candidates (tchunk 1..16 x flags) on scratch
  * fields with the given links (complex128 for F64, complex64 otherwise) and
  * pins the fastest for the process; thr_dslash_set_config pins a given shape;
  * both apply to every later launch (solvers included) with these dims and
- * precision.  Without a pinned shape a launch takes a default by its size; on
- * small launches that is one site per thread with every load up front, which
- * the flags do not express: thr_dslash_get_config reports its tiling with
- * tchunk 1, and pinning that pair selects the march. */
+ * precision.  Without a pinned shape a launch takes a default by its size,
+ * which thr_dslash_get_config reports: the pair names the same kernel when it
+ * is pinned. */
 #define THR_SHAPE_XCD_REMAP 1
 #define THR_SHAPE_UNIFORM_LINKS 2
 #define THR_SHAPE_LANESHIFT 4
@@ -308,6 +313,7 @@ int thr_dslash_dev(void *out, float *out_norm, const void *in, const float *in_n
 #define THR_SHAPE_NT_STORES 32
 #define THR_SHAPE_OCC_SHIFT 6
 #define THR_SHAPE_LDS_Y 256
+#define THR_SHAPE_ONE_SITE (THR_SHAPE_LDS_X | (3 << THR_SHAPE_OCC_SHIFT))
 int thr_dslash_autotune(const void *links, const int dims[4], int prec, int *tchunk, int *flags,
                         void *stream);
 /* thr_dslash_autotune timing launches over nrhs right-hand sides (1..32), for
@@ -317,6 +323,9 @@ int thr_dslash_autotune(const void *links, const int dims[4], int prec, int *tch
 int thr_dslash_autotune_nrhs(const void *links, const int dims[4], int prec, int nrhs,
                              int *tchunk, int *flags, void *stream);
 int thr_dslash_set_config(const int dims[4], int prec, int tchunk, int flags);
+/* forgets the shapes pinned for dims and prec, of both batch classes; their
+ * launches take the defaults again (dims NULL: of every lattice and precision) */
+int thr_dslash_clear_config(const int dims[4], int prec);
 int thr_dslash_get_config(const int dims[4], int prec, int *tchunk, int *flags);
 /* the shape a launch of nrhs right-hand sides uses: shapes are pinned per
  * batch class (one right-hand side, or several); thr_dslash_autotune_nrhs

@@ -751,11 +751,40 @@ int thr_dslash_dev(void *out, float *out_norm, const void *in, const float *in_n
   return done_if_default(stream, launch_dslash(L, pick(stream)));
 }
 
-static int shape_flags(const DslashConfig &c) {
-  return (c.remap ? THR_SHAPE_XCD_REMAP : 0) | (c.uniform_links ? THR_SHAPE_UNIFORM_LINKS : 0) |
-         (c.laneshift ? THR_SHAPE_LANESHIFT : 0) | (c.box ? THR_SHAPE_XCD_BOXES : 0) |
-         (c.lds_x ? THR_SHAPE_LDS_X : 0) | (c.nt_stores ? THR_SHAPE_NT_STORES : 0) |
+// flags that only the march reads; THR_SHAPE_ONE_SITE is one setting of them
+// that no march is tuned or documented with (LDS_X without UNIFORM_LINKS)
+constexpr int MARCH_FLAGS = THR_SHAPE_UNIFORM_LINKS | THR_SHAPE_LANESHIFT | THR_SHAPE_LDS_X |
+                            (3 << THR_SHAPE_OCC_SHIFT) | THR_SHAPE_LDS_Y;
+
+// the pair that names shape c, and the shape that a pair names
+static void shape_pair(const DslashConfig &c, int *tchunk, int *flags) {
+  int f = (c.remap ? THR_SHAPE_XCD_REMAP : 0) | (c.box ? THR_SHAPE_XCD_BOXES : 0) |
+          (c.nt_stores ? THR_SHAPE_NT_STORES : 0);
+  if (c.site)
+    f |= THR_SHAPE_ONE_SITE;
+  else
+    f |= (c.uniform_links ? THR_SHAPE_UNIFORM_LINKS : 0) |
+         (c.laneshift ? THR_SHAPE_LANESHIFT : 0) | (c.lds_x ? THR_SHAPE_LDS_X : 0) |
          ((c.occ_cap & 3) << THR_SHAPE_OCC_SHIFT) | (c.lds_y ? THR_SHAPE_LDS_Y : 0);
+  if (tchunk) *tchunk = c.site ? 1 : c.tchunk;
+  if (flags) *flags = f;
+}
+static DslashConfig pair_shape(int tchunk, int flags) {
+  DslashConfig c;
+  c.tchunk = tchunk;
+  c.remap = (flags & THR_SHAPE_XCD_REMAP) ? 1 : 0;
+  c.box = (flags & THR_SHAPE_XCD_BOXES) ? 1 : 0;
+  c.nt_stores = (flags & THR_SHAPE_NT_STORES) ? 1 : 0;
+  if (tchunk == 1 && (flags & MARCH_FLAGS) == THR_SHAPE_ONE_SITE) {
+    c.site = 1;
+    return c;
+  }
+  c.uniform_links = (flags & THR_SHAPE_UNIFORM_LINKS) ? 1 : 0;
+  c.laneshift = (flags & THR_SHAPE_LANESHIFT) ? 1 : 0;
+  c.lds_x = (flags & THR_SHAPE_LDS_X) ? 1 : 0;
+  c.occ_cap = (flags >> THR_SHAPE_OCC_SHIFT) & 3;
+  c.lds_y = (flags & THR_SHAPE_LDS_Y) ? 1 : 0;
+  return c;
 }
 
 int thr_dslash_autotune(const void *links, const int dims[4], int prec, int *tchunk, int *flags,
@@ -765,8 +794,7 @@ int thr_dslash_autotune(const void *links, const int dims[4], int prec, int *tch
   THR_CHECK(prec >= 0 && prec <= 2, THR_ERR_ARG, "prec must be THR_F64, THR_F32 or THR_F16");
   DslashConfig c;
   TRY(dslash_autotune(mkdims(dims), prec, links, &c, pick(stream)));
-  if (tchunk) *tchunk = c.tchunk;
-  if (flags) *flags = shape_flags(c);
+  shape_pair(c, tchunk, flags);
   return THR_OK;
 }
 
@@ -778,8 +806,7 @@ int thr_dslash_autotune_nrhs(const void *links, const int dims[4], int prec, int
   THR_CHECK(nrhs >= 1 && nrhs <= MAXRHS, THR_ERR_ARG, "nrhs out of range (1..32)");
   DslashConfig c;
   TRY(dslash_autotune(mkdims(dims), prec, links, &c, pick(stream), nrhs));
-  if (tchunk) *tchunk = c.tchunk;
-  if (flags) *flags = shape_flags(c);
+  shape_pair(c, tchunk, flags);
   return THR_OK;
 }
 
@@ -788,17 +815,19 @@ int thr_dslash_set_config(const int dims[4], int prec, int tchunk, int flags) {
   THR_CHECK(prec >= 0 && prec <= 2, THR_ERR_ARG, "prec must be THR_F64, THR_F32 or THR_F16");
   THR_CHECK(tchunk >= 1 && tchunk <= dims[2], THR_ERR_ARG, "tchunk must be in 1..Lt");
   THR_CHECK((flags & ~511) == 0, THR_ERR_ARG, "unknown shape flags");
-  DslashConfig c;
-  c.tchunk = tchunk;
-  c.remap = (flags & THR_SHAPE_XCD_REMAP) ? 1 : 0;
-  c.uniform_links = (flags & THR_SHAPE_UNIFORM_LINKS) ? 1 : 0;
-  c.laneshift = (flags & THR_SHAPE_LANESHIFT) ? 1 : 0;
-  c.box = (flags & THR_SHAPE_XCD_BOXES) ? 1 : 0;
-  c.lds_x = (flags & THR_SHAPE_LDS_X) ? 1 : 0;
-  c.nt_stores = (flags & THR_SHAPE_NT_STORES) ? 1 : 0;
-  c.occ_cap = (flags >> THR_SHAPE_OCC_SHIFT) & 3;
-  c.lds_y = (flags & THR_SHAPE_LDS_Y) ? 1 : 0;
-  dslash_set_config(mkdims(dims), prec, c);
+  dslash_set_config(mkdims(dims), prec, pair_shape(tchunk, flags));
+  return THR_OK;
+}
+
+int thr_dslash_clear_config(const int dims[4], int prec) {
+  if (dims) {
+    TRY(check_dims(dims));
+    THR_CHECK(prec >= 0 && prec <= 2, THR_ERR_ARG, "prec must be THR_F64, THR_F32 or THR_F16");
+    const Dims d = mkdims(dims);
+    dslash_clear_config(&d, prec);
+  } else {
+    dslash_clear_config(nullptr, 0);
+  }
   return THR_OK;
 }
 
@@ -811,8 +840,7 @@ int thr_dslash_get_config_nrhs(const int dims[4], int prec, int nrhs, int *tchun
   THR_CHECK(prec >= 0 && prec <= 2, THR_ERR_ARG, "prec must be THR_F64, THR_F32 or THR_F16");
   THR_CHECK(nrhs >= 1 && nrhs <= MAXRHS, THR_ERR_ARG, "nrhs out of range (1..32)");
   const DslashConfig c = dslash_config(mkdims(dims), prec, nrhs);
-  if (tchunk) *tchunk = c.tchunk;
-  if (flags) *flags = shape_flags(c);
+  shape_pair(c, tchunk, flags);
   return THR_OK;
 }
 

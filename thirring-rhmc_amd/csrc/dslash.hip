@@ -1338,6 +1338,12 @@ void dslash_set_config(const Dims &d, int prec, DslashConfig c, int which) {
     if (which < 0 || which == m) g_tuned[TuneKey{d.lx, d.ly, d.lt, d.ls, prec, m}] = c;
 }
 
+void dslash_clear_config(const Dims *d, int prec) {
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  if (!d) return g_tuned.clear();
+  for (int m = 0; m < 2; m++) g_tuned.erase(TuneKey{d->lx, d->ly, d->lt, d->ls, prec, m});
+}
+
 // block -> lattice mapping of a launch with configuration c; *nblocks
 // receives the grid's x extent (blocks per right-hand side)
 static Tiling make_tiling(const Dims &d, const DslashConfig &c, unsigned *nblocks) {
@@ -1675,8 +1681,7 @@ int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *be
       if (!rc) first.push_back({ms, c});
     }
   }
-  // one site per thread, on both tilings (not one of the pinnable flags: a
-  // shape pinned by flags always marches)
+  // one site per thread, on both tilings
   for (int v = 0; v < 4 && !rc; v++) {
     DslashConfig c;
     c.site = 1;

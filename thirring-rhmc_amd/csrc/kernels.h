@@ -140,6 +140,8 @@ long dslash_grid_blocks(const Dims &d, const DslashConfig &c);
 DslashConfig dslash_config(const Dims &d, int prec, int nrhs = 1);
 // which: 0 single-RHS class, 1 batches, -1 both
 void dslash_set_config(const Dims &d, int prec, DslashConfig c, int which = -1);
+// forget the shapes pinned for d and prec (d null: all of them)
+void dslash_clear_config(const Dims *d, int prec);
 // times the launch shapes on scratch fields of nrhs right-hand sides and pins
 // the fastest for (d, prec) in nrhs's batch class
 int dslash_autotune(const Dims &d, int prec, const void *links, DslashConfig *best,

@@ -66,6 +66,7 @@ _SIGS = {
     "thr_dslash_autotune": ([P, P, I32, IP, IP, P], I32),
     "thr_dslash_autotune_nrhs": ([P, P, I32, I32, IP, IP, P], I32),
     "thr_dslash_set_config": ([P, I32, I32, I32], I32),
+    "thr_dslash_clear_config": ([P, I32], I32),
     "thr_dslash_get_config": ([P, I32, IP, IP], I32),
     "thr_dslash_get_config_nrhs": ([P, I32, I32, IP, IP], I32),
     "thr_links_to_f32_dev": ([P, P, P, P], I32),
@@ -536,6 +537,7 @@ def dslash_dev(out, inp, links, dims, am, imass=3, am3=1.0, dagger=False, prec="
 
 SHAPE_XCD_REMAP, SHAPE_UNIFORM_LINKS, SHAPE_LANESHIFT, SHAPE_XCD_BOXES, SHAPE_LDS_X = 1, 2, 4, 8, 16
 SHAPE_NT_STORES = 32
+SHAPE_ONE_SITE = SHAPE_LDS_X | 3 << 6  # with tchunk 1: one site per thread, no march
 
 
 def dslash_autotune(links, dims, prec="f64", stream=None, nrhs=1):
@@ -557,6 +559,13 @@ def dslash_set_config(dims, prec, tchunk, flags):
     init()
     _check(lib().thr_dslash_set_config(_dims(dims), PREC[prec], int(tchunk), int(flags)),
            "dslash_set_config")
+
+
+def dslash_clear_config(dims=None, prec="f64"):
+    """Forgets the shapes pinned for dims and precision (dims None: all of
+    them): launches take the defaults again."""
+    _check(lib().thr_dslash_clear_config(None if dims is None else _dims(dims), PREC[prec]),
+           "dslash_clear_config")
 
 
 def dslash_get_config(dims, prec="f64", nrhs=1):
