@@ -76,3 +76,27 @@ def test_clear_unpins_both_batch_classes():
     assert get((4, 4, 4, 8), "f64") == other
     assert G.lib().thr_dslash_clear_config(G._dims((4, 0, 4, 8)), 0) == 1
     assert G.lib().thr_dslash_clear_config(G._dims(dims), 3) == 1
+
+
+# the environment's settings take effect on launches whose default is the
+# one-site kernel, too: those that only the march reads select it
+@pytest.mark.parametrize("name,value,want", [
+    ("TCHUNK", "3", (3, 0)), ("UNIFORM", "1", (1, 2)), ("LANESHIFT", "0", (1, 0)),
+    ("LDSX", "1", (1, 16)), ("LDSY", "1", (1, 256)), ("OCC", "2", (1, 128))])
+def test_environment_selects_the_march(monkeypatch, name, value, want):
+    dims = (4, 4, 6, 12)
+    assert one_site(get(dims, "f64"))
+    monkeypatch.setenv("THR_DSLASH_" + name, value)
+    tc, fl = get(dims, "f64")
+    assert (tc, fl & MARCH_FLAGS) == want
+    monkeypatch.setenv("THR_DSLASH_SITE", "1")
+    assert one_site(get(dims, "f64"))
+
+
+@pytest.mark.parametrize("name,bit", [("REMAP", 1), ("BOXES", 8), ("NT", 32)])
+def test_environment_settings_of_both_kernels(monkeypatch, name, bit):
+    for dims in ((4, 4, 6, 12), (32, 32, 32, 64)):
+        was = get(dims, "f64")
+        monkeypatch.setenv("THR_DSLASH_" + name, "0" if was[1] & bit else "1")
+        assert get(dims, "f64") == (was[0], was[1] ^ bit)
+        monkeypatch.delenv("THR_DSLASH_" + name)

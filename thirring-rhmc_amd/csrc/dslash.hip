@@ -1234,7 +1234,7 @@ static bool box_split(const Dims &d, unsigned &px, unsigned &py, unsigned &pt) {
 // identical run to run); dslash_autotune times the candidates on scratch
 // fields and pins the fastest for the process.  THR_DSLASH_TCHUNK / _REMAP /
 // _UNIFORM / _LANESHIFT / _BOXES / _LDSX / _LDSY / _NT / _OCC / _SITE override the
-// default.
+// default; one that only the march reads selects it, unless _SITE=1 is given too.
 // ---------------------------------------------------------------------------
 namespace {
 // shapes are pinned per lattice, precision and batch class (one right-hand
@@ -1308,6 +1308,10 @@ DslashConfig default_config(const Dims &d, int prec, int nrhs) {
   c.uniform_links = lines ? 1 : 0;
   c.lds_x = c.uniform_links;
   if (!dslash_env_set()) return c;
+  // settings that only the march reads ask for the march
+  for (const char *v : {"THR_DSLASH_TCHUNK", "THR_DSLASH_UNIFORM", "THR_DSLASH_LANESHIFT",
+                        "THR_DSLASH_LDSX", "THR_DSLASH_LDSY", "THR_DSLASH_OCC"})
+    if (std::getenv(v)) c.site = 0;
   if (const char *e = std::getenv("THR_DSLASH_SITE")) c.site = std::atoi(e) ? 1 : 0;
   if (const char *e = std::getenv("THR_DSLASH_TCHUNK")) c.tchunk = std::max(1, std::atoi(e));
   if (const char *e = std::getenv("THR_DSLASH_REMAP")) c.remap = std::atoi(e) ? 1 : 0;
