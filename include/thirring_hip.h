@@ -370,7 +370,16 @@ int thr_derivs_batch_dev(const void *const *r, const void *const *x2, const doub
                          const int *iflag, int npair, const int dims[4], void *dsdpi,
                          void *stream);
 
-/* reference-faithful multishift on device fields; out [ndiagq][4*V5] complex128 */
+/* reference-faithful multishift on device fields; out [ndiagq][4*V5] complex128.
+ * The FP64 solve (use_sp = 0; also in thr_qmrherm, thr_force, thr_hamilton,
+ * thr_evolve_theta_pp and thr_multishift_plain_dev) updates its shifts once
+ * per 32 iterations from a ring of 32 residuals in the bound context: 2 KiB a
+ * 5-D site (403 MB at 16^3 x 48, 4.3 GB at 32^3 x 64).  The ring is taken up to
+ * 16 GiB and a quarter of the free device memory; without it every iteration
+ * updates the shifts (same results to rounding, slower).  The context keeps it
+ * for the next solve, gives it back when one of its own allocations would
+ * fail, and thr_context_trim frees it; THR_MULTISHIFT_RING=0 in the
+ * environment does without it. */
 int thr_multishift_dev(const void *links64, const int dims[4], float am, int imass, float am3,
                        int ndiagq, const double *aden, const double *anum, void *out,
                        const void *input, float res, int maxcg, int use_sp, int kernel,

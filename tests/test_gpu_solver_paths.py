@@ -38,3 +38,37 @@ def test_congrad_stopped_by_alpha_leaves_x(G, path):
             G.congrad_dev(phi, x, l64, dims, 0.0, 0.1, 3, niterc=50,
                           kernel="wilson" if path == "wilson" else "shamir")
     assert np.array_equal(x.to_host(), x0)
+
+
+def test_ring_is_given_back(G):
+    """The FP64 multishift's ring of 32 residuals stays in the context, and an
+    allocation of the context that fails takes it back (here one of 512 GiB,
+    which no card holds and the call reports before any launch)."""
+    from hiprt import DeviceArray
+    dims = (16, 16, 16, 16)
+    lx, ly, lt, ls = dims
+    v5 = lx * ly * lt * ls
+    rng = np.random.default_rng(52)
+    links = np.stack([np.ones(3 * lx * ly * lt), 0.4 * rng.standard_normal(3 * lx * ly * lt)], -1)
+    l64 = DeviceArray.from_host(links)
+    b, x = DeviceArray.from_host(rng.standard_normal((4 * v5, 2))), DeviceArray((4 * v5, 2), np.float64)
+    ring = 32 * 64 * v5
+    ctx = G.Context()
+    ctx.bind()
+    try:
+        print("case: ring given back", flush=True)
+        G.multishift_dev(l64, dims, 0.1, 3, [0.5], [1.0], x, b, 1e-4, 100)
+        assert ctx.scratch_bytes() > ring
+        big = (64, 64, 64, 1024)  # 16 GiB fields, 32 shifts
+        with pytest.raises(G.ThrError) as e:
+            G.multishift_dev(l64, big, 0.1, 3, np.ones(32), np.ones(32), x, b, 1e-4, 100)
+        assert e.value.status == G.STATUS["hip"]
+        assert ctx.scratch_bytes() - 64 * int(np.prod(big)) < ring
+        ctx.trim()
+        # and the context still solves
+        G.multishift_dev(l64, dims, 0.1, 3, [0.5], [1.0], x, b, 1e-4, 100)
+        assert ctx.scratch_bytes() > ring
+        ctx.trim()
+    finally:
+        ctx.unbind()
+        ctx.destroy()

@@ -25,6 +25,11 @@ void context_destroy(Context *c);
 void context_bind(Context *c);
 size_t workspace_bytes();
 void *workspace(int slot, size_t bytes);
+// workspace that the caller can do without: null where it would take more than
+// a quarter of the free memory or cannot be had.  Held until release_spare;
+// then the context frees it as soon as another of its allocations fails.
+void *spare_workspace(int slot, size_t bytes);
+void release_spare(int slot);
 // pinned host buffer of the bound context (state read-backs and uploads go
 // through these: pageable async copies are staged through runtime buffers
 // shared by all threads)

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -31,6 +32,9 @@ namespace {
 struct Buf {
   void *p = nullptr;
   size_t n = 0;
+  // a buffer that a call can do without: freed when another allocation of the
+  // context fails, unless a call holds it
+  bool spare = false, held = false;
 };
 }  // namespace
 
@@ -82,22 +86,62 @@ void context_destroy(Context *c) {
 
 void context_bind(Context *c) { t_ctx = c; }
 
+// device memory for b, or null with no error left behind
+static bool grow(Buf &b, size_t bytes) {
+  if (b.p) (void)hipFree(b.p);
+  b.p = nullptr;
+  b.n = 0;
+  if (hipMalloc(&b.p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    b.p = nullptr;
+    return false;
+  }
+  b.n = bytes;
+  return true;
+}
+
 void *workspace(int slot, size_t bytes) {
   Context &c = cur();
   std::lock_guard<std::mutex> lk(c.mu);
   Buf &b = c.ws[slot];
-  if (b.n < bytes) {
-    if (b.p) (void)hipFree(b.p);
-    b.p = nullptr;
-    b.n = 0;
-    if (hipMalloc(&b.p, bytes) != hipSuccess) {
+  if (b.n < bytes && !grow(b, bytes)) {
+    bool freed = false;
+    for (auto &kv : c.ws) {
+      Buf &o = kv.second;
+      if (!o.spare || o.held || !o.p) continue;
+      (void)hipFree(o.p);
+      o.p = nullptr;
+      o.n = 0;
+      freed = true;
+    }
+    if (!freed || !grow(b, bytes)) {
       set_error("hipMalloc of workspace failed");
-      b.p = nullptr;
       return nullptr;
     }
-    b.n = bytes;
   }
   return b.p;
+}
+
+void *spare_workspace(int slot, size_t bytes) {
+  Context &c = cur();
+  std::lock_guard<std::mutex> lk(c.mu);
+  Buf &b = c.ws[slot];
+  if (b.n < bytes) {
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (bytes > (free + b.n) / 4 || !grow(b, bytes)) return nullptr;
+  }
+  b.spare = b.held = true;
+  return b.p;
+}
+
+void release_spare(int slot) {
+  Context &c = cur();
+  std::lock_guard<std::mutex> lk(c.mu);
+  c.ws[slot].held = false;
 }
 
 void *host_workspace(int slot, size_t bytes) {
@@ -844,14 +888,22 @@ int multishift_reference(const OpDesc &op, int n, const double *aden, const doub
   double *partial = partial_buffer(2 * np);
   THR_CHECK(h && ps && st && partial, THR_ERR_HIP, "workspace allocation failed");
   // Blocked updates keep MSR residuals (16 GiB at most here: 512 MiB fields;
-  // 32^3 x 64 takes 4.3); larger fields, and contexts where the ring does not
-  // fit beside the caller's memory, update every shift in every iteration.
+  // 32^3 x 64 takes 4.3).  Larger fields, and a card on which the ring is more
+  // than a quarter of the free memory, update every shift in every iteration:
+  // 16^3 x 48, 25 shifts 8.0 ms with the ring, 49.4 ms without.
+  // THR_MULTISHIFT_RING=0: never.  The context keeps the ring, and gives it
+  // back when one of its own allocations would fail.
+  const char *ring_env = std::getenv("THR_MULTISHIFT_RING");
   const size_t ring_bytes = sizeof(double2) * ns * MSR;
-  double2 *ring = nullptr;
-  if (ring_bytes <= (size_t(16) << 30)) {
-    ring = (double2 *)workspace(26, ring_bytes);
-    if (!ring) (void)hipGetLastError();
-  }
+  struct Ring {
+    double2 *p = nullptr;
+    ~Ring() {
+      if (p) release_spare(26);
+    }
+  } held;
+  if (!(ring_env && std::atoi(ring_env) == 0) && ring_bytes <= (size_t(16) << 30))
+    held.p = (double2 *)spare_workspace(26, ring_bytes);
+  double2 *ring = held.p;
   int rc = ms_setup(st, n, aden, anum, res, maxcg, s, plain);
   if (rc) return rc;
   const DslashConfig cfg = dslash_config(d, P64);
