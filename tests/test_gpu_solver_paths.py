@@ -4,6 +4,9 @@ lattice do not take, and what the solvers leave behind when they stop."""
 import numpy as np
 import pytest
 
+import dense as D
+import oracle as O
+
 pytestmark = pytest.mark.gpu
 
 
@@ -72,3 +75,37 @@ def test_ring_is_given_back(G):
     finally:
         ctx.unbind()
         ctx.destroy()
+
+
+# The FP64 multishift's paths: updates once per 32 iterations, with the scalar
+# steps as kernels of their own (a march: also the default from 2^18 sites with
+# Ls = 32 and 64, from 2^20 with others) and around separate epilogues (Wilson
+# kernel, Ls > 64); and updates in every iteration (no ring), behind passes of
+# each kind.  Caps inside the first block of 32, at its end, one past it, and in
+# the third block.
+@pytest.mark.parametrize("path", ["march", "wilson80", "one_site_no_ring", "march_no_ring",
+                                  "wilson_no_ring", "wilson80_no_ring"])
+@pytest.mark.parametrize("maxcg", [0, 1, 31, 32, 33, 65])
+def test_multishift_paths_at_the_cap(G, monkeypatch, maxcg, path):
+    """Against the oracle: fewer than 100 iterations on smooth links (spread
+    0.4) amplify rounding by less than 1e4, so 1e-11; iteration counts equal."""
+    dims = (2, 3, 2, 80) if "80" in path else (3, 5, 4, 12)
+    kernel = "wilson" if "wilson" in path else "shamir"
+    if "no_ring" in path:
+        monkeypatch.setenv("THR_MULTISHIFT_RING", "0")
+    if "march" in path:
+        G.dslash_set_config(dims, "f64", 2, G.SHAPE_XCD_REMAP)
+    rng = np.random.default_rng(53)
+    u = O.coef((0.4 * rng.standard_normal(dims[:3] + (3,))).astype(np.float32), dims)
+    inp = D.rand_spinor(dims, rng)
+    sig = np.array([1e-4, 0.05, 0.7, 9.0])
+    print("case: multishift path", path, maxcg, flush=True)
+    og, cg, cgs = G.multishift(u, dims, 0.05, 3, sig, np.ones(4), inp, res=1e-5, maxcg=maxcg,
+                               kernel=kernel)
+    oo, co, cos = O.multishift(u, dims, 0.05, 3, sig, np.ones(4), inp, res=1e-5, maxcg=maxcg,
+                               kernel=kernel)
+    assert cg == co and np.array_equal(cgs, cos)
+    if maxcg == 0:
+        assert not og.any()
+    else:
+        assert np.linalg.norm(og - oo) <= 1e-11 * np.linalg.norm(oo)
