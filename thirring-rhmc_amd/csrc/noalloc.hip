@@ -30,8 +30,6 @@ __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 std::mutex g_noalloc_mu;
 void *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
-// the stop-flag read-back of the solver loop (pageable: no pinned allocation)
-thread_local int t_host_flag;
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -102,7 +100,7 @@ int thr_congrad_dev_noalloc(const void *phi, void *x, const void *links64, const
   op.u64 = (const double2 *)links64;
   // no stream given: the null stream (creating one could allocate)
   return cg_reference_bufs(op, (const double2 *)phi, (double2 *)x, res, niterc, itercg,
-                           iterations, (hipStream_t)stream, B, &t_host_flag);
+                           iterations, (hipStream_t)stream, B, true);
 }
 
 }  // extern "C"

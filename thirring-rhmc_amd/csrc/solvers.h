@@ -51,10 +51,10 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
 
 // the same CG on caller-provided device buffers: three spinors, the solver
 // state (cg_state_bytes()) and dslash_blocks(d) partial sums.  None needs
-// clearing (every one is written before it is read).  host_flag (optional)
-// is the host int the stop flag is polled into; given one, nothing is
-// allocated (then only the Shamir kernel is allowed: the Wilson kernel's
-// unfused epilogue needs library scratch).
+// clearing (every one is written before it is read).  no_alloc: allocate
+// nothing, pinned host memory included (then only the Shamir kernel is
+// allowed: the Wilson kernel's separate epilogue above Ls = 64 needs library
+// scratch).
 struct CgBuffers {
   double2 *h, *r, *p;
   void *state;
@@ -64,7 +64,7 @@ struct CgBuffers {
 size_t cg_state_bytes();
 int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float res, int niterc,
                       int *itercg, int *iterations, hipStream_t s, const CgBuffers &B,
-                      int *host_flag);
+                      bool no_alloc);
 
 // reference-faithful multishift CG (multishift_module.F90:13-284), FP64 vectors.
 // out: [n][4*V5] shift solutions.

@@ -2,8 +2,9 @@
 //
 // The reference runs every dot product through an MPI_AllReduce and a host
 // round trip.  Here all scalars (alpha, beta, zeta recurrences, convergence
-// window) live in a small device state struct written by single-block
-// "finalize" kernels that sum the per-block partials in a fixed order, so
+// window) live in a small device state struct.  One block at a time writes it,
+// summing the per-block partials in a fixed order: the first block of the
+// operator launch that follows, or a kernel of its own (krylov_scalars.h).  So
 // results are deterministic and the host only polls a stop flag every few
 // iterations.  Kernels of an iteration that starts after the stop flag was
 // raised exit immediately, so the iteration counts and final vectors are
@@ -651,7 +652,7 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
   B.partial = partial_buffer(2 * np);
   THR_CHECK(B.h && B.r && B.p && B.state && B.partial, THR_ERR_HIP, "workspace allocation failed");
   B.partial2 = B.partial + np;
-  return cg_reference_bufs(op, phi, x, res, niterc, itercg, iterations, s, B, nullptr);
+  return cg_reference_bufs(op, phi, x, res, niterc, itercg, iterations, s, B, false);
 }
 
 // The reference's CG with h = M p by recurrence (h_new = M r + beta h; M is
@@ -662,14 +663,14 @@ int cg_reference(const OpDesc &op, const double2 *phi, double2 *x, float res, in
 // us per iteration with five launches, 15 with two.
 int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float res, int niterc,
                       int *itercg, int *iterations, hipStream_t s, const CgBuffers &B,
-                      int *host_flag) {
+                      bool no_alloc) {
   const Dims &d = op.d;
   const DslashConfig cfg = dslash_config(d, P64);
   const int nb = op_partials(op, cfg);
   double2 *h = B.h, *r = B.r, *p = B.p;
   CgState *st = (CgState *)B.state;
   THR_CHECK(h && r && p && st && B.partial, THR_ERR_ARG, "congrad: missing buffers");
-  THR_CHECK(op.kernel == 0 || !host_flag, THR_ERR_ARG,
+  THR_CHECK(op.kernel == 0 || !no_alloc, THR_ERR_ARG,
             "congrad on caller buffers runs the Shamir kernel only");
   const bool fused = B.partial2 && op_fuses_scalars(op, cfg);
   double *apart = B.partial, *lpart = fused ? B.partial2 : B.partial;  // |h|^2 and |r|^2 sums
@@ -736,8 +737,8 @@ int cg_reference_bufs(const OpDesc &op, const double2 *phi, double2 *x, float re
   // enqueued past the end is two launches that find the stop flag (6 us).  From
   // the third poll on the next batch is most of what the mean rate of decay
   // since the last poll leaves to do.
-  CgState local;
-  CgState *pinned = host_flag ? nullptr : (CgState *)host_workspace(22, sizeof(CgState));
+  CgState local;  // pageable: the read-back of a solve that may not allocate
+  CgState *pinned = no_alloc ? nullptr : (CgState *)host_workspace(22, sizeof(CgState));
   CgState &hs = pinned ? *pinned : local;
   int batch = 4;
   double was = 0.0;
