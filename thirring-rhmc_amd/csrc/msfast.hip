@@ -284,8 +284,10 @@ __device__ inline cx<double> widen(cx<float> v) {
 
 // apply the block's coefficients of ring slots [q0, q0 + QN) to x_i and p_i
 // (FP64), reading each residual once, all of it non-temporal and with the next
-// shift's x_i, p_i loaded ahead (24^3 x 32, 8 sources, 12 shifts, 64 FP32 slots:
-// 15.4 GB in 2.89 ms, 5.3 TB/s; 3.19 ms through the caches).  A 64-iteration block takes one launch
+// shift's x_i, p_i loaded ahead.  24^3 x 32, 8 sources: 64 FP32 slots with 6
+// shifts in the window 12.7 GB in 2.93 ms (4.3 TB/s), 32 FP64 slots with 8 to 12
+// 12.0 GB in 2.43 and 16.3 GB in 3.12 ms (4.9 and 5.2).  Median FP32 launch of
+// the solve 2.89 ms, 3.19 ms through the caches.  A 64-iteration block takes one launch
 // with FP32/FP16 residuals (held as such, widened per use) and two with FP64
 // ones (q0 = 0, 32: the second adds its slots to the x_i, p_i the first
 // wrote).

@@ -6,9 +6,9 @@
 // the alpha recurrences, an M^dagger pass (r += omega M^+ h, |r|^2), a grid
 // barrier, the lambda recurrences and the shift updates x_i -= omega_i p_i,
 // p_i = gamma_i p_i + zeta_i r.  On a lattice of a few 10^4 sites per source
-// the streaming solver spends its iteration in kernel dispatch (four launches
+// the streaming solver spends its iteration in kernel dispatch (two launches
 // of a few microseconds each); here an iteration costs two grid barriers,
-// which on this GPU cost about as much (see msfast_persistent_fits), so the
+// which on this GPU cost more (see msfast_persistent_fits), so the
 // solver is an option (THR_PERSIST=1), not the default.
 //
 // Blocks are assigned to sources (blocks [src * bs, (src + 1) * bs) sweep
@@ -382,9 +382,9 @@ __global__ __launch_bounds__(BLK) void k_msf_persistent(PArgs A, GridBar B) {
 
 bool msfast_persistent_fits(const MsfArgs &A) {
   // opt-in (THR_PERSIST=1).  Measured on MI355X, 4 sources of (M^+M) x = b:
-  // at 8^3 x Ls=8 an iteration takes 22.1 us here against 22.9 us for the
-  // streaming kernels (four launches), and at 12^2 x 24 x Ls=16 100 us at
-  // best against 39 us.  A grid barrier across the 8 XCDs has to write back
+  // at 8^3 x Ls=8 an iteration takes 22.4 us here against 13.2 us for the
+  // streaming kernels (two launches), and at 12^2 x 24 x Ls=16 94 us against
+  // 26 us.  A grid barrier across the 8 XCDs has to write back
   // and invalidate each XCD's L2 as a kernel boundary does, so it costs about
   // what a launch costs, and the per-site operator here is slower than the
   // streaming Dslash kernels.

@@ -411,8 +411,9 @@ __global__ __launch_bounds__(BLK) void k_ms_coef(MsState *st, const double *part
 // iteration updates its shifts).  The residuals of an element stay in
 // registers for all shifts.  Nothing here is read again before 32 iterations
 // have passed through the caches, so all of it is non-temporal: 1.0 GB at 16^3
-// x 48 with 12 shifts in 208 us (4.8 TB/s), 244 without, 256 without the load
-// of the next shift ahead of this one's work (four shifts ahead: 304).  The
+// x 48 with 12 shifts in the window in 190 us (5.2 TB/s).  Median launch of a
+// solve of 25 shifts there 208 us; 244 through the caches, 256 also without the
+// load of the next shift ahead of this one's work (four shifts ahead: 304).  The
 // first block starts from p_i = b, x_i = 0 and writes every shift (x_i = 0
 // where nothing was updated).
 __global__ __launch_bounds__(BLK) void k_ms_flush(long ns, const MsState *S, const double2 *b,
