@@ -451,20 +451,21 @@ __global__ __launch_bounds__(BLK) void k_ms_flush(long ns, const MsState *S, con
   fetch(0);
   for (int i = 0; i < n; i++) {
     const cx<double> base = pn;
-    cx<double> x = xn;
+    const cx<double> x = xn;
     fetch(i + 1);
     if (!scnt[i]) {
       if (first) st(X, i * ns + e, cx<double>{0.0, 0.0});
       if (first && sact[i]) st(P, i * ns + e, bv);
       continue;
     }
-    x = x + sc[i] * base;
+    // the block's own sum first: its roundings are of its size, not of x_i's
+    cx<double> dx = sc[i] * base;
     if (sact[i]) {
       cx<double> p = sa[i] * base;
 #pragma unroll
       for (int q = 0; q < MSR; q++) {
         if (q < jc) {
-          x = x + sd[i][q] * R[q];
+          dx = dx + sd[i][q] * R[q];
           p = p + sb[i][q] * R[q];
         }
       }
@@ -472,9 +473,9 @@ __global__ __launch_bounds__(BLK) void k_ms_flush(long ns, const MsState *S, con
     } else {
 #pragma unroll
       for (int q = 0; q < MSR; q++)
-        if (q < jc) x = x + sd[i][q] * R[q];
+        if (q < jc) dx = dx + sd[i][q] * R[q];
     }
-    st_nt(X, i * ns + e, x);
+    st_nt(X, i * ns + e, x + dx);
   }
 }
 
